@@ -388,9 +388,7 @@ __global__ __launch_bounds__(256) void sample_faces(Grid g, const double *U, Flu
     for (int k = 0; k < artra::kFeat; ++k) feat[t * artra::kFeat + k] = x[k];
     artra::FaceState fs;
     artra::face_state<S>(mdl, st[2], st[3], fs);
-    double F[5], lab = 0.0;
-    artra::weno_flux<S>(fs, st, F, &lab);
-    label[t] = (float)lab;
+    label[t] = (float)artra::weno_label<S>(fs, st);
 }
 
 // ---------------------------------------------------------------- boundary

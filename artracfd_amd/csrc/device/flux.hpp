@@ -283,73 +283,129 @@ __host__ __device__ __forceinline__ void viscous_flux(const FluxModel &mdl, cons
 // Fast variant.  Same numerical flux, evaluated with fewer FP64 instructions;
 // results agree with the reference order to rounding level (checked against
 // the 1e-10 relative-L2 contract on every golden case):
-//  * one reciprocal per density instead of one division per velocity;
+//  * one reciprocal per density instead of one division per velocity, shared
+//    by the two nodes of a face;
 //  * the characteristic projection uses the structure of the left
 //    eigenvectors: with K = q U0 - vel.mom + U4 and M = un U0 - U_{1+S},
-//    W = (bK + dM, U0 - 2bK [entropy] / U_{1+t} - 2b vel_t K [shear], bK - dM),
-//    12 instead of 50 operations per stencil node;
-//  * WENO weights without their own divisions: with d_k = (eps + IS_k)^2,
-//    omega_k = C_k prod_{j!=k} d_j / sum_l C_l prod_{j!=l} d_j, and the two
-//    split sides of a field summed over one common denominator
-//    (weno5_field_parts);
+//    W = (bK + dM, U0 - 2bK [entropy] / U_{1+t} - 2b vel_t K [shear], bK - dM);
+//  * WENO weights without their own divisions (weno5_field);
+//  * reciprocals and square roots by Newton steps on the hardware estimates
+//    (within an ulp), without the scaling and fix-up of the IEEE sequences:
+//    densities, sound speeds and weight sums are far from the ends of the
+//    exponent range;
 //  * fused multiply-adds throughout.
+// The sweeps are bound by FP64 issue, so instructions are what counts: the
+// WENO5 sweep kernel holds 622 FP64 instructions with the arrangement below
+// and 787 with expanded smoothness indicators, IEEE divisions and roots
+// (six steps at 255^3 and the field's read-back: 57.5 against 62.6 ms).
 namespace artra {
 namespace fast {
 
+// 1 / x: the hardware estimate (about 2^-26) refined twice.  Zero,
+// infinity and subnormal x are outside its domain.
+__host__ __device__ __forceinline__ double reciprocal(double x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    double y = __builtin_amdgcn_rcp(x);
+    y = fma(fma(-x, y, 1.0), y, y);
+    return fma(fma(-x, y, 1.0), y, y);
+#else
+    return 1.0 / x;
+#endif
+}
+
+// sqrt(x) and 1 / sqrt(x) of a positive normal x: the hardware reciprocal
+// root refined by two coupled Goldschmidt steps, the root then corrected by
+// its residual.
+__host__ __device__ __forceinline__ void root_pair(double x, double &root, double &inverse)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    r = fma(-h, g, 0.5);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    root = g;
+    inverse = h + h;
+#else
+    root = sqrt(x);
+    inverse = 1.0 / root;
+#endif
+}
+
+__host__ __device__ __forceinline__ double root(double x)
+{
+    double g, h;
+    root_pair(x, g, h);
+    return g;
+}
+
 // One characteristic field of the split WENO5 flux, h = WENO5(lp W0..lp W4)
 // + WENO5(ln W5..ln W1), from the field's six stencil values W0..W5 and its
-// split eigenvalues, as num / den: Jiang-Shu WENO5 (weno5 above) of the
-// scaled values lp W and ln W, arranged for fewer operations and one
-// division per field (the two sides over a common denominator):
-//  * the smoothness indicators are quadratic forms, IS(l f) = l^2 IS(f), so
-//    they are formed once on W (their second differences shared between the
-//    two sides) and scaled by lp^2 or ln^2;
-//  * 12 IS = 13 a^2 + 3 b^2 and eps are scaled by 12 together, a common
-//    factor that cancels in the weights t_k = C_k prod_{j != k} (eps + IS_j)^2
-//    (C scaled by 10 likewise);
-//  * the candidate values are the central node plus differences,
-//    6 q_k = 6 W2 + R_k (6 W3 + R_k on the mirrored side), so
-//    h = lp W2 + ln W3 + (lp N+ D- + ln N- D+) / (6 D+ D-), N = sum t_k R_k,
-//    D = sum t_k, returned as num = base * den + (...).
-// den >= 6 (1.2e-5)^8: no underflow; it overflows only for smoothness
-// indicators far beyond any flow state (about 1e18).
-__host__ __device__ __forceinline__ void weno5_field_parts(const double W[6], double lp, double ln, double &num,
-                                                           double &den)
+// split eigenvalues, as h = base + num / den: Jiang-Shu WENO5 (weno5 above)
+// of the scaled values lp W and ln W, arranged for fewer operations and one
+// division per field (the two sides over a common denominator).
+//  * The smoothness indicators are quadratic forms of the differences
+//    d_i = W_{i+1} - W_i, so they are formed once on W and scaled by lp^2 or
+//    ln^2.  Completed squares leave three shared terms c d_i^2, c = 39/64:
+//    13 a^2 + 3 b^2 = 16 ((d0 - 11/8 d1)^2 + c d1^2) for the outer
+//    sub-stencils, 16 ((d1 - 5/8 d2)^2 + c d2^2) for the middle one: sums of
+//    squares, no cancellation.
+//  * 3/4 (eps + IS) replaces eps + IS: the common factor cancels in the
+//    weights t_k = 10 C_k prod_{j != k} (eps + IS_j)^2.
+//  * The candidate values are the central node plus differences,
+//    q_k = W2 + R_k / 6 (W3 - R_k / 6 on the mirrored side), so each side is
+//    its central value plus N / (6 D), N = sum t_k R_k, D = sum t_k.
+// den >= (7.5e-7)^8: no underflow; the product of two dens (divide pairs
+// below) overflows only for smoothness indicators beyond about 1e19.
+__host__ __device__ __forceinline__ void weno5_field(const double W[6], double lp, double ln, double &num, double &den,
+                                                     double &base)
 {
-    const double eps12 = 12.0e-6;
+    const double eps34 = 0.75e-6, c = 39.0 / 64.0;
     const double d0 = W[1] - W[0], d1 = W[2] - W[1], d2 = W[3] - W[2], d3 = W[4] - W[3], d4 = W[5] - W[4];
-    const double D0 = d1 - d0, D1 = d2 - d1, D2 = d3 - d2, D3 = d4 - d3;   // second differences
-    const double A0 = (13.0 * D0) * D0, A1 = (13.0 * D1) * D1, A2 = (13.0 * D2) * D2, A3 = (13.0 * D3) * D3;
-    // first-derivative terms of the six sub-stencils: plus side (W0..W4), minus side (W5..W1)
-    const double bp0 = fma(2.0, d1, D0), bp1 = d1 + d2, bp2 = fma(-2.0, d2, D2);
-    const double bm0 = fma(-2.0, d3, D3), bm1 = d2 + d3, bm2 = fma(2.0, d2, D1);
+    const double s1 = (c * d1) * d1, s2 = (c * d2) * d2, s3 = (c * d3) * d3;
+    // plus side (W0..W4), minus side (W5..W1)
+    const double xp0 = fma(-1.375, d1, d0), xp1 = fma(-0.625, d2, d1), xp2 = fma(-1.375, d2, d3);
+    const double xm0 = fma(-1.375, d3, d4), xm1 = fma(-0.625, d2, d3), xm2 = fma(-1.375, d2, d1);
     const double lp2 = lp * lp, ln2 = ln * ln;
-    const double ep0 = fma(lp2, fma(3.0 * bp0, bp0, A0), eps12);
-    const double ep1 = fma(lp2, fma(3.0 * bp1, bp1, A1), eps12);
-    const double ep2 = fma(lp2, fma(3.0 * bp2, bp2, A2), eps12);
-    const double em0 = fma(ln2, fma(3.0 * bm0, bm0, A3), eps12);
-    const double em1 = fma(ln2, fma(3.0 * bm1, bm1, A2), eps12);
-    const double em2 = fma(ln2, fma(3.0 * bm2, bm2, A1), eps12);
+    const double ep0 = fma(lp2, fma(xp0, xp0, s1), eps34);
+    const double ep1 = fma(lp2, fma(xp1, xp1, s2), eps34);
+    const double ep2 = fma(lp2, fma(xp2, xp2, s2), eps34);
+    const double em0 = fma(ln2, fma(xm0, xm0, s3), eps34);
+    const double em1 = fma(ln2, fma(xm1, xm1, s2), eps34);
+    const double em2 = fma(ln2, fma(xm2, xm2, s2), eps34);
     const double gp0 = ep0 * ep0, gp1 = ep1 * ep1, gp2 = ep2 * ep2;
     const double gm0 = em0 * em0, gm1 = em1 * em1, gm2 = em2 * em2;
-    const double tp0 = gp1 * gp2, tp1 = 6.0 * (gp0 * gp2), tp2 = 3.0 * (gp0 * gp1);
-    const double tm0 = gm1 * gm2, tm1 = 6.0 * (gm0 * gm2), tm2 = 3.0 * (gm0 * gm1);
-    // 6 q_k - 6 (central node) of each side's candidates
-    const double Rp0 = fma(5.0, d1, -2.0 * d0), Rp1 = fma(2.0, d2, d1), Rp2 = fma(4.0, d2, -d3);
-    const double Rm0 = fma(2.0, d4, -5.0 * d3), Rm1 = -fma(2.0, d2, d3), Rm2 = fma(-4.0, d2, d1);
-    const double Np = fma(tp0, Rp0, fma(tp1, Rp1, tp2 * Rp2)), Dp = tp0 + tp1 + tp2;
-    const double Nm = fma(tm0, Rm0, fma(tm1, Rm1, tm2 * Rm2)), Dm = tm0 + tm1 + tm2;
-    den = 6.0 * (Dp * Dm);
-    const double base = fma(lp, W[2], ln * W[3]);
-    num = fma(base, den, fma(lp * Np, Dm, (ln * Nm) * Dp));
+    // D = g1 g2 + 3 g0 (2 g2 + g1), N / 2 = g1 g2 (R0 / 2) + 3 g0 (g2 R1 + g1 R2 / 2)
+    const double pp = gp1 * gp2, hp = 3.0 * gp0, pm = gm1 * gm2, hm = 3.0 * gm0;
+    const double Dp = fma(hp, fma(2.0, gp2, gp1), pp), Dm = fma(hm, fma(2.0, gm2, gm1), pm);
+    const double dd2 = d2 + d2;
+    const double Np = fma(hp, fma(gp2, d1 + dd2, gp1 * fma(-0.5, d3, dd2)), pp * fma(2.5, d1, -d0));
+    const double Nm = fma(hm, fma(gm2, d3 + dd2, gm1 * fma(-0.5, d1, dd2)), pm * fma(2.5, d3, -d4));
+    const double third = 1.0 / 3.0;
+    base = fma(ln, W[3], lp * W[2]);
+    den = Dp * Dm;
+    num = fma((third * lp) * Np, Dm, -(((third * ln) * Nm) * Dp));
 }
 
 // Two quotients from one division: a/b and c/d as a (d q) and c (b q), q = 1/(b d).
 __host__ __device__ __forceinline__ void divide_pair(double a, double b, double c, double d, double &x, double &y)
 {
-    const double q = 1.0 / (b * d);
+    const double q = reciprocal(b * d);
     x = a * (d * q);
     y = c * (b * q);
+}
+
+// x + a/b and y + c/d from one division.
+__host__ __device__ __forceinline__ void add_quotients(double x, double a, double b, double y, double c, double d,
+                                                       double &u, double &v)
+{
+    const double q = reciprocal(b * d);
+    u = fma(a, d * q, x);
+    v = fma(c, b * q, y);
 }
 
 __host__ __device__ __forceinline__ double weno3(double f0, double f1, double f2)
@@ -358,169 +414,238 @@ __host__ __device__ __forceinline__ double weno3(double f0, double f1, double f2
     const double e0 = eps + (f1 - f0) * (f1 - f0), e1 = eps + (f2 - f1) * (f2 - f1);
     const double t0 = (1.0 / 3.0) * (e1 * e1), t1 = (2.0 / 3.0) * (e0 * e0);
     const double Q0 = fma(3.0, f1, -f0), Q1 = f1 + f2;
-    return fma(t0, Q0, t1 * Q1) / (2.0 * (t0 + t1));
+    return fma(t0, Q0, t1 * Q1) * reciprocal(2.0 * (t0 + t1));
 }
+
+}  // namespace fast
+
+// Average state and split eigenvalues of a face (fast arithmetic).
+struct FaceState {
+    double u, v, w, hT, c, q, b, d, un, g1;
+    double lp[5], ln[5];
+};
+
+// Velocities and total enthalpy of one node from its conserved state and
+// the reciprocal of its density.
+__host__ __device__ __forceinline__ void velocity_enthalpy(double gamma, const double U[5], double r, double nv[4])
+{
+    nv[0] = U[1] * r;
+    nv[1] = U[2] * r;
+    nv[2] = U[3] * r;
+    nv[3] = fma(-0.5 * (gamma - 1.0), fma(nv[2], nv[2], fma(nv[1], nv[1], nv[0] * nv[0])), gamma * (U[4] * r));
+}
+
+template <int S>
+__host__ __device__ __forceinline__ void face_state(const FluxModel &mdl, const double UL[5], const double UR[5],
+                                                    FaceState &fs)
+{
+    double rL, rR, nL[4], nR[4];
+    fast::divide_pair(1.0, UL[0], 1.0, UR[0], rL, rR);
+    velocity_enthalpy(mdl.gamma, UL, rL, nL);
+    velocity_enthalpy(mdl.gamma, UR, rR, nR);
+    if (mdl.roe) {
+        const double D = fast::root(UR[0] * rL);
+        const double inv = fast::reciprocal(1.0 + D);
+        fs.u = fma(D, nR[0], nL[0]) * inv;
+        fs.v = fma(D, nR[1], nL[1]) * inv;
+        fs.w = fma(D, nR[2], nL[2]) * inv;
+        fs.hT = fma(D, nR[3], nL[3]) * inv;
+    } else {
+        fs.u = 0.5 * (nL[0] + nR[0]);
+        fs.v = 0.5 * (nL[1] + nR[1]);
+        fs.w = 0.5 * (nL[2] + nR[2]);
+        fs.hT = 0.5 * (nL[3] + nR[3]);
+    }
+    fs.q = 0.5 * fma(fs.u, fs.u, fma(fs.v, fs.v, fs.w * fs.w));
+    fs.g1 = mdl.gamma - 1.0;
+    // b = (gamma - 1) / (2 c^2) and d = 1 / (2 c) of the eigenvectors
+    double rc;
+    fast::root_pair(fs.g1 * (fs.hT - fs.q), fs.c, rc);
+    fs.d = 0.5 * rc;
+    fs.b = (0.5 * fs.g1) * (rc * rc);
+    fs.un = (S == 0) ? fs.u : (S == 1) ? fs.v : fs.w;
+    const double lam[5] = {fs.un - fs.c, fs.un, fs.un, fs.un, fs.un + fs.c};
+    if (mdl.sw) {
+#pragma unroll
+        for (int r = 0; r < 5; ++r) {
+            const double size = fast::root(fma(lam[r], lam[r], 1.0e-6));
+            fs.lp[r] = 0.5 * (lam[r] + size);
+            fs.ln[r] = 0.5 * (lam[r] - size);
+        }
+    } else {
+        const double star = fabs(fs.un) + fs.c;
+#pragma unroll
+        for (int r = 0; r < 5; ++r) {
+            fs.lp[r] = 0.5 * (lam[r] + star);
+            fs.ln[r] = 0.5 * (lam[r] - star);
+        }
+    }
+}
+
+// F = R h (right eigenvectors along S).
+template <int S>
+__host__ __device__ __forceinline__ void project_back(const FaceState &fs, const double h[5], double F[5])
+{
+    const double vel[3] = {fs.u, fs.v, fs.w};
+    const double ha = h[0] + h[4], chd = fs.c * (h[4] - h[0]);
+    F[0] = ha + h[1 + S];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) F[1 + m] = (m == S) ? fma(vel[m], F[0], chd) : fma(vel[m], ha, h[1 + m]);
+    double e = fma(fs.un, chd, fs.hT * ha);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) e = fma((t == S) ? fma(fs.un, fs.un, -fs.q) : vel[t], h[1 + t], e);
+    F[4] = e;
+}
+
+// The fast WENO5 flux at the face between stencil nodes 2 and 3, at(m, c)
+// giving component c of node m = 0..5.  The fields are formed one after the
+// other from the per-node projections K and M (acoustic fields 0 and 4
+// first, then the entropy and shear fields, whose node components are read
+// again), so that only one field's stencil values are live.  The one
+// definition every sweep uses: a face's flux does not depend on the kernel
+// that computes it.
+template <int S, class At>
+__host__ __device__ __forceinline__ void weno5_flux(const FluxModel &mdl, const At &at, double F[5])
+{
+    FaceState fs;
+    {
+        double UL[5], UR[5];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+            UL[c] = at(2, c);
+            UR[c] = at(3, c);
+        }
+        face_state<S>(mdl, UL, UR, fs);
+    }
+    double K[6], M[6];                              // b K and M
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+        const double U0 = at(m, 0), U1 = at(m, 1), U2 = at(m, 2), U3 = at(m, 3), U4 = at(m, 4);
+        K[m] = fs.b * fma(-fs.v, U2, fma(-fs.u, U1, fma(-fs.w, U3, fma(fs.q, U0, U4))));
+        M[m] = fma(fs.un, U0, -((S == 0) ? U1 : (S == 1) ? U2 : U3));
+    }
+    double h[5];
+    {
+        double W[6], num[2], den[2], base[2];
+#pragma unroll
+        for (int m = 0; m < 6; ++m) W[m] = fma(fs.d, M[m], K[m]);
+        fast::weno5_field(W, fs.lp[0], fs.ln[0], num[0], den[0], base[0]);
+#pragma unroll
+        for (int m = 0; m < 6; ++m) W[m] = fma(-fs.d, M[m], K[m]);
+        fast::weno5_field(W, fs.lp[4], fs.ln[4], num[1], den[1], base[1]);
+        fast::add_quotients(base[0], num[0], den[0], base[1], num[1], den[1], h[0], h[4]);
+    }
+    const double vel[3] = {fs.u, fs.v, fs.w};
+    double num[3], den[3], base[3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+        const double k = (t == S) ? -2.0 : -2.0 * vel[t];
+        double W[6];
+#pragma unroll
+        for (int m = 0; m < 6; ++m) W[m] = fma(k, K[m], at(m, (t == S) ? 0 : 1 + t));
+        fast::weno5_field(W, fs.lp[1 + t], fs.ln[1 + t], num[t], den[t], base[t]);
+    }
+    fast::add_quotients(base[0], num[0], den[0], base[1], num[1], den[1], h[1], h[2]);
+    h[3] = fma(num[2], fast::reciprocal(den[2]), base[2]);
+    project_back<S>(fs, h, F);
+}
+
+namespace fast {
 
 template <int S, int NS>
 __host__ __device__ __forceinline__ void convective_flux(const FluxModel &mdl, const double st[NS][5], double F[5])
 {
+    if (NS == 6) {
+        weno5_flux<S>(mdl, [&](int m, int c) { return st[m][c]; }, F);
+        return;
+    }
     constexpr int K0 = (NS == 6) ? 2 : 1;
-    const double gamma = mdl.gamma;
-    const double g1 = gamma - 1.0;
-    const double *UL = st[K0];
-    const double *UR = st[K0 + 1];
-    double rL, rR;
-    divide_pair(1.0, UL[0], 1.0, UR[0], rL, rR);
-    const double uL = UL[1] * rL, vL = UL[2] * rL, wL = UL[3] * rL;
-    const double uR = UR[1] * rR, vR = UR[2] * rR, wR = UR[3] * rR;
-    const double hTL = fma(gamma, UL[4] * rL, -0.5 * g1 * fma(uL, uL, fma(vL, vL, wL * wL)));
-    const double hTR = fma(gamma, UR[4] * rR, -0.5 * g1 * fma(uR, uR, fma(vR, vR, wR * wR)));
-    double u, v, w, hT;
-    if (mdl.roe) {
-        const double D = sqrt(UR[0] * rL);
-        const double inv = 1.0 / (1.0 + D);
-        u = fma(D, uR, uL) * inv;
-        v = fma(D, vR, vL) * inv;
-        w = fma(D, wR, wL) * inv;
-        hT = fma(D, hTR, hTL) * inv;
-    } else {
-        u = 0.5 * (uL + uR);
-        v = 0.5 * (vL + vR);
-        w = 0.5 * (wL + wR);
-        hT = 0.5 * (hTL + hTR);
-    }
-    const double q = 0.5 * fma(u, u, fma(v, v, w * w));
-    const double c = sqrt(g1 * (hT - q));
-    const double rc = 1.0 / c;
-    const double d = 0.5 * rc;
-    const double b = 0.5 * g1 * rc * rc;
-    const double vel[3] = {u, v, w};
-    const double un = vel[S];
-    const double lam[5] = {un - c, un, un, un, un + c};
-    double lp[5], ln[5];
-    if (mdl.sw) {
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {
-            const double root = sqrt(fma(lam[r], lam[r], 1.0e-6));
-            lp[r] = 0.5 * (lam[r] + root);
-            ln[r] = 0.5 * (lam[r] - root);
-        }
-    } else {
-        const double star = fabs(un) + c;
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {
-            lp[r] = 0.5 * (lam[r] + star);
-            ln[r] = 0.5 * (lam[r] - star);
-        }
-    }
-    // characteristic variables: per stencil node K = q U0 - vel.mom + U4 and
-    // M = un U0 - U_{1+S}; the fields are formed one at a time from them
-    // (acoustic fields 0 and 4, then the entropy and shear fields), so that
-    // only one field's stencil values are live at once
-    const double m2b = -2.0 * b;
-    double sh[3];
-#pragma unroll
-    for (int t = 0; t < 3; ++t) sh[t] = m2b * vel[t];
-    double K[NS], M[NS];
+    FaceState fs;
+    face_state<S>(mdl, st[K0], st[K0 + 1], fs);
+    const double vel[3] = {fs.u, fs.v, fs.w};
+    double W[5][NS];
 #pragma unroll
     for (int m = 0; m < NS; ++m) {
         const double *U = st[m];
-        K[m] = fma(q, U[0], U[4]) - fma(u, U[1], fma(v, U[2], w * U[3]));
-        M[m] = fma(un, U[0], -U[1 + S]);
+        const double K = fs.b * fma(-fs.u, U[1], fma(-fs.v, U[2], fma(-fs.w, U[3], fma(fs.q, U[0], U[4]))));
+        const double M = fma(fs.un, U[0], -U[1 + S]);
+        W[0][m] = fma(fs.d, M, K);
+        W[4][m] = fma(-fs.d, M, K);
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            W[1 + t][m] = (t == S) ? fma(-2.0, K, U[0]) : fma(-2.0 * vel[t], K, U[1 + t]);
     }
     double h[5];
-    if (NS == 6) {
-        double num[5], den[5];
-        {
-            double wa[6], wb[6];
 #pragma unroll
-            for (int m = 0; m < 6; ++m) {
-                const double bK = b * K[m], dM = d * M[m];
-                wa[m] = bK + dM;
-                wb[m] = bK - dM;
-            }
-            weno5_field_parts(wa, lp[0], ln[0], num[0], den[0]);
-            weno5_field_parts(wb, lp[4], ln[4], num[4], den[4]);
-        }
-        divide_pair(num[0], den[0], num[4], den[4], h[0], h[4]);
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            double wf[6];
-#pragma unroll
-            for (int m = 0; m < 6; ++m) wf[m] = (t == S) ? fma(m2b, K[m], st[m][0]) : fma(sh[t], K[m], st[m][1 + t]);
-            weno5_field_parts(wf, lp[1 + t], ln[1 + t], num[1 + t], den[1 + t]);
-        }
-        divide_pair(num[1], den[1], num[2], den[2], h[1], h[2]);
-        h[3] = num[3] / den[3];
-    } else {
-        double W[5][NS];
-#pragma unroll
-        for (int m = 0; m < NS; ++m) {
-            const double bK = b * K[m], dM = d * M[m];
-            W[0][m] = bK + dM;
-            W[4][m] = bK - dM;
-#pragma unroll
-            for (int t = 0; t < 3; ++t) W[1 + t][m] = (t == S) ? fma(m2b, K[m], st[m][0]) : fma(sh[t], K[m], st[m][1 + t]);
-        }
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {
-            const double hp = weno3(lp[r] * W[r][0], lp[r] * W[r][1], lp[r] * W[r][2]);
-            const double hn = weno3(ln[r] * W[r][3], ln[r] * W[r][2], ln[r] * W[r][1]);
-            h[r] = hp + hn;
-        }
+    for (int r = 0; r < 5; ++r) {
+        const double hp = weno3(fs.lp[r] * W[r][0], fs.lp[r] * W[r][1], fs.lp[r] * W[r][2]);
+        const double hn = weno3(fs.ln[r] * W[r][3], fs.ln[r] * W[r][2], fs.ln[r] * W[r][1]);
+        h[r] = hp + hn;
     }
-    // F = R h with the right eigenvectors along S
-    const double ha = h[0] + h[4], hd = h[4] - h[0];
-    F[0] = ha + h[1 + S];
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        double acc = fma(vel[m], ha, (m == S) ? c * hd : 0.0);
-        acc = (m == S) ? fma(vel[m], h[1 + S], acc) : acc + h[1 + m];
-        F[1 + m] = acc;
-    }
-    double e = fma(hT, ha, un * c * hd);
-#pragma unroll
-    for (int t = 0; t < 3; ++t) e = fma((t == S) ? fma(un, un, -q) : vel[t], h[1 + t], e);
-    F[4] = e;
+    project_back<S>(fs, h, F);
 }
 
+// Differences across a node along the transverse axis T: velocity
+// components S and T of its +T neighbour R less those of its -T neighbour L
+// (a face along S needs no other transverse gradient).
+template <int S, int T>
+__host__ __device__ __forceinline__ void transverse_difference(const double L[5], const double R[5], double out[2])
+{
+    double rL, rR;
+    divide_pair(1.0, L[0], 1.0, R[0], rL, rR);
+    out[0] = fma(R[1 + S], rR, -(L[1 + S] * rL));
+    out[1] = fma(R[1 + T], rR, -(L[1 + T] * rL));
+}
+
+// Viscous flux at the face between P and its +S neighbour E from their
+// states and transverse differences (tP, tE: [0..1] along the first
+// tangential axis, [2..3] along the second).
 template <int S>
 __host__ __device__ __forceinline__ void viscous_flux(const FluxModel &mdl, const double dd[3], const double P[5],
-                                             const double E[5], const double nb[8][5], double F[5])
+                                                      const double E[5], const double tP[4], const double tE[4],
+                                                      double F[5])
 {
     constexpr int TA = (S == 0) ? 1 : 0;
     constexpr int TB = (S == 2) ? 1 : 2;
-    const double rP = 1.0 / P[0], rE = 1.0 / E[0];
+    double rP, rE;
+    divide_pair(1.0, P[0], 1.0, E[0], rP, rE);
     const double velP[3] = {P[1] * rP, P[2] * rP, P[3] * rP};
     const double velE[3] = {E[1] * rE, E[2] * rE, E[3] * rE};
     const double rcv = 1.0 / mdl.cv;
     const double TP = (P[4] * rP - 0.5 * fma(velP[0], velP[0], fma(velP[1], velP[1], velP[2] * velP[2]))) * rcv;
     const double TE = (E[4] * rE - 0.5 * fma(velE[0], velE[0], fma(velE[1], velE[1], velE[2] * velE[2]))) * rcv;
-    double rn[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) rn[q] = 1.0 / nb[q][0];
-    double g[3][3];
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        g[m][S] = (velE[m] - velP[m]) * dd[S];
-        g[m][TA] = 0.25 * dd[TA] *
-                   (fma(nb[1][1 + m], rn[1], nb[5][1 + m] * rn[5]) - fma(nb[0][1 + m], rn[0], nb[4][1 + m] * rn[4]));
-        g[m][TB] = 0.25 * dd[TB] *
-                   (fma(nb[3][1 + m], rn[3], nb[7][1 + m] * rn[7]) - fma(nb[2][1 + m], rn[2], nb[6][1 + m] * rn[6]));
-    }
+    const double qa = 0.25 * dd[TA], qb = 0.25 * dd[TB];
+    const double gSA = qa * (tP[0] + tE[0]), gAA = qa * (tP[1] + tE[1]);       // d u_S / d a, d u_a / d a
+    const double gSB = qb * (tP[2] + tE[2]), gBB = qb * (tP[3] + tE[3]);
+    const double gSS = (velE[S] - velP[S]) * dd[S];
+    const double gAS = (velE[TA] - velP[TA]) * dd[S], gBS = (velE[TB] - velP[TB]) * dd[S];
     const double Ts = 0.5 * (TP + TE) * mdl.refT;
-    const double mu = mdl.refMu * (1.458e-6 * Ts * sqrt(Ts) / (Ts + 110.4));
+    const double mu = (mdl.refMu * 1.458e-6) * (Ts * root(Ts)) * reciprocal(Ts + 110.4);
     const double heatK = mdl.gamma * mdl.cv * (1.0 / 0.71) * mu;
-    const double divV = g[0][0] + g[1][1] + g[2][2];
+    const double divV = gSS + gAA + gBB;
     F[0] = 0.0;
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        F[1 + m] = (m == S) ? mu * fma(2.0, g[S][S], (-2.0 / 3.0) * divV) : mu * (g[m][S] + g[S][m]);
-    }
+    F[1 + S] = mu * fma(2.0, gSS, (-2.0 / 3.0) * divV);
+    F[1 + TA] = mu * (gAS + gSA);
+    F[1 + TB] = mu * (gBS + gSB);
     const double uh = 0.5 * (velP[0] + velE[0]);
     const double vh = 0.5 * (velP[1] + velE[1]);
     const double wh = 0.5 * (velP[2] + velE[2]);
     F[4] = fma(heatK, (TE - TP) * dd[S], fma(F[1], uh, fma(F[2], vh, F[3] * wh)));
+}
+
+// The same from the eight neighbours nb of the exact form above.
+template <int S>
+__host__ __device__ __forceinline__ void viscous_flux(const FluxModel &mdl, const double dd[3], const double P[5],
+                                                      const double E[5], const double nb[8][5], double F[5])
+{
+    constexpr int TA = (S == 0) ? 1 : 0;
+    constexpr int TB = (S == 2) ? 1 : 2;
+    double tP[4], tE[4];
+    transverse_difference<S, TA>(nb[0], nb[1], tP);
+    transverse_difference<S, TB>(nb[2], nb[3], tP + 2);
+    transverse_difference<S, TA>(nb[4], nb[5], tE);
+    transverse_difference<S, TB>(nb[6], nb[7], tE + 2);
+    viscous_flux<S>(mdl, dd, P, E, tP, tE, F);
 }
 
 }  // namespace fast

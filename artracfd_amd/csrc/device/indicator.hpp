@@ -124,66 +124,6 @@ __host__ __device__ __forceinline__ double weno5_weight_deviation(double f0, dou
     return fabs(t0 * inv - 0.1) + fabs(t1 * inv - 0.6) + fabs(t2 * inv - 0.3);
 }
 
-// Face state shared by the WENO and linear fluxes (fast arithmetic).
-struct FaceState {
-    double u, v, w, hT, c, q, b, d, un, g1;
-    double lp[5], ln[5];
-};
-
-// b = (gamma - 1) / (2 c^2) and d = 1 / (2 c) of the eigenvectors; only the
-// characteristic projections need them.
-__host__ __device__ __forceinline__ void face_scales(FaceState &fs)
-{
-    const double rc = 1.0 / fs.c;
-    fs.d = 0.5 * rc;
-    fs.b = 0.5 * fs.g1 * rc * rc;
-}
-
-template <int S>
-__host__ __device__ __forceinline__ void face_state(const FluxModel &mdl, const double UL[5], const double UR[5], FaceState &fs)
-{
-    const double gamma = mdl.gamma, g1 = gamma - 1.0;
-    double rL, rR;
-    fast::divide_pair(1.0, UL[0], 1.0, UR[0], rL, rR);
-    const double uL = UL[1] * rL, vL = UL[2] * rL, wL = UL[3] * rL;
-    const double uR = UR[1] * rR, vR = UR[2] * rR, wR = UR[3] * rR;
-    const double hTL = fma(gamma, UL[4] * rL, -0.5 * g1 * fma(uL, uL, fma(vL, vL, wL * wL)));
-    const double hTR = fma(gamma, UR[4] * rR, -0.5 * g1 * fma(uR, uR, fma(vR, vR, wR * wR)));
-    if (mdl.roe) {
-        const double D = sqrt(UR[0] * rL);
-        const double inv = 1.0 / (1.0 + D);
-        fs.u = fma(D, uR, uL) * inv;
-        fs.v = fma(D, vR, vL) * inv;
-        fs.w = fma(D, wR, wL) * inv;
-        fs.hT = fma(D, hTR, hTL) * inv;
-    } else {
-        fs.u = 0.5 * (uL + uR);
-        fs.v = 0.5 * (vL + vR);
-        fs.w = 0.5 * (wL + wR);
-        fs.hT = 0.5 * (hTL + hTR);
-    }
-    fs.q = 0.5 * fma(fs.u, fs.u, fma(fs.v, fs.v, fs.w * fs.w));
-    fs.c = sqrt(g1 * (fs.hT - fs.q));
-    fs.g1 = g1;
-    fs.un = (S == 0) ? fs.u : (S == 1) ? fs.v : fs.w;
-    const double lam[5] = {fs.un - fs.c, fs.un, fs.un, fs.un, fs.un + fs.c};
-    if (mdl.sw) {
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {
-            const double root = sqrt(fma(lam[r], lam[r], 1.0e-6));
-            fs.lp[r] = 0.5 * (lam[r] + root);
-            fs.ln[r] = 0.5 * (lam[r] - root);
-        }
-    } else {
-        const double star = fabs(fs.un) + fs.c;
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {
-            fs.lp[r] = 0.5 * (lam[r] + star);
-            fs.ln[r] = 0.5 * (lam[r] - star);
-        }
-    }
-}
-
 // Characteristic variables W = L U of one state (structured form).
 template <int S>
 __host__ __device__ __forceinline__ void characteristic(const FaceState &fs, const double U[5], double W[5])
@@ -197,25 +137,6 @@ __host__ __device__ __forceinline__ void characteristic(const FaceState &fs, con
     W[4] = bK - dM;
 #pragma unroll
     for (int t = 0; t < 3; ++t) W[1 + t] = (t == S) ? fma(m2b, K, U[0]) : fma(m2b * vel[t], K, U[1 + t]);
-}
-
-// F = R h (right eigenvectors along S).
-template <int S>
-__host__ __device__ __forceinline__ void project_back(const FaceState &fs, const double h[5], double F[5])
-{
-    const double vel[3] = {fs.u, fs.v, fs.w};
-    const double ha = h[0] + h[4], hd = h[4] - h[0];
-    F[0] = ha + h[1 + S];
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        double acc = fma(vel[m], ha, (m == S) ? fs.c * hd : 0.0);
-        acc = (m == S) ? fma(vel[m], h[1 + S], acc) : acc + h[1 + m];
-        F[1 + m] = acc;
-    }
-    double e = fma(fs.hT, ha, fs.un * fs.c * hd);
-#pragma unroll
-    for (int t = 0; t < 3; ++t) e = fma((t == S) ? fma(fs.un, fs.un, -fs.q) : vel[t], h[1 + t], e);
-    F[4] = e;
 }
 
 // Linear fifth-order upwind flux: the WENO5 flux with every nonlinear weight
@@ -235,9 +156,8 @@ __host__ __device__ __forceinline__ void linear_averages(const double st[6][5], 
 }
 
 template <int S>
-__host__ __device__ __forceinline__ void linear_flux_from(FaceState fs, const double Up[5], const double Un[5], double F[5])
+__host__ __device__ __forceinline__ void linear_flux_from(const FaceState &fs, const double Up[5], const double Un[5], double F[5])
 {
-    face_scales(fs);
     double Wp[5], Wn[5], h[5];
     characteristic<S>(fs, Up, Wp);
     characteristic<S>(fs, Un, Wn);
@@ -265,11 +185,7 @@ __device__ __forceinline__ void face_state_mean(double gamma, const double nL[4]
 // Velocities and total enthalpy of one node (as face_state computes them per side).
 __device__ __forceinline__ void node_velocity_enthalpy(double gamma, const double U[5], double nv[4])
 {
-    const double r = 1.0 / U[0];
-    nv[0] = U[1] * r;
-    nv[1] = U[2] * r;
-    nv[2] = U[3] * r;
-    nv[3] = fma(gamma, U[4] * r, -0.5 * (gamma - 1.0) * fma(nv[0], nv[0], fma(nv[1], nv[1], nv[2] * nv[2])));
+    velocity_enthalpy(gamma, U, fast::reciprocal(U[0]), nv);
 }
 
 // Sum and difference of the two linear combinations, sum c+ U + sum c- U and
@@ -342,151 +258,30 @@ __host__ __device__ __forceinline__ void linear_flux(const FaceState &fs, const 
     linear_flux_from<S>(fs, Up, Un, F);
 }
 
-// The WENO5 sum of one characteristic field of the face flux, h_r =
-// WENO5(lp W_r) over the nodes f-2 .. f+2 plus WENO5(ln W_r) over the
-// mirrored nodes f+3 .. f-1 (for a line held node-major, [n][5]), as a
-// numerator and denominator (fs needs face_scales applied).
-template <int S>
-__device__ __forceinline__ void weno_field_parts(const FaceState &fs, const double *st, int f, int r, bool sw,
-                                                 double &num, double &den)
-{
-    const double vel[3] = {fs.u, fs.v, fs.w};
-    const double m2b = -2.0 * fs.b;
-    const bool edge = (r == 0) || (r == 4);
-    const double sgn = (r == 0) ? 1.0 : -1.0;
-    const int t = edge ? 0 : r - 1;
-    const double cK = (t == S) ? m2b : m2b * ((t == 0) ? vel[0] : (t == 1) ? vel[1] : vel[2]);
-    const int idx = (t == S) ? 0 : 1 + t;
-    const double lam = (r == 0) ? fs.un - fs.c : (r == 4) ? fs.un + fs.c : fs.un;
-    double lp, ln;
-    if (sw) {
-        const double root = sqrt(fma(lam, lam, 1.0e-6));
-        lp = 0.5 * (lam + root);
-        ln = 0.5 * (lam - root);
-    } else {
-        const double star = fabs(fs.un) + fs.c;
-        lp = 0.5 * (lam + star);
-        ln = 0.5 * (lam - star);
-    }
-    double w[6];                                    // the field's value at nodes f-2 .. f+3
-#pragma unroll
-    for (int m = 0; m < 6; ++m) {
-        const int node = f - 2 + m;
-        const double *Un = st + node * 5;
-        const double U0 = Un[0], U1 = Un[1], U2 = Un[2], U3 = Un[3], U4 = Un[4];
-        const double K = fma(fs.q, U0, U4) - fma(fs.u, U1, fma(fs.v, U2, fs.w * U3));
-        const double M = fma(fs.un, U0, -Un[1 + S]);
-        const double bK = fs.b * K, dM = fs.d * M;
-        const double Ui = Un[idx];
-        w[m] = edge ? bK + sgn * dM : fma(cK, K, Ui);
-    }
-    fast::weno5_field_parts(w, lp, ln, num, den);
-}
-
-// The field sums of a face from their numerators and denominators
-// num/den[r] = parts[2 r], parts[2 r + 1], with the divisions
-// fast::convective_flux makes (fields 0 and 4, and 1 and 2, share one), so
-// that h is bit-identical to it.
-__host__ __device__ __forceinline__ void fields_from_parts(const double *parts, double h[5])
-{
-    fast::divide_pair(parts[0], parts[1], parts[8], parts[9], h[0], h[4]);
-    fast::divide_pair(parts[2], parts[3], parts[4], parts[5], h[1], h[2]);
-    h[3] = parts[6] / parts[7];
-}
-
 // The fast WENO5 flux of the face between nodes f and f + 1 of a line held
-// node-major, [n][5] (in LDS), bit-identical to fast::convective_flux on the same
-// six nodes.  The fields are formed one at a time from the per-node
-// projections K and M (acoustic fields 0 and 4 first, then the entropy and
-// shear fields, whose node components are read again), so that only one
-// field's stencil values are live: the sweep then fits in 128 registers.
+// node-major, [n][5] (in LDS).
 template <int S>
 __device__ __forceinline__ void weno_flux_line(const FluxModel &mdl, const double *st, int f, double F[5])
 {
-    FaceState fs;
-    {
-        double UL[5], UR[5];
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            UL[c] = st[f * 5 + c];
-            UR[c] = st[(f + 1) * 5 + c];
-        }
-        face_state<S>(mdl, UL, UR, fs);
-    }
-    face_scales(fs);
-    double K[6], M[6];
-#pragma unroll
-    for (int m = 0; m < 6; ++m) {
-        const int node = f - 2 + m;
-        const double *Un = st + node * 5;
-        const double U0 = Un[0], U1 = Un[1], U2 = Un[2], U3 = Un[3], U4 = Un[4];
-        K[m] = fma(fs.q, U0, U4) - fma(fs.u, U1, fma(fs.v, U2, fs.w * U3));
-        M[m] = fma(fs.un, U0, -Un[1 + S]);
-    }
-    double parts[10];
-    {
-        double wa[6], wb[6];
-#pragma unroll
-        for (int m = 0; m < 6; ++m) {
-            const double bK = fs.b * K[m], dM = fs.d * M[m];
-            wa[m] = bK + dM;
-            wb[m] = bK - dM;
-        }
-        fast::weno5_field_parts(wa, fs.lp[0], fs.ln[0], parts[0], parts[1]);
-        fast::weno5_field_parts(wb, fs.lp[4], fs.ln[4], parts[8], parts[9]);
-    }
-    const double vel[3] = {fs.u, fs.v, fs.w};
-    const double m2b = -2.0 * fs.b;
-#pragma unroll
-    for (int t = 0; t < 3; ++t) {
-        const double cK = (t == S) ? m2b : m2b * vel[t];
-        const int idx = (t == S) ? 0 : 1 + t;
-        double w[6];
-#pragma unroll
-        for (int m = 0; m < 6; ++m) w[m] = fma(cK, K[m], st[(f - 2 + m) * 5 + idx]);
-        fast::weno5_field_parts(w, fs.lp[1 + t], fs.ln[1 + t], parts[2 + 2 * t], parts[3 + 2 * t]);
-    }
-    double h[5];
-    fields_from_parts(parts, h);
-    project_back<S>(fs, h, F);
+    const double *p = st + (f - 2) * 5;
+    weno5_flux<S>(mdl, [=](int m, int c) { return p[m * 5 + c]; }, F);
 }
 
-// Full WENO5 flux from the same face state (matches fast::convective_flux).
-// With label != nullptr also returns the weight-deviation label.
+// Weight-deviation label of a face: the largest over the characteristic
+// fields and the two split sides.
 template <int S>
-__host__ __device__ __forceinline__ void weno_flux(FaceState fs, const double st[6][5], double F[5], double *label)
+__host__ __device__ __forceinline__ double weno_label(const FaceState &fs, const double st[6][5])
 {
-    face_scales(fs);
-    double W[5][6];
+    double W[6][5], dev = 0.0;
 #pragma unroll
-    for (int m = 0; m < 6; ++m) {
-        double t[5];
-        characteristic<S>(fs, st[m], t);
-#pragma unroll
-        for (int r = 0; r < 5; ++r) W[r][m] = t[r];
-    }
-    double h[5], num[5], den[5];
-    double dev = 0.0;
+    for (int m = 0; m < 6; ++m) characteristic<S>(fs, st[m], W[m]);
 #pragma unroll
     for (int r = 0; r < 5; ++r) {
         const double lp = fs.lp[r], ln = fs.ln[r];
-        fast::weno5_field_parts(W[r], lp, ln, num[r], den[r]);
-        if (label) {
-            dev = fmax(dev, weno5_weight_deviation(lp * W[r][0], lp * W[r][1], lp * W[r][2], lp * W[r][3],
-                                                   lp * W[r][4]));
-            dev = fmax(dev, weno5_weight_deviation(ln * W[r][5], ln * W[r][4], ln * W[r][3], ln * W[r][2],
-                                                   ln * W[r][1]));
-        }
+        dev = fmax(dev, weno5_weight_deviation(lp * W[0][r], lp * W[1][r], lp * W[2][r], lp * W[3][r], lp * W[4][r]));
+        dev = fmax(dev, weno5_weight_deviation(ln * W[5][r], ln * W[4][r], ln * W[3][r], ln * W[2][r], ln * W[1][r]));
     }
-    if (label) *label = dev;
-    double parts[10];
-#pragma unroll
-    for (int r = 0; r < 5; ++r) {
-        parts[2 * r] = num[r];
-        parts[2 * r + 1] = den[r];
-    }
-    fields_from_parts(parts, h);
-    project_back<S>(fs, h, F);
+    return dev;
 }
 
 // ------------------------------------------------------------ the MLP
