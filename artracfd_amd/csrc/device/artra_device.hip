@@ -1,15 +1,11 @@
 // artra_device.hip - device side of libartra_hip for gfx950 (MI355X).
 //
 // Kernels
-//   sweep_x        directional sweep along x (fluid_dynamics.c:157-274 for
-//                  s = X): one thread per face, faces of consecutive lines
-//                  flattened so every 256-thread block updates 255 nodes;
-//                  face fluxes meet in LDS and each node takes its left and
-//                  right flux from there (LU + SolveOperator fused).
-//   sweep_march    sweeps along y and z: a thread walks a column segment,
-//                  carrying the stencil window and the previous face flux in
-//                  registers, so each face flux is computed once; loads are
-//                  coalesced along x across the wavefront.
+//   sweep_tile     one Runge-Kutta stage along one axis
+//                  (fluid_dynamics.c:157-274): a tile of line segments in
+//                  LDS, one thread per face, then the node updates (LU +
+//                  SolveOperator fused) in memory order.
+//   rk_line        all stages of one directional operator, lines in LDS.
 //   bc_group       a group of TreatBoundary boxes whose nodes do not
 //                  interact (boundary_treatment.c:28-192).
 //   ib_fill        the immersed-boundary fill of one ghost layer (or of all
@@ -59,9 +55,6 @@ int Fail(const char *fmt, ...)
         if (e_ != hipSuccess) return Fail("%s failed: %s", #expr, hipGetErrorString(e_));       \
     } while (0)
 
-constexpr int kXBlock = 256;        // threads (faces) per sweep_x block
-constexpr int kMarchX = 64;         // x extent of a sweep_march block (one wavefront)
-constexpr int kMarchT = 4;          // transverse extent of a sweep_march block
 constexpr int kMaxGroup = 8;        // boxes per bc_group launch
 constexpr int kListBlocks = 768;    // persistent blocks of rk_line_list (3 per CU)
 constexpr int kMarchChunk = ARTRA_DEV_MARCH_CHUNK;   // steps per device-stepped march call (the record's length)
@@ -95,7 +88,7 @@ struct StageArgs {
     const double *Utn;              // level read by the stencils
     const double *Uto;              // level of the a-term
     double *Utm;                    // level written
-    const uint8_t *fluid;
+    const uint8_t *fluid;           // null in a sweep where every interior node is fluid
     double a, b, r;                 // U_tm = a U_to + b (U_tn + r Phi)
     int accumulate;                 // U_tm += b r Phi (unsplit, non-x)
     int toIsTn;                     // U_to and U_tn are the same level
@@ -140,53 +133,11 @@ __device__ __forceinline__ void LoadNode(const double *U, long idx, double out[5
     for (int c = 0; c < 5; ++c) out[c] = p[c];
 }
 
-// Solution operator of one node (fluid_dynamics.c:243-274).  FAST evaluates
-// the same expression with fused multiply-adds.
-template <bool VISC, bool FAST>
-__device__ __forceinline__ void UpdateNode(const StageArgs &sa, long idx, const double FL[5], const double FR[5],
-                                           const double FvL[5], const double FvR[5], const double Un[5])
-{
-    double phi[5];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-        if (FAST) phi[c] = VISC ? (FL[c] - FR[c]) + (FvR[c] - FvL[c]) : FL[c] - FR[c];
-        else phi[c] = VISC ? ((FL[c] - FR[c]) + FvR[c]) - FvL[c] : ((FL[c] - FR[c]) + 0.0) - 0.0;
-    }
-    if (sa.accumulate) {
-        const double br = sa.b * sa.r;
-        double *um = NodeAt(sa.Utm, idx);
-#pragma unroll
-        for (int c = 0; c < 5; ++c) um[c] = FAST ? fma(br, phi[c], um[c]) : um[c] + br * phi[c];
-        return;
-    }
-    double Uo[5];
-    if (sa.toIsTn) {
-#pragma unroll
-        for (int c = 0; c < 5; ++c) Uo[c] = Un[c];
-    } else {
-        LoadNode(sa.Uto, idx, Uo);
-    }
-    double *um = NodeAt(sa.Utm, idx);
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-        if (FAST) um[c] = fma(sa.a, Uo[c], sa.b * fma(sa.r, phi[c], Un[c]));
-        else um[c] = sa.a * Uo[c] + sa.b * (Un[c] + sa.r * phi[c]);
-    }
-}
-
 template <int S, int NS, bool FAST>
 __device__ __forceinline__ void ConvFlux(const FluxModel &mdl, const double st[NS][5], double F[5])
 {
     if (FAST) artra::fast::convective_flux<S, NS>(mdl, st, F);
     else artra::convective_flux<S, NS>(mdl, st, F);
-}
-
-template <int S, bool FAST>
-__device__ __forceinline__ void ViscFlux(const FluxModel &mdl, const double dd[3], const double P[5], const double E[5],
-                                         const double nb[8][5], double F[5])
-{
-    if (FAST) artra::fast::viscous_flux<S>(mdl, dd, P, E, nb, F);
-    else artra::viscous_flux<S>(mdl, dd, P, E, nb, F);
 }
 
 // Neighbour states of the viscous face stencil at (P, E = P + e_S).
@@ -208,113 +159,293 @@ __device__ __forceinline__ void LoadViscousNeighbours(const Grid &g, const doubl
 }
 
 // ------------------------------------------------------------------ sweeps
-template <int NS, bool VISC, bool FAST>
-__global__ __launch_bounds__(kXBlock) void sweep_x(Grid g, StageArgs sa, FluxModel mdl)
+// Blocks are dealt to the XCDs round robin; this bijection gives each XCD a
+// contiguous run of lines, so lines that share cache lines (adjacent x for
+// y and z lines) meet in the same L2.
+__device__ __forceinline__ long XcdLine(long b, long nb)
 {
-    if (!ResolveStep(sa)) return;
-    constexpr int SL = (NS == 6) ? -2 : -1;
-    constexpr int K0 = -SL;
-    __shared__ double sF[5][kXBlock];
-    __shared__ double sFv[VISC ? 5 : 1][kXBlock];
-    const int faces = g.hi[0] - g.lo[0] + 1;           // faces per x line
-    const int ny = g.hi[1] - g.lo[1];
-    const long total = (long)faces * ny * (g.hi[2] - g.lo[2]);
-    const long gface = (long)blockIdx.x * (kXBlock - 1) + threadIdx.x;
-    int f = 0, j = 0, k = 0;
-    double Un[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (gface < total) {
-        const long line = gface / faces;
-        f = (int)(gface - line * faces);
-        j = g.lo[1] + (int)(line % ny);
-        k = g.lo[2] + (int)(line / ny);
-        const int i = g.lo[0] - 1 + f;                 // face between i and i + 1
-        const int base = Index(g, i, j, k);
-        double st[NS][5];
-#pragma unroll
-        for (int m = 0; m < NS; ++m) LoadNode(sa.Utn, base + SL + m, st[m]);
-        double F[5];
-        ConvFlux<0, NS, FAST>(mdl, st, F);
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            sF[c][threadIdx.x] = F[c];
-            Un[c] = st[K0 + 1][c];                     // node i + 1, updated by this thread
-        }
-        if (VISC) {
-            double nb[8][5], Fv[5];
-            LoadViscousNeighbours<0>(g, sa.Utn, base, nb);
-            ViscFlux<0, FAST>(mdl, sa.dd, st[K0], st[K0 + 1], nb, Fv);
-#pragma unroll
-            for (int c = 0; c < 5; ++c) sFv[VISC ? c : 0][threadIdx.x] = Fv[c];
-        }
+    const long q = nb / 8, rem = nb % 8;
+    const long x = b % 8, i = b / 8;
+    return (x < rem) ? x * (q + 1) + i : rem * (q + 1) + (x - rem) * q + i;
+}
+
+// One Runge-Kutta stage along S, a tile of P lines and seg nodes a block.
+// The tile's nodes (seg and half a stencil either side) are copied to LDS
+// once, consecutive doubles by consecutive lanes; then each thread computes
+// one face, and the nodes are updated component by component in the order of
+// the copy, so that every global access is coalesced and a face is computed
+// once per segment.  The P lines of a tile are neighbours in y (x sweeps) or
+// in x (y and z sweeps).  Everything the tile needs from memory is asked for
+// at once, before anything waits: states, the a-term's states, the fluid
+// flags and the step; three to four wavefronts per SIMD then hide most of
+// one memory latency per tile, but not of several in a row.
+//
+// The kernel replaces a face per thread straight from memory (x) and marches
+// of 32 nodes per thread in a register window (y, z): those asked the L1 for
+// 30 to 70 strided 8-byte loads per face, and the marches left small grids
+// with a few hundred blocks.
+struct SweepTile {
+    int P;                          // lines per tile
+    int seg, nseg;                  // nodes per segment, segments per line
+    int groups, others;             // tiles across the line axis, extent of the third axis
+    int rows;                       // nodes per line in LDS: seg + 2 halo
+    int perPass;                    // x: threads per line; y and z: rows of the tile the block copies at a time
+    int threads;                    // of a block
+    int tiles;
+};
+
+constexpr int kTileThreads = 256;
+constexpr int kTileIn = 11, kTileOut = 6;            // doubles per thread of a tile's states and of its a-term
+
+// Doubles of LDS: node states, face fluxes, with the viscous flux the
+// transverse differences of every node a face touches and then, in their
+// place, the viscous fluxes, and the a-term's states.
+__host__ __device__ __forceinline__ int TileSpare(int P, int seg, bool visc)
+{
+    const int faces = P * (seg + 1), differences = (faces + P) * 4;
+    return !visc ? 0 : (differences > 5 * faces) ? differences : 5 * faces;
+}
+
+__host__ __device__ __forceinline__ size_t TileDoubles(int P, int seg, int rows, bool visc)
+{
+    return (size_t)5 * P * (rows + (seg + 1) + seg) + TileSpare(P, seg, visc);
+}
+
+// The transverse differences of node idx (see viscous_flux): components S
+// and the tangential one along each tangential axis.
+template <int S>
+__device__ __forceinline__ void TransverseDifferences(const Grid &g, const double *U, int idx, double t[4])
+{
+    constexpr int TA = (S == 0) ? 1 : 0;
+    constexpr int TB = (S == 2) ? 1 : 2;
+    const int stride[3] = {1, g.nx, g.nx * g.ny};
+    double L[5], R[5];
+    LoadNode(U, idx - stride[TA], L);
+    LoadNode(U, idx + stride[TA], R);
+    artra::fast::transverse_difference<S, TA>(L, R, t);
+    LoadNode(U, idx - stride[TB], L);
+    LoadNode(U, idx + stride[TB], R);
+    artra::fast::transverse_difference<S, TB>(L, R, t + 2);
+}
+
+// A tile's place: the node index of its first line's first node, its lines
+// and its nodes along S.
+struct TileAt {
+    int first, lines, len;
+};
+
+template <int S>
+__device__ __forceinline__ TileAt TilePlace(const Grid &g, const SweepTile &ts, int tile)
+{
+    constexpr int L = (S == 0) ? 1 : 0;              // the axis across the tile's lines
+    constexpr int O = (S == 2) ? 1 : 2;              // the third
+    int grp, sg, o;
+    if (S == 0) {                                    // segments of a line side by side
+        sg = tile % ts.nseg;
+        tile /= ts.nseg;
+        grp = tile % ts.groups;
+        o = tile / ts.groups;
+    } else {                                         // in the order of memory
+        grp = tile % ts.groups;
+        tile /= ts.groups;
+        sg = (S == 1) ? tile % ts.nseg : tile / ts.others;
+        o = (S == 1) ? tile / ts.nseg : tile % ts.others;
     }
-    __syncthreads();
-    // node between this thread's face and the next thread's face
-    if (threadIdx.x < kXBlock - 1 && gface + 1 < total && f + 1 < faces) {
-        const int i = g.lo[0] + f;
-        const int idx = Index(g, i, j, k);
-        if (sa.fluid[idx]) {
-            double FL[5], FR[5], FvL[5], FvR[5];
-#pragma unroll
-            for (int c = 0; c < 5; ++c) {
-                FL[c] = sF[c][threadIdx.x];
-                FR[c] = sF[c][threadIdx.x + 1];
-                FvL[c] = VISC ? sFv[VISC ? c : 0][threadIdx.x] : 0.0;
-                FvR[c] = VISC ? sFv[VISC ? c : 0][threadIdx.x + 1] : 0.0;
-            }
-            UpdateNode<VISC, FAST>(sa, idx, FL, FR, FvL, FvR, Un);
-        }
+    int c[3];
+    c[S] = g.lo[S] + sg * ts.seg;
+    c[L] = g.lo[L] + grp * ts.P;
+    c[O] = g.lo[O] + o;
+    TileAt t;
+    t.first = Index(g, c[0], c[1], c[2]);
+    t.lines = min(ts.P, g.hi[L] - c[L]);
+    t.len = min(ts.seg, g.hi[S] - c[S]);
+    return t;
+}
+
+// How the threads share out the doubles of a tile: x, each line's threads
+// take the line's doubles in turn; y and z, whole rows of 5 P contiguous
+// doubles, perPass rows at a time.  Element k of a thread is then k uniform
+// steps from its first, which costs no address arithmetic.
+struct TileShare {
+    int row, col;                   // the first element: x, line and double of the line; y and z, row and double of the row
+    int perPass;                    // doubles (x) or rows (y, z) from one element to the next
+    bool on;
+};
+
+template <int S>
+__device__ __forceinline__ TileShare ShareOf(const SweepTile &ts)
+{
+    const int tid = threadIdx.x;
+    TileShare h;
+    h.perPass = ts.perPass;
+    if (S == 0) {
+        h.row = tid / h.perPass;
+        h.col = tid - h.row * h.perPass;
+        h.on = h.row < ts.P;
+    } else {
+        h.row = tid / (5 * ts.P);
+        h.col = tid - h.row * (5 * ts.P);
+        h.on = h.row < h.perPass;
     }
+    return h;
+}
+
+// A thread's doubles of n nodes per line, from the node `before` ahead of
+// the tile's first.  Addresses are a uniform base and a byte offset.
+template <int S, int N>
+__device__ __forceinline__ void TileFetch(const Grid &g, const double *U, const TileAt &t, const TileShare &h, int before,
+                                          int n, double v[N])
+{
+    const int stride = (S == 2) ? g.nx * g.ny : g.nx;                        // between rows
+    const double *base = U + ((long)t.first - (long)before * ((S == 0) ? 1 : stride)) * 5;
+    const unsigned at = (unsigned)(h.row * stride * 5 + h.col) * 8u;
+    const long step = (S == 0) ? h.perPass : (long)h.perPass * stride * 5;
+    const bool on = h.on && ((S == 0) ? h.row < t.lines : h.col < 5 * t.lines);
+    const int end = (S == 0) ? 5 * n - h.col : n - h.row;
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = (on && k * h.perPass < end) ? *(const double *)((const char *)(base + k * step) + at) : 0.0;
 }
 
 template <int S, int NS, bool VISC, bool FAST>
-__global__ __launch_bounds__(kMarchX *kMarchT) __attribute__((amdgpu_waves_per_eu(2))) void sweep_march(Grid g, StageArgs sa, FluxModel mdl, int segment)
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(FAST ? 3 : 2))) void sweep_tile(
+    Grid g, StageArgs sa, FluxModel mdl, SweepTile ts)
 {
-    if (!ResolveStep(sa)) return;
-    constexpr int SL = (NS == 6) ? -2 : -1;
-    constexpr int K0 = -SL;
-    constexpr int T2 = (S == 1) ? 2 : 1;               // the other transverse axis
-    const int i = g.lo[0] + blockIdx.x * kMarchX + threadIdx.x;
-    const int t2 = g.lo[T2] + blockIdx.y * kMarchT + threadIdx.y;
-    if (i >= g.hi[0] || t2 >= g.hi[T2]) return;
-    const int s0 = g.lo[S] + blockIdx.z * segment;
-    const int s1 = min(g.hi[S], s0 + segment);
-    if (s0 >= s1) return;
-    const int stride = (S == 1) ? g.nx : g.nx * g.ny;
-    const int idx0 = (S == 1) ? Index(g, i, s0, t2) : Index(g, i, t2, s0);
-    // window for the face between s0 - 1 and s0
-    double st[NS][5];
+    constexpr int halo = NS / 2;
+    extern __shared__ double lds[];
+    const int P = ts.P, rows = ts.rows, F = ts.seg + 1, tid = threadIdx.x;
+    double *st = lds;                                // node states: x [P][rows][5], else [rows][P][5]
+    double *fb = st + rows * P * 5;                  // face fluxes: x [P][F][5], else [F][P][5]
+    double *vb = fb + F * P * 5;                     // see TileDoubles
+    const int stride = (S == 0) ? 1 : (S == 1) ? g.nx : g.nx * g.ny;         // along S
+    const int lineStride = (S == 0) ? g.nx : 1, rowStride = (S == 0) ? g.nx : stride;
+    const TileShare h = ShareOf<S>(ts);
+    const TileAt t = TilePlace<S>(g, ts, (int)XcdLine(blockIdx.x, ts.tiles));
+    // the states the update adds to (a-term, or the accumulated level)
+    const double *other = sa.accumulate ? sa.Utm : sa.toIsTn ? nullptr : sa.Uto;
+    double in[kTileIn], out[kTileOut];
+    unsigned fluid = ~0u;                            // bit k: element k belongs to a fluid node
+    TileFetch<S, kTileIn>(g, sa.Utn, t, h, halo, t.len + 2 * halo, in);
+    if (other) TileFetch<S, kTileOut>(g, other, t, h, 0, t.len, out);
+    const bool updates = h.on && ((S == 0) ? h.row < t.lines : h.col < 5 * t.lines);
+    const int endOut = updates ? ((S == 0) ? 5 * t.len - h.col : t.len - h.row) : 0;
+    if (sa.fluid) {
+        fluid = 0u;
 #pragma unroll
-    for (int m = 0; m < NS; ++m) LoadNode(sa.Utn, idx0 + (SL - 1 + m) * stride, st[m]);
-    double FL[5], FvL[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    ConvFlux<S, NS, FAST>(mdl, st, FL);
-    if (VISC) {
-        double nb[8][5];
-        LoadViscousNeighbours<S>(g, sa.Utn, idx0 - stride, nb);
-        ViscFlux<S, FAST>(mdl, sa.dd, st[K0], st[K0 + 1], nb, FvL);
+        for (int k = 0; k < kTileOut; ++k) {
+            if (k * h.perPass >= endOut) continue;
+            const int node = (S == 0) ? h.row * rowStride + (h.col + k * h.perPass) / 5
+                                      : (h.row + k * h.perPass) * rowStride + h.col / 5;
+            fluid |= (unsigned)sa.fluid[t.first + node] << k;
+        }
     }
-    int idx = idx0;
-    for (int s = s0; s < s1; ++s, idx += stride) {
+    const double step = sa.step ? *sa.step : 0.0;
+    // this thread's line and face: face q is the left face of the line's q-th node
+    const int slot = (S == 0) ? h.row : tid % P, q = (S == 0) ? h.col : tid / P;
+    const int lineStep = (S == 0) ? rows * 5 : 5, rowStep = (S == 0) ? 5 : 5 * P;
+    const int faceAt = ((S == 0) ? slot * F * 5 : slot * 5) + q * rowStep;
+    const int diffAt = ((S == 0) ? slot * (F + 1) + q : q * P + slot) * 4;
+    const int left = t.first + slot * lineStride + (q - 1) * stride;         // node index of the face's left node
+    const bool mine = slot < t.lines;
+    if (VISC && FAST) {
+        // rows 0 .. len + 1 of nodes from the one before the segment to the one after it
+        if (mine && q < t.len + 2) {
+            double d[4];
+            TransverseDifferences<S>(g, sa.Utn, left, d);
 #pragma unroll
-        for (int m = 0; m < NS - 1; ++m) {
+            for (int c = 0; c < 4; ++c) vb[diffAt + c] = d[c];
+        }
+    }
+    // element k of a thread: x, double col + k perPass of line row; y and z, row row + k perPass
+    const int shareAt = (S == 0) ? h.col : h.row * 5 * P + h.col, shareStep = (S == 0) ? h.perPass : h.perPass * 5 * P;
+    if (h.on) {
+        const int end = (S == 0) ? 5 * rows - h.col : rows - h.row;
+        double *d = st + ((S == 0) ? h.row * rows * 5 : 0) + shareAt;
 #pragma unroll
-            for (int c = 0; c < 5; ++c) st[m][c] = st[m + 1][c];
+        for (int k = 0; k < kTileIn; ++k) {
+            if (k * h.perPass < end) d[k * shareStep] = in[k];
         }
-        LoadNode(sa.Utn, idx + (SL + NS - 1) * stride, st[NS - 1]);
-        double FR[5], FvR[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (VISC) {
-            // the viscous flux first: its neighbour values are dead before
-            // the characteristic projection needs its registers
-            double nb[8][5];
-            LoadViscousNeighbours<S>(g, sa.Utn, idx, nb);
-            ViscFlux<S, FAST>(mdl, sa.dd, st[K0], st[K0 + 1], nb, FvR);
-        }
-        ConvFlux<S, NS, FAST>(mdl, st, FR);
-        if (sa.fluid[idx]) UpdateNode<VISC, FAST>(sa, idx, FL, FR, FvL, FvR, st[K0]);
+    }
+    if (other && updates) {
+        // each thread reads back only what it writes here
+        double *d = vb + TileSpare(P, ts.seg, VISC) + ((S == 0) ? h.row * ts.seg * 5 : 0) + shareAt;
 #pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            FL[c] = FR[c];
-            FvL[c] = FvR[c];
+        for (int k = 0; k < kTileOut; ++k) {
+            if (k * h.perPass < endOut) d[k * shareStep] = out[k];
         }
+    }
+    __syncthreads();
+    const bool face = mine && q <= t.len;
+    const double *p = st + slot * lineStep + q * rowStep;                    // the face's first stencil node
+    if (VISC) {
+        double Fv[5];
+        if (face) {
+            double A[5], B[5];
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                A[c] = p[(halo - 1) * rowStep + c];
+                B[c] = p[halo * rowStep + c];
+            }
+            if (FAST) {
+                double a[4], b[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    a[c] = vb[diffAt + c];
+                    b[c] = vb[diffAt + ((S == 0) ? 4 : 4 * P) + c];
+                }
+                artra::fast::viscous_flux<S>(mdl, sa.dd, A, B, a, b, Fv);
+            } else {
+                double nb[8][5];
+                LoadViscousNeighbours<S>(g, sa.Utn, left, nb);
+                artra::viscous_flux<S>(mdl, sa.dd, A, B, nb, Fv);
+            }
+        }
+        if (FAST) __syncthreads();                   // the fluxes take the differences' place
+        if (face) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) vb[faceAt + c] = Fv[c];
+        }
+    }
+    if (face) {
+        double Fx[5];
+        if (FAST && NS == 6) {
+            artra::weno5_flux<S>(mdl, [=](int m, int c) { return p[m * rowStep + c]; }, Fx);
+        } else {
+            double w[NS][5];
+#pragma unroll
+            for (int m = 0; m < NS; ++m)
+#pragma unroll
+                for (int c = 0; c < 5; ++c) w[m][c] = p[m * rowStep + c];
+            ConvFlux<S, NS, FAST>(mdl, w, Fx);
+        }
+#pragma unroll
+        for (int c = 0; c < 5; ++c) fb[faceAt + c] = Fx[c];
+    }
+    __syncthreads();
+    if (sa.step && step == 0.0) return;              // a march that has reached its end time: nothing moves
+    const double r = sa.step ? step * sa.dds : sa.r, br = sa.b * r;
+    // solution operator (fluid_dynamics.c:243-274), component by component
+    const double *f = fb + ((S == 0) ? h.row * F * 5 : 0) + shareAt;
+    const double *v = vb + ((S == 0) ? h.row * F * 5 : 0) + shareAt;
+    const double *u = vb + TileSpare(P, ts.seg, VISC) + ((S == 0) ? h.row * ts.seg * 5 : 0) + shareAt;
+    const double *un = st + ((S == 0) ? (h.row * rows + halo) * 5 : halo * 5 * P) + shareAt;
+    const unsigned at = (unsigned)(h.row * rowStride * 5 + h.col) * 8u;
+    double *base = sa.Utm + (size_t)t.first * 5;
+    const long pass = (S == 0) ? h.perPass : (long)h.perPass * rowStride * 5;
+#pragma unroll
+    for (int k = 0; k < kTileOut; ++k) {
+        if (k * h.perPass >= endOut || !((fluid >> k) & 1u)) continue;
+        const int e = k * shareStep;
+        const double FL = f[e], FR = f[e + rowStep];
+        double phi;
+        if (FAST) phi = VISC ? (FL - FR) + (v[e + rowStep] - v[e]) : FL - FR;
+        else phi = VISC ? ((FL - FR) + v[e + rowStep]) - v[e] : ((FL - FR) + 0.0) - 0.0;
+        double *um = (double *)((char *)(base + k * pass) + at);
+        if (sa.accumulate) {
+            *um = FAST ? fma(br, phi, u[e]) : u[e] + br * phi;
+            continue;
+        }
+        const double Un = un[e], Uo = sa.toIsTn ? Un : u[e];
+        *um = FAST ? fma(sa.a, Uo, sa.b * fma(r, phi, Un)) : sa.a * Uo + sa.b * (Un + r * phi);
     }
 }
 
@@ -621,16 +752,6 @@ struct LineHybrid {
                                     // classified, [2] faces of overflowed lines
     float smoothVariation;          // faces varying less than this (relative) skip the network; 0: none
 };
-
-// Blocks are dealt to the XCDs round robin; this bijection gives each XCD a
-// contiguous run of lines, so lines that share cache lines (adjacent x for
-// y and z lines) meet in the same L2.
-__device__ __forceinline__ long XcdLine(long b, long nb)
-{
-    const long q = nb / 8, rem = nb % 8;
-    const long x = b % 8, i = b / 8;
-    return (x < rem) ? x * (q + 1) + i : rem * (q + 1) + (x - rem) * q + i;
-}
 
 // A value every lane of the wavefront holds alike, moved to scalar
 // registers (it then holds no vector registers through the stage loop).
@@ -2261,7 +2382,7 @@ struct ArtraDevice {
     std::vector<GeoBodyDev> geoBodies;
     std::vector<int> layerStart;
     FluxModel mdl{};
-    int segment = 32;
+    int segment = 0;                // longest segment of the y and z stage sweeps (0: as the tile allows)
     int exact = 0;                  // 1: reference operation order (bit-faithful), 0: fast arithmetic
     int partialFill = 1;            // axis-only fills between the stages of inviscid split sweeps
     int hybrid = 0;                 // learned-indicator routing of WENO5 faces
@@ -2345,29 +2466,71 @@ int Harvest(ArtraDevice *dev)
     return 0;
 }
 
+// Tile of a stage sweep along s: of the shapes that fit a block of at most
+// kTileThreads, the one whose blocks cost least in all.  A wavefront's faces
+// cost about 650 issue slots, an element copied in or out 8 or 20 per
+// wavefront (instruction counts of the kernel), a cache line moved about 6;
+// idle lanes of a partly filled wavefront, the halo of a short segment and
+// the broken cache lines of a narrow tile show in these counts.
+SweepTile TileOf(const Grid &g, int s, int halo, bool visc, int longest)
+{
+    SweepTile best{};
+    double bestCost = 0.0;
+    const int line = (s == 0) ? 1 : 0, third = (s == 2) ? 1 : 2;
+    const int es = g.hi[s] - g.lo[s], across = g.hi[line] - g.lo[line], others = g.hi[third] - g.lo[third];
+    const int extra = visc ? 2 : 1;                  // threads per line beyond its nodes
+    for (int P = 1; P <= across && P <= kTileThreads / 2; ++P) {
+        int seg = std::min(es, kTileThreads / P - extra);
+        if (seg < 1) break;
+        if (s > 0 && longest > 0) seg = std::min(seg, longest);
+        const int nseg = (es + seg - 1) / seg;
+        seg = (es + nseg - 1) / nseg;
+        const int rows = seg + 2 * halo;
+        // x: enough threads per line for its faces and for kTileIn elements each
+        const int perLine = (s == 0) ? std::max(seg + extra, (5 * rows + kTileIn - 1) / kTileIn) : seg + extra;
+        const int faceWaves = (P * perLine + 63) / 64;
+        if (TileDoubles(P, seg, rows, visc) * sizeof(double) > 48 * 1024) continue;
+        for (int waves = faceWaves; 64 * waves <= kTileThreads; ++waves) {
+            // y and z: rows of 5 P doubles per pass of the block
+            if (s == 0 && waves > faceWaves) break;
+            const int perPass = (s == 0) ? perLine : 64 * waves / (5 * P);
+            if (perPass < 1) continue;
+            const int in = (((s == 0) ? 5 * rows : rows) + perPass - 1) / perPass;
+            const int out = (((s == 0) ? 5 * seg : seg) + perPass - 1) / perPass;
+            if (in > kTileIn || out > kTileOut) continue;
+            const double cacheLines = (s == 0) ? P * ((rows + 2 * seg) * 40.0 / 128.0 + 2.25)
+                                               : (rows + 2 * seg) * (P * 40.0 / 128.0 + 0.75);
+            const double tiles = (double)((across + P - 1) / P) * others * nseg;
+            const double cost = tiles * (650.0 * faceWaves + waves * (8.0 * in + 20.0 * out) + 6.0 * cacheLines);
+            if (best.P && cost >= bestCost) continue;
+            best.P = P;
+            best.seg = seg;
+            best.nseg = nseg;
+            best.groups = (across + P - 1) / P;
+            best.others = others;
+            best.rows = rows;
+            best.perPass = perPass;
+            best.threads = 64 * waves;
+            best.tiles = best.groups * others * nseg;
+            bestCost = cost;
+        }
+    }
+    return best;
+}
+
 template <int NS, bool VISC, bool FAST>
 void LaunchSweep(ArtraDevice *dev, int s, const StageArgs &sa)
 {
     const Grid &g = dev->g;
-    if (s == 0) {
-        const long faces = (long)(g.hi[0] - g.lo[0] + 1) * (g.hi[1] - g.lo[1]) * (g.hi[2] - g.lo[2]);
-        const long blocks = (faces - 1 + (kXBlock - 2)) / (kXBlock - 1);
-        if (blocks <= 0) return;
-        hipLaunchKernelGGL((sweep_x<NS, VISC, FAST>), dim3((unsigned)blocks), dim3(kXBlock), 0, dev->stream, g, sa,
-                           dev->mdl);
-        return;
+    for (int q = 0; q < 3; ++q) {
+        if (g.hi[q] <= g.lo[q]) return;
     }
-    const int T2 = (s == 1) ? 2 : 1;
-    const int ex = g.hi[0] - g.lo[0], et = g.hi[T2] - g.lo[T2], es = g.hi[s] - g.lo[s];
-    const int seg = dev->segment;
-    if (ex <= 0 || et <= 0 || es <= 0) return;
-    dim3 grid((ex + kMarchX - 1) / kMarchX, (et + kMarchT - 1) / kMarchT, (es + seg - 1) / seg);
-    dim3 block(kMarchX, kMarchT);
-    if (s == 1) {
-        hipLaunchKernelGGL((sweep_march<1, NS, VISC, FAST>), grid, block, 0, dev->stream, g, sa, dev->mdl, seg);
-    } else {
-        hipLaunchKernelGGL((sweep_march<2, NS, VISC, FAST>), grid, block, 0, dev->stream, g, sa, dev->mdl, seg);
-    }
+    const SweepTile ts = TileOf(g, s, NS / 2, VISC, dev->segment);
+    const size_t lds = TileDoubles(ts.P, ts.seg, ts.rows, VISC) * sizeof(double);
+    const dim3 grid((unsigned)ts.tiles), block(ts.threads);
+    if (s == 0) hipLaunchKernelGGL((sweep_tile<0, NS, VISC, FAST>), grid, block, lds, dev->stream, g, sa, dev->mdl, ts);
+    else if (s == 1) hipLaunchKernelGGL((sweep_tile<1, NS, VISC, FAST>), grid, block, lds, dev->stream, g, sa, dev->mdl, ts);
+    else hipLaunchKernelGGL((sweep_tile<2, NS, VISC, FAST>), grid, block, lds, dev->stream, g, sa, dev->mdl, ts);
 }
 
 int Sweep(ArtraDevice *dev, double dt, double a, double b, int to, int tn, int tm, int p)
@@ -2378,7 +2541,7 @@ int Sweep(ArtraDevice *dev, double dt, double a, double b, int to, int tn, int t
         sa.Utn = Level(dev, tn);
         sa.Uto = Level(dev, to);
         sa.Utm = Level(dev, tm);
-        sa.fluid = dev->fluid;
+        sa.fluid = dev->allFluid ? nullptr : dev->fluid;
         sa.a = a;
         sa.b = b;
         sa.r = dt * dev->par.dd[s];

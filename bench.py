@@ -159,11 +159,11 @@ def reference_rate(name, steps):
 # (case, timed steps, CPU sample case, CPU sample steps, dominant kernel family,
 # measured HBM bytes per cell-stage of its sweeps, profiles/sweep_tgv128_cylinder.md)
 SIDE_WORKLOADS = (
-    ("tgv128", 20, "tgv64", 4, "sweep_x/sweep_march with the viscous flux (stage-by-stage sweeps)", 176.6),
-    ("cylinder", 40, "cyl64", 100, "sweep_x/sweep_march with the immersed-boundary fill (stage-by-stage sweeps)",
+    ("tgv128", 20, "tgv64", 4, "sweep_tile with the viscous flux (stage-by-stage sweeps)", 176.6),
+    ("cylinder", 40, "cyl64", 100, "sweep_tile with the immersed-boundary fill (stage-by-stage sweeps)",
      126.0),
     ("cylinder_moving", 40, "cyl64_moving", 10,
-     "sweep_x/sweep_march with the immersed-boundary fill; solid half-steps (surface force, kinematics, motion, "
+     "sweep_tile with the immersed-boundary fill; solid half-steps (surface force, kinematics, motion, "
      "reclassification, ghost tables) between the fluid steps", 126.0),
 )
 
@@ -397,7 +397,7 @@ def main():
         per = TRAFFIC_B_PER_CELL_STAGE if not args.unfused else UNFUSED_TRAFFIC_B_PER_CELL_STAGE
         traffic = round(per * cells * stages_per_launch)
     kernel = ("rk_line (fused directional sweep, all RK stages of one line in LDS)" if fused_axes
-              else "sweep_x/sweep_march (stage-by-stage directional sweeps)")
+              else "sweep_tile (stage-by-stage directional sweeps)")
     out = {
         "metric": METRIC,
         "value": round(value, 3),
