@@ -338,7 +338,10 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(FA
             fluid |= (unsigned)sa.fluid[t.first + node] << k;
         }
     }
+    // a march that has reached its end time (or an output instant): nothing
+    // moves; looked at with the loads above in flight
     const double step = sa.step ? *sa.step : 0.0;
+    if (sa.step && step == 0.0) return;
     // this thread's line and face: face q is the left face of the line's q-th node
     const int slot = (S == 0) ? h.row : tid % P, q = (S == 0) ? h.col : tid / P;
     const int lineStep = (S == 0) ? rows * 5 : 5, rowStep = (S == 0) ? 5 : 5 * P;
@@ -421,7 +424,6 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(FA
         for (int c = 0; c < 5; ++c) fb[faceAt + c] = Fx[c];
     }
     __syncthreads();
-    if (sa.step && step == 0.0) return;              // a march that has reached its end time: nothing moves
     const double r = sa.step ? step * sa.dds : sa.r, br = sa.b * r;
     // solution operator (fluid_dynamics.c:243-274), component by component
     const double *f = fb + ((S == 0) ? h.row * F * 5 : 0) + shareAt;
