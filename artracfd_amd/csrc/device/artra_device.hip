@@ -561,7 +561,7 @@ __device__ __forceinline__ void Primitive(double gamma, double gasR, const doubl
     Uo[5] = Uo[4] / (Uo[0] * gasR);
 }
 
-__device__ __forceinline__ void Conservative(double gamma, const double Uo[6], double U[5])
+__host__ __device__ __forceinline__ void Conservative(double gamma, const double Uo[6], double U[5])
 {
     U[0] = Uo[0];
     U[1] = Uo[0] * Uo[1];
@@ -674,51 +674,20 @@ __global__ __launch_bounds__(256) void bc_gather(GatherArgs ga, const int *__res
 }
 
 // ------------------------------------------------- fused directional sweep
-// All Runge-Kutta stages of one split directional operator for one grid line
-// per block: the line (ghosts included) is read from HBM once, the stages run
-// on it in LDS - face fluxes into an LDS face buffer, node updates in place,
-// the ghost ends refilled between stages by per-line copy rules - and the
-// interior is written back once.  Valid where a stage along S reads nothing
-// but its own line: inviscid, split, no immersed body, and a between-stage
-// fill that only copies along the line (derived from the resolved gather).
-// With HYB the learned indicator routes each face: smooth faces take the
-// linear fifth-order upwind flux, troubled ones the full WENO5 flux.
+// All Runge-Kutta stages of a split directional operator with the line held
+// in LDS: its interior is read from HBM once, the stages run on it - face
+// fluxes into an LDS face buffer, node updates in place, the ghost ends
+// refilled between stages by per-line rules - and the interior is written
+// back once.  Valid where a stage along S reads nothing but its own line:
+// inviscid, split, no immersed body, and a fill along S that copies along
+// the line, prescribes a state or mirrors about a wall.
+//
+// The ghosts an operator starts from follow from the line's own interior by
+// the same rules, so the operators of a step need no boundary fill between
+// them; only the first operator of a call takes its ghosts from memory, as
+// the caller left them.  Two operators along the same axis in a row (x, x in
+// the middle of the three-dimensional step) run in one launch.
 constexpr int kLineRules = 12;
-constexpr int kRefillPerNode = 4;   // ghosts a line's node refills between stages, at most
-
-// The ghosts a node feeds, kRefillPerNode line positions packed two to a
-// register (16 bits each, 0xffff for none; line positions are below 2^16).
-struct Feeds {
-    unsigned w[kRefillPerNode / 2];
-};
-
-// (every slot is written through a compile-time index, so the set stays in
-// registers)
-__device__ __forceinline__ Feeds FeedsOf(const int *rules, int nrules, int node)
-{
-    static_assert(kRefillPerNode == 4, "two packed registers");
-    unsigned w0 = 0xffffffffu, w1 = 0xffffffffu;
-    int nf = 0;
-    for (int e = 0; e < nrules; ++e) {
-        if (rules[kLineRules + e] != node || nf >= kRefillPerNode) continue;
-        const unsigned pos = (unsigned)rules[e];
-        const unsigned sh = 16u * (nf & 1);
-        const unsigned mask = ~(0xffffu << sh);
-        if (nf < 2) w0 = (w0 & mask) | (pos << sh);
-        else w1 = (w1 & mask) | (pos << sh);
-        ++nf;
-    }
-    Feeds f;
-    f.w[0] = w0;
-    f.w[1] = w1;
-    return f;
-}
-
-__device__ __forceinline__ int FeedAt(const Feeds &f, int e)
-{
-    const unsigned v = (f.w[e >> 1] >> (16u * (e & 1))) & 0xffffu;
-    return (v == 0xffffu) ? -1 : (int)v;
-}
 // The face tallies of the indicator are spread over slots on separate
 // 128-byte lines (block b adds into slot b mod kCountSlots): one counter
 // pair taking an atomic from every block serialises tens of thousands of
@@ -735,15 +704,22 @@ struct LineArgs {
     int n1;                         // interior extent of the first transverse axis
     int lo1, lo2;                   // interior starts of the transverse axes
     int stride, stride1, stride2;   // node-index strides along S and the transverse axes
+    int lines;                      // n1 times the interior extent of the second transverse axis
     int stages;
+    int operators;                  // operators along this axis in a row (one or two)
     double a[3], b[3];
     double r;                       // dt / ds
     const double *dt;               // when set, the step's dt on the device (r = *dt * dd)
     double dd;                      // 1 / ds
-    double gamma;
+    double gamma, gasR;
+    int memoryGhosts;               // the ghosts the line starts from: 0 by the rules, 1 as memory holds them, 2 as
+    const double *steps;            // memory holds them in the first step of a march (*steps == 1)
     int nrules;
     int rdst[kLineRules], rsrc[kLineRules];   // src >= 0: line position, src < 0: constant state -1 - src
-    double given[2][6];             // primitive states of constant (inflow) rules
+    int reach;                      // the copied nodes are among the first or last `reach` of the interior
+    double state[2][5];             // conservative states of constant (inflow) rules
+    int wall[2];                    // low and high end: 0, or the wall type (2 slip, 3 no-slip) that mirrors there
+    double wallT[2];                // its temperature (negative: adiabatic)
 };
 
 struct LineHybrid {
@@ -765,40 +741,18 @@ __device__ __forceinline__ double Uniform(double x)
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// LDS of one line: the states [n][5] and a work area holding the face
-// fluxes [F][5], the operator's initial state of the interior nodes
-// [F - 1][5] and the fill rules with their constant states (kRuleBytes);
-// with the indicator (hyb) also the FP32 density and pressure of every node
-// [2][n] (the network's features).
+// LDS of one line: the states [n][5], the face fluxes [F][5] and the
+// operator's initial state of the interior nodes [F - 1][5]; with the
+// indicator (hyb) also the FP32 density and pressure of every node [2][n]
+// (the network's features).
 __host__ __device__ __forceinline__ size_t LineStateBytes(int n)
 {
     return ((size_t)5 * n * sizeof(double) + 15) / 16 * 16;
 }
 
-// The fill rules in LDS: destinations and sources [2][kLineRules] (ints),
-// then the conservative state of every constant-state rule [kLineRules][5].
-constexpr size_t kRuleBytes = (size_t)2 * kLineRules * sizeof(int) + (size_t)kLineRules * 5 * sizeof(double);
-
-// The rules and the constant states of one line's fill into LDS (threads tt
-// of T); the caller's barrier publishes them.
-__device__ __forceinline__ void LoadRules(const LineArgs &la, int *rules, int tt, int T)
-{
-    double *cst = (double *)(rules + 2 * kLineRules);
-    for (int e = tt; e < la.nrules; e += T) {
-        rules[e] = la.rdst[e];
-        rules[kLineRules + e] = la.rsrc[e];
-        if (la.rsrc[e] < 0) {
-            double v[5];
-            Conservative(la.gamma, la.given[-1 - la.rsrc[e]], v);
-#pragma unroll
-            for (int c = 0; c < 5; ++c) cst[e * 5 + c] = v[c];
-        }
-    }
-}
-
 __host__ __device__ __forceinline__ size_t LineWorkPlainBytes(int F)
 {
-    return ((size_t)(5 * F + 5 * (F - 1)) * sizeof(double) + kRuleBytes + 15) / 16 * 16;
+    return ((size_t)(5 * F + 5 * (F - 1)) * sizeof(double) + 15) / 16 * 16;
 }
 
 __host__ __device__ __forceinline__ size_t LineWorkBytes(int n, int F, bool hyb)
@@ -816,6 +770,113 @@ __device__ __forceinline__ long LineBase(const LineArgs &la, long line)
 {
     const int a1 = (int)(line % la.n1), a2 = (int)(line / la.n1);
     return (long)(la.lo1 + a1) * la.stride1 + (long)(la.lo2 + a2) * la.stride2;
+}
+
+// The ghosts beyond a wall at the low (side 0) or high end of a line held in
+// LDS, from its interior (boundary_treatment.c:84-185, in the order of the
+// ordered fill: the boundary node r = 0 from its neighbour, then r = 1, 2
+// mirrored about the stored boundary node).  Threads tt of T, one ghost
+// each; a barrier before and after.
+template <int S>
+__device__ __forceinline__ void WallGhosts(const LineArgs &la, int half, double *st, int tt, int T)
+{
+    for (int w = tt; w < 2 * half; w += T) {
+        const int side = w / half, r = w - side * half;
+        const int type = la.wall[side];
+        if (!type) continue;
+        const int inward = side ? -1 : 1, wall = side ? la.hi : la.lo - 1;
+        const double *h = st + (wall + inward) * 5;
+        const double Uh[5] = {h[0], h[1], h[2], h[3], h[4]};
+        double Uoh[6], Uo[6], out[5];
+        Primitive(la.gamma, la.gasR, Uh, Uoh);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) Uo[1 + c] = (type == 2 && c != S) ? Uoh[1 + c] : 0.0;
+        Uo[4] = Uoh[4];
+        Uo[5] = (0.0 > la.wallT[side]) ? Uoh[5] : la.wallT[side];
+        Uo[0] = Uo[4] / (Uo[5] * la.gasR);
+        Conservative(la.gamma, Uo, out);
+        if (r > 0) {
+            double UoO[6], UoI[6];
+            Primitive(la.gamma, la.gasR, out, UoO);
+            const double *q = st + (wall + r * inward) * 5;
+            const double UI[5] = {q[0], q[1], q[2], q[3], q[4]};
+            Primitive(la.gamma, la.gasR, UI, UoI);
+#pragma unroll
+            for (int c = 1; c < 4; ++c) Uo[c] = UoO[c] + UoO[c] - UoI[c];
+            Uo[4] = UoI[4];
+            Uo[5] = UoI[5];
+            Uo[0] = Uo[4] / (Uo[5] * la.gasR);
+            Conservative(la.gamma, Uo, out);
+        }
+        double *g = st + (wall - r * inward) * 5;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) g[c] = out[c];
+    }
+}
+
+// Whether a line starts from the ghosts memory holds.
+__device__ __forceinline__ bool FromMemory(const LineArgs &la)
+{
+    return la.memoryGhosts == 1 || (la.memoryGhosts == 2 && *la.steps == 1.0);
+}
+
+// The ghost node g of 2 half (low end, then high end) of a line: its
+// position, and in U its state by the line's rules or as memory holds it;
+// false where neither gives one (a wall's, which WallGhosts makes).
+__device__ __forceinline__ bool GhostNode(const LineArgs &la, long base, int g, int half, bool memory, int &pos, double U[5])
+{
+    pos = (g < half) ? la.lo - half + g : la.hi + g - half;
+    int src = memory ? pos : -3;
+#pragma unroll
+    for (int e = 0; e < kLineRules; ++e) {
+        if (!memory && e < la.nrules && la.rdst[e] == pos) src = la.rsrc[e];
+    }
+    if (src >= 0) {
+        LoadNode(la.U, base + (long)src * la.stride, U);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 5; ++c) U[c] = (src == -1) ? la.state[0][c] : la.state[1][c];
+    }
+    return src > -3;
+}
+
+// A line into LDS by its T threads, one interior node each with K = 1 and
+// two with K = 2: whole nodes (three loads from one address), every load
+// asked for before the first is waited for.
+template <int K>
+__device__ __forceinline__ void LoadLine(const LineArgs &la, long base, int tt, int T, int half, bool memory, double *st)
+{
+    const int I = la.hi - la.lo;
+    double v[K][5];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (tt + k * T < I) LoadNode(la.U, base + (long)(la.lo + tt + k * T) * la.stride, v[k]);
+    }
+    for (int g = tt; g < 2 * half; g += T) {
+        int pos;
+        double w[5];
+        if (!GhostNode(la, base, g, half, memory, pos, w)) continue;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) st[pos * 5 + c] = w[c];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (tt + k * T >= I) continue;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) st[(la.lo + tt + k * T) * 5 + c] = v[k][c];
+    }
+}
+
+// The ghosts that copy interior node i, refilled with its new state v.
+__device__ __forceinline__ void Refill(const LineArgs &la, int i, const double v[5], double *st)
+{
+    if (i - la.lo >= la.reach && la.hi - 1 - i >= la.reach) return;
+#pragma unroll
+    for (int e = 0; e < kLineRules; ++e) {
+        if (e >= la.nrules || la.rsrc[e] != i) continue;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) st[la.rdst[e] * 5 + c] = v[c];
+    }
 }
 
 // The linear fifth-order face flux of the learned hybrid at the face between
@@ -889,13 +950,118 @@ __device__ __forceinline__ bool ClassifyFace(const LineHybrid &hy, const float *
     return troubled;
 }
 
-// All stages of the directional operator on one line, run by the T threads
-// tt = 0..T-1 (a multiple of the wavefront).  Every thread of the block must
-// call it with the same loop trip counts (same n, lo, hi, stages), because
-// the stages are separated by block barriers.  With write = false the line
-// is computed but not stored (padding slots of a batched block).
+// The operators on one line, run by T threads tt = 0 .. T - 1: thread tt
+// holds the nodes lo + tt + T k and the faces to their left (T covers the F
+// faces with K per thread).  Every thread of the block must call it with the
+// same stage counts, because the stages are separated by block barriers;
+// lines that are not `active` (past the last of the block) only keep the
+// barriers.
+template <int S, int NS, bool FAST, int K>
+__device__ __forceinline__ void PlainLine(const LineArgs &la, const FluxModel &mdl, long line, int tt, int T, char *mem,
+                                          bool active, bool memory)
+{
+    constexpr int SL = (NS == 6) ? 2 : 1;           // stencil nodes left of the face's left node
+    const int n = la.n, F = la.hi - la.lo + 1;
+    double *st = (double *)mem;                     // [n][5]
+    double *fb = (double *)(mem + LineStateBytes(n));   // [F][5]
+    double *u0 = fb + 5 * F;                        // [F - 1][5]
+    const long base = LineBase(la, line);
+    const bool walls = la.wall[0] || la.wall[1];
+    const double r = Uniform(la.dt ? *la.dt * la.dd : la.r);
+    if (active) LoadLine<K>(la, base, tt, T, SL + 1, memory, st);
+    if (la.dt && *la.dt == 0.0) return;             // past the march's end: the same for the whole block
+    __syncthreads();
+    for (int todo = la.stages * la.operators, s = 0;; --todo) {
+        if (walls && !memory) {
+            if (active) WallGhosts<S>(la, SL + 1, st, tt, T);
+            __syncthreads();
+        }
+        memory = false;
+        double FL[5];
+#pragma nounroll
+        for (int k = 0; k < K; ++k) {
+            const int q = tt + T * k;               // face between nodes lo - 1 + q and lo + q
+            if (!active || q >= F) continue;
+            double Fx[5];
+            if (FAST && NS == 6) {
+                artra::weno_flux_line<S>(mdl, st, la.lo - 1 + q, Fx);
+            } else {
+                double w[NS][5];
+#pragma unroll
+                for (int j = 0; j < NS; ++j)
+#pragma unroll
+                    for (int c = 0; c < 5; ++c) w[j][c] = st[(la.lo - 1 + q - SL + j) * 5 + c];
+                ConvFlux<S, NS, FAST>(mdl, w, Fx);
+            }
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                fb[q * 5 + c] = Fx[c];
+                FL[c] = Fx[c];
+            }
+        }
+        __syncthreads();
+        // node updates (fluid_dynamics.c:243-274); each thread reads and
+        // writes only its own nodes and, before another stage, refills the
+        // ghosts they feed (the line's fill)
+        const double a = la.a[s], b = la.b[s];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int q = tt + T * k, i = la.lo + q;
+            if (!active || i >= la.hi) continue;
+            double v[5];
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                const double L = (K == 1) ? FL[c] : fb[q * 5 + c], R = fb[(q + 1) * 5 + c];
+                const double phi = FAST ? L - R : ((L - R) + 0.0) - 0.0;
+                const double Un = st[i * 5 + c];
+                double Uo = Un;
+                if (s == 0) u0[q * 5 + c] = Un;     // an operator begins from this state
+                else Uo = u0[q * 5 + c];
+                v[c] = FAST ? fma(a, Uo, b * fma(r, phi, Un)) : a * Uo + b * (Un + r * phi);
+            }
+            if (todo == 1) {
+                StoreNode(la.U, LineBase(la, line) + (long)i * la.stride, v);
+                continue;
+            }
+#pragma unroll
+            for (int c = 0; c < 5; ++c) st[i * 5 + c] = v[c];
+            Refill(la, i, v, st);
+        }
+        if (todo == 1) return;
+        __syncthreads();
+        s = (s + 1 == la.stages) ? 0 : s + 1;
+    }
+}
+
+// LoadLine with the network's features: the FP32 density and pressure of
+// every node, formed from the registers the node passes through.
+template <int K>
+__device__ __forceinline__ void LoadRoutedLine(const LineArgs &la, long base, int tt, int T, bool memory, double gamma,
+                                               double *st, float *nodeRP)
+{
+    const int I = la.hi - la.lo;
+    double v[K + 1][5];
+    int pos = -1;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (tt + k * T < I) LoadNode(la.U, base + (long)(la.lo + tt + k * T) * la.stride, v[k]);
+    }
+    // (T is a whole wavefront or more: a thread for every ghost)
+    if (tt < 6 && !GhostNode(la, base, tt, 3, memory, pos, v[K])) pos = -1;
+#pragma unroll
+    for (int k = 0; k <= K; ++k) {
+        const int p = (k == K) ? pos : (tt + k * T < I) ? la.lo + tt + k * T : -1;
+        if (p < 0) continue;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) st[p * 5 + c] = v[k][c];
+        artra::node_rho_p(gamma, v[k], nodeRP[p], nodeRP[la.n + p]);
+    }
+}
+
+// The learned hybrid's operator on one line, run by the T threads
+// tt = 0..T-1 (a multiple of the wavefront).
 //
-// With HYB, the indicator classifies the faces once per operator (at its
+// The indicator classifies the faces once per operator (at its
 // first RK stage, before the stage loop: the solution moves less than a
 // cell within one operator, and the network's fragments are then dead in
 // the flux passes) and the routing is per wavefront: a wavefront whose 64
@@ -904,174 +1070,134 @@ __device__ __forceinline__ bool ClassifyFace(const LineHybrid &hy, const float *
 // wavefront takes, never both branches), so a line crossed by a shock pays
 // full WENO5 only on the wavefronts around the shock and no wavefront pays
 // more than the plain kernel.
-template <int S, int NS, bool FAST, bool HYB, int K>
-__device__ __forceinline__ void LineBody(const LineArgs &la, const FluxModel &mdl, const LineHybrid &hy, long line,
-                                         int tt, int T, char *mem, bool write, unsigned long long *tally,
-                                         const float *bias, const artra::MlpWave &frags)
+template <int S, int K>
+__device__ __forceinline__ void RoutedLine(const LineArgs &la, const FluxModel &mdl, const LineHybrid &hy, long line,
+                                           int tt, int T, char *mem, bool write, bool memory, unsigned long long *tally,
+                                           const float *bias, const artra::MlpWave &frags)
 {
-    constexpr int SL = (NS == 6) ? 2 : 1;           // stencil nodes left of the face's left node
     const int n = la.n, F = la.hi - la.lo + 1;
     double *st = (double *)mem;                     // [n][5]
     char *work = mem + LineStateBytes(n);
     double *fb = (double *)work;                    // [F][5]
     double *u0 = fb + 5 * F;                        // [F - 1][5]
-    int *rules = (int *)(u0 + 5 * (F - 1));         // [2][kLineRules]: destinations, sources
-    const double *cst = (const double *)(rules + 2 * kLineRules);   // [kLineRules][5] constant states
-    float *nodeRP = (float *)(work + LineWorkPlainBytes(F));   // [2][n] (HYB)
+    float *nodeRP = (float *)(work + LineWorkPlainBytes(F));   // [2][n]
     const long base = LineBase(la, line);
-    for (int p = tt; p < n; p += T) {
-        double v[5];
-        LoadNode(la.U, base + (long)p * la.stride, v);
-#pragma unroll
-        for (int c = 0; c < 5; ++c) st[p * 5 + c] = v[c];
-        if (p >= la.lo && p < la.hi) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) u0[(p - la.lo) * 5 + c] = v[c];
-        }
-        if (HYB) artra::node_rho_p(mdl.gamma, v, nodeRP[p], nodeRP[n + p]);
-    }
-    // the line's fill rules into LDS: read per lane from the argument
-    // block once here, where the field loads hide the latency
-    LoadRules(la, rules, tt, T);
-    // the nodes this thread updates (every interior node of a fused line is
-    // a fluid node: the fused path runs only where all are)
-    bool own[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) own[k] = la.lo + tt + T * k < la.hi;
+    LoadRoutedLine<K>(la, base, tt, T, memory, mdl.gamma, st, nodeRP);
     __syncthreads();
-    // between-stage refill duties: the ghosts this thread's nodes feed, and
-    // (threads tt < nrules) one constant-state rule
-    Feeds feed[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) feed[k] = FeedsOf(rules, la.nrules, la.lo + tt + T * k);
-    const int constRule = (tt < la.nrules && rules[kLineRules + tt] < 0) ? tt : -1;
     const int M = (F + T - 1) / T;
     const double r = Uniform(la.dt ? *la.dt * la.dd : la.r);
     if (la.dt && *la.dt == 0.0) write = false;      // a batched case past its end time
-    // With HYB the faces are dealt to the wavefronts rotated by a whole
+    // The faces are dealt to the wavefronts rotated by a whole
     // wavefront per line: the troubled faces of a shock crossing every line
     // at the same place then fall on a different wavefront (and SIMD) from
     // line to line instead of loading one SIMD with all of them.
     const int QT = M * T;
-    const int rot = HYB ? (int)(line % (QT / 64)) * 64 : 0;
+    const int rot = (int)(line % (QT / 64)) * 64;
     // bit m: this wavefront's faces of pass m take the full WENO5 flux
-    unsigned wenoPasses = HYB ? 0u : ~0u;
-    if (HYB) {
-        // classification (every thread runs the same trip count)
-        unsigned long long wenoFaces = 0, faces = 0, flagged = 0;
-        for (int m = 0; m < M; ++m) {
-            const int q = (tt + T * m + rot) % QT;
-            const bool valid = q < F;
-            const int f = la.lo - 1 + (valid ? q : F - 1);
-            const bool troubled = ClassifyFace(hy, nodeRP, n, f, valid, frags, bias);
-            const unsigned long long here = __popcll(__ballot(valid));
-            const unsigned long long marked = __popcll(__ballot(troubled));
-            if (marked) {
-                wenoPasses |= 1u << m;
-                wenoFaces += here;
-                flagged += marked;
-            }
-            faces += here;
+    unsigned wenoPasses = 0u;
+    // classification (every thread runs the same trip count)
+    unsigned long long wenoFaces = 0, faces = 0, flagged = 0;
+    for (int m = 0; m < M; ++m) {
+        const int q = (tt + T * m + rot) % QT;
+        const bool valid = q < F;
+        const int f = la.lo - 1 + (valid ? q : F - 1);
+        const bool troubled = ClassifyFace(hy, nodeRP, n, f, valid, frags, bias);
+        const unsigned long long here = __popcll(__ballot(valid));
+        const unsigned long long marked = __popcll(__ballot(troubled));
+        if (marked) {
+            wenoPasses |= 1u << m;
+            wenoFaces += here;
+            flagged += marked;
         }
-        wenoPasses = __builtin_amdgcn_readfirstlane(wenoPasses);
-        // tallies per wavefront: faces on the linear flux, faces classified,
-        // faces on the full WENO5 flux, faces the indicator flagged troubled
-        if (__lane_id() == 0 && write) {
-            atomicAdd(&tally[0], faces - wenoFaces);
-            atomicAdd(&tally[1], faces);
-            if (wenoFaces) {
-                atomicAdd(&tally[2], wenoFaces);
-                atomicAdd(&tally[3], flagged);
-            }
+        faces += here;
+    }
+    wenoPasses = __builtin_amdgcn_readfirstlane(wenoPasses);
+    // tallies per wavefront: faces on the linear flux, faces classified,
+    // faces on the full WENO5 flux, faces the indicator flagged troubled
+    if (__lane_id() == 0 && write) {
+        atomicAdd(&tally[0], faces - wenoFaces);
+        atomicAdd(&tally[1], faces);
+        if (wenoFaces) {
+            atomicAdd(&tally[2], wenoFaces);
+            atomicAdd(&tally[3], flagged);
         }
     }
     for (int s = 0; s < la.stages; ++s) {
         for (int m = 0; m < M; ++m) {
-            const int q = HYB ? (tt + T * m + rot) % QT : tt + T * m;
-            if (q >= F) {
-                if (HYB) continue;
-                break;
-            }
+            const int q = (tt + T * m + rot) % QT;
+            if (q >= F) continue;
             const int f = la.lo - 1 + q;   // face between f and f + 1
             double Fx[5];
-            if (HYB && !((wenoPasses >> m) & 1u)) {
-                LinearFaceFlux<S>(mdl, st, f, Fx);
-            } else if (FAST && NS == 6) {
-                artra::weno_flux_line<S>(mdl, st, f, Fx);
-            } else {
-                double w[NS][5];
-#pragma unroll
-                for (int j = 0; j < NS; ++j)
-#pragma unroll
-                    for (int c = 0; c < 5; ++c) w[j][c] = st[(f - SL + j) * 5 + c];
-                ConvFlux<S, NS, FAST>(mdl, w, Fx);
-            }
+            if (!((wenoPasses >> m) & 1u)) LinearFaceFlux<S>(mdl, st, f, Fx);
+            else artra::weno_flux_line<S>(mdl, st, f, Fx);
 #pragma unroll
             for (int c = 0; c < 5; ++c) fb[q * 5 + c] = Fx[c];
         }
         __syncthreads();
-        // node updates (fluid_dynamics.c:243-274); each thread reads and
-        // writes only its own nodes and, before another stage, refills the
-        // ghosts they feed (the line's between-stage fill)
         const double a = la.a[s], b = la.b[s];
-        const bool refill = s + 1 < la.stages;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            if (!own[k]) continue;
-            const int i = la.lo + tt + T * k;
-            const int q = i - la.lo;
+            const int q = tt + T * k, i = la.lo + q;
+            if (i >= la.hi) continue;
             double v[5];
 #pragma unroll
             for (int c = 0; c < 5; ++c) {
                 const double FL = fb[q * 5 + c], FR = fb[(q + 1) * 5 + c];
-                const double phi = FAST ? FL - FR : ((FL - FR) + 0.0) - 0.0;
+                const double phi = FL - FR;
                 const double Un = st[i * 5 + c];
-                const double Uo = (s == 0) ? Un : u0[q * 5 + c];
-                v[c] = FAST ? fma(a, Uo, b * fma(r, phi, Un)) : a * Uo + b * (Un + r * phi);
-                st[i * 5 + c] = v[c];
+                double Uo = Un;
+                if (s == 0) u0[q * 5 + c] = Un;
+                else Uo = u0[q * 5 + c];
+                v[c] = fma(a, Uo, b * fma(r, phi, Un));
+            }
+            if (s + 1 == la.stages) {
+                if (write) StoreNode(la.U, LineBase(la, line) + (long)i * la.stride, v);
+                continue;
             }
 #pragma unroll
-            for (int e = 0; e < kRefillPerNode; ++e) {
-                const int d = FeedAt(feed[k], e);
-                if (!refill || d < 0) continue;
-#pragma unroll
-                for (int c = 0; c < 5; ++c) st[d * 5 + c] = v[c];
-            }
+            for (int c = 0; c < 5; ++c) st[i * 5 + c] = v[c];
+            Refill(la, i, v, st);
         }
-        if (refill && constRule >= 0) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) st[rules[constRule] * 5 + c] = cst[constRule * 5 + c];
-        }
-        __syncthreads();
-    }
-    if (!write) return;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        if (!own[k]) continue;
-        const int i = la.lo + tt + T * k;
-#pragma unroll
-        for (int c = 0; c < 5; ++c) NodeAt(la.U, base + (long)i * la.stride)[c] = st[i * 5 + c];
+        if (s + 1 < la.stages) __syncthreads();
     }
 }
 
-// One line per block.
-template <int S, int NS, bool FAST, bool HYB, int K>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HYB ? 3 : FAST ? 3 : 2))) void rk_line(LineArgs la, FluxModel mdl,
+// Plain lines, as many per block as its threads hold: `perLine` threads a
+// line, one per face up to 256 faces (K = 1), two faces each beyond (K = 2).
+// Bound by FP64 vector issue (534 of 675 vector instructions a stage and
+// node; 75-80 % of the issue cycles are taken at three wavefronts per SIMD).
+// At 256^3 an operator takes 1.17 ms along y, 1.14 along z, the two along x
+// in one launch 2.12 (one line to a block of whole wavefronts, component by
+// component loads, a launch per operator: 1.28, 1.25, 1.23 each with the same
+// flux arithmetic); on the 5-node lines of a 256 x 4 x 4 tube 10 us against 20.
+template <int S, int NS, bool FAST, int K>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? 3 : 2))) void rk_line(LineArgs la, FluxModel mdl,
+                                                                                                 int perLine, int perBlock)
+{
+    extern __shared__ double lds[];
+    const int slot = threadIdx.x / perLine, tt = threadIdx.x - slot * perLine;
+    const long line = XcdLine(blockIdx.x, gridDim.x) * perBlock + slot;
+    const bool active = slot < perBlock && line < la.lines;
+    char *mem = (char *)lds + (size_t)slot * LineLdsBytes(la.n, la.hi - la.lo + 1, false);
+    PlainLine<S, NS, FAST, K>(la, mdl, active ? line : 0, tt, perLine, mem, active, FromMemory(la));
+}
+
+// One routed line per block.
+template <int S, int K>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rk_routed(LineArgs la, FluxModel mdl,
                                                                                         LineHybrid hy)
 {
     if (la.dt && *la.dt == 0.0) return;             // a device-stepped march past its end time
     extern __shared__ double lds[];
     __shared__ unsigned long long tally[kTallies];
-    __shared__ float bias[HYB ? 3 * artra::kHidden : 1];
+    __shared__ float bias[3 * artra::kHidden];
     artra::MlpWave frags;
-    if (HYB) {
-        for (int e = threadIdx.x; e < 3 * artra::kHidden; e += blockDim.x) bias[e] = hy.bias[e];
-        if (threadIdx.x < kTallies) tally[threadIdx.x] = 0ull;
-        artra::mlp_wave_fragments(hy.W1, hy.W2, frags);
-    }
+    for (int e = threadIdx.x; e < 3 * artra::kHidden; e += blockDim.x) bias[e] = hy.bias[e];
+    if (threadIdx.x < kTallies) tally[threadIdx.x] = 0ull;
+    artra::mlp_wave_fragments(hy.W1, hy.W2, frags);
     const long line = XcdLine(blockIdx.x, gridDim.x);
-    LineBody<S, NS, FAST, HYB, K>(la, mdl, hy, line, threadIdx.x, blockDim.x, (char *)lds, true, tally, bias, frags);
-    if (HYB && threadIdx.x == 0) {
+    RoutedLine<S, K>(la, mdl, hy, line, threadIdx.x, blockDim.x, (char *)lds, true, FromMemory(la), tally, bias, frags);
+    if (threadIdx.x == 0) {
         unsigned long long *slot = hy.counts + (blockIdx.x % kCountSlots) * kCountStride;
         atomicAdd(slot, tally[0]);
         atomicAdd(slot + 1, tally[1]);
@@ -1082,13 +1208,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HYB ? 3 : F
 
 // The learned hybrid's lean pass: one line per block, T >= interior nodes
 // (one node and at most two faces per thread).  The line is loaded and its
-// faces classified exactly as LineBody classifies them (ClassifyFace); a
+// faces classified exactly as RoutedLine classifies them (ClassifyFace); a
 // line with any troubled face is not computed here but appended to defer[]
 // (rk_line_list runs it again with the full hybrid body), every other line
 // runs all RK stages with the linear fifth-order flux only (LinearFaceFlux):
 // no WENO5 code and no network fragments past the classification, so it
 // holds fewer registers and runs more lines per compute unit.  Its faces
-// are those LineBody computes for the same line, bit for bit.
+// are those RoutedLine computes for the same line, bit for bit.
 template <int S, bool MEAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 4))) void rk_lean(
     LineArgs la, FluxModel mdl, LineHybrid hy, int *defer, int *ndefer, unsigned long long *deferTotal)
@@ -1101,23 +1227,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 
     const int n = la.n, F = la.hi - la.lo + 1;
     double *st = lds;                                   // [n][5]
     double *fb = st + 5 * n;                            // [F][5]
-    int *rules = (int *)(fb + 5 * F);                   // [2][kLineRules], constant states
-    const double *cst = (const double *)(rules + 2 * kLineRules);
-    float *nodeRP = (float *)((char *)rules + kRuleBytes);   // [2][n]
+    float *nodeRP = (float *)(fb + 5 * F);              // [2][n]
     const long line = XcdLine(blockIdx.x, gridDim.x);
-    const int a1 = (int)(line % la.n1), a2 = (int)(line / la.n1);
-    const long base = (long)(la.lo1 + a1) * la.stride1 + (long)(la.lo2 + a2) * la.stride2;
+    const long base = LineBase(la, line);
     artra::MlpWave frags;
     artra::mlp_wave_fragments(hy.W1, hy.W2, frags);
     for (int e = tt; e < 3 * artra::kHidden; e += T) bias[e] = hy.bias[e];
-    for (int p = tt; p < n; p += T) {
-        double v[5];
-        LoadNode(la.U, base + (long)p * la.stride, v);
-#pragma unroll
-        for (int c = 0; c < 5; ++c) st[p * 5 + c] = v[c];
-        artra::node_rho_p(mdl.gamma, v, nodeRP[p], nodeRP[n + p]);
-    }
-    LoadRules(la, rules, tt, T);
+    LoadRoutedLine<1>(la, base, tt, T, FromMemory(la), mdl.gamma, st, nodeRP);
     const int i = la.lo + tt;                       // this thread's node
     const bool own = i < la.hi;
     if (tt == 0) troubledAny = 0;
@@ -1149,9 +1265,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 
 #pragma unroll
     for (int c = 0; c < 5; ++c) U0[c] = st[(own ? i : la.lo) * 5 + c];
     const double r = Uniform(la.dt ? *la.dt * la.dd : la.r);
-    // between-stage refill duties (as in LineBody)
-    const Feeds feed = FeedsOf(rules, la.nrules, i);
-    const int constRule = (tt < la.nrules && rules[kLineRules + tt] < 0) ? tt : -1;
     for (int s = 0; s < la.stages; ++s) {
         for (int m = 0; m < M; ++m) {
             const int q = tt + T * m;
@@ -1162,9 +1275,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 
             for (int c = 0; c < 5; ++c) fb[q * 5 + c] = Fx[c];
         }
         __syncthreads();
-        // node update (fluid_dynamics.c:243-274) and, before another
-        // stage, the refill of the ghosts this node feeds
-        const bool refill = s + 1 < la.stages;
+        // node update (fluid_dynamics.c:243-274) and the refill of the
+        // ghosts this node feeds
         if (own) {
             const double a = la.a[s], b = la.b[s];
             const int q = i - la.lo;
@@ -1175,33 +1287,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 
                 const double Un = st[i * 5 + c];
                 const double Uo = (s == 0) ? Un : U0[c];
                 v[c] = fma(a, Uo, b * fma(r, phi, Un));
-                st[i * 5 + c] = v[c];
             }
+            if (s + 1 == la.stages) {
+                StoreNode(la.U, LineBase(la, line) + (long)i * la.stride, v);
+            } else {
 #pragma unroll
-            for (int e = 0; e < kRefillPerNode; ++e) {
-                const int d = FeedAt(feed, e);
-                if (!refill || d < 0) continue;
-#pragma unroll
-                for (int c = 0; c < 5; ++c) st[d * 5 + c] = v[c];
+                for (int c = 0; c < 5; ++c) st[i * 5 + c] = v[c];
+                Refill(la, i, v, st);
             }
         }
-        if (refill && constRule >= 0) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) st[rules[constRule] * 5 + c] = cst[constRule * 5 + c];
-        }
-        __syncthreads();
-    }
-    if (own) {
-#pragma unroll
-        for (int c = 0; c < 5; ++c) NodeAt(la.U, base + (long)i * la.stride)[c] = st[i * 5 + c];
+        if (s + 1 < la.stages) __syncthreads();
     }
 }
 
-// LDS of rk_lean: states [n][5], face fluxes [F][5], fill rules and
-// constant states, FP32 density and pressure [2][n].
+// LDS of rk_lean: states [n][5], face fluxes [F][5], FP32 density and
+// pressure [2][n].
 __host__ __device__ __forceinline__ size_t LeanLdsBytes(int n, int F)
 {
-    return (size_t)(5 * n + 5 * F) * sizeof(double) + kRuleBytes + (size_t)2 * n * sizeof(float);
+    return (size_t)(5 * n + 5 * F) * sizeof(double) + (size_t)2 * n * sizeof(float);
 }
 
 // The full hybrid kernel over a list of lines (those rk_lean deferred):
@@ -1229,8 +1332,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
         asm volatile("" ::: "memory");
         artra::MlpWave frags;
         artra::mlp_wave_fragments(hy.W1, hy.W2, frags);
-        LineBody<S, 6, true, true, 1>(la, mdl, hy, list[w], threadIdx.x, blockDim.x, (char *)lds, true, tally, bias,
-                                      frags);
+        RoutedLine<S, 1>(la, mdl, hy, list[w], threadIdx.x, blockDim.x, (char *)lds, true, FromMemory(la), tally, bias,
+                         frags);
         __syncthreads();
     }
     if (threadIdx.x == 0) {
@@ -1243,9 +1346,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
 }
 
 // Many independent cases in one persistent launch: blocks of 256 threads
-// walk a tile list; a tile is P = 256 / T lines of one case, each run by T
-// threads (the tile shape picked per grid size).  Lines past the case's end
-// in its last tile are computed on a copy of its last line and not stored.
+// walk a tile list; a tile is 256 / T lines of one case, each run by T
+// threads.  Plain lines take a thread per face (K = 1; two faces each with
+// K = 2); with the indicator T is a multiple of the wavefront, the tile
+// shape picked per grid size, and lines past the case's end in its last tile
+// are computed on a copy of its last line and not stored.
 struct BatchTile {
     int c;                          // case
     int T;                          // threads per line
@@ -1254,36 +1359,52 @@ struct BatchTile {
     long first;                     // first line of the tile
 };
 
-template <int S, int NS, bool HYB>
+template <int S, int K>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rk_batch(const BatchTile *tiles,
                                                                                          int ntiles,
                                                                                          const LineArgs *args,
-                                                                                         FluxModel mdl, LineHybrid hy)
+                                                                                         FluxModel mdl, const double *first)
 {
     extern __shared__ double lds[];
-    __shared__ unsigned long long tally[kTallies];
-    __shared__ float bias[HYB ? 3 * artra::kHidden : 1];
-    if (HYB) {
-        for (int e = threadIdx.x; e < 3 * artra::kHidden; e += blockDim.x) bias[e] = hy.bias[e];
-        if (threadIdx.x < kTallies) tally[threadIdx.x] = 0ull;
+    const bool memory = first && *first == 1.0;     // the march's first operator: ghosts as memory holds them
+    for (long w = blockIdx.x; w < ntiles; w += gridDim.x) {
+        const BatchTile bt = tiles[w];
+        const LineArgs &la = args[bt.c];
+        const int slot = threadIdx.x / bt.T, tt = threadIdx.x - slot * bt.T;
+        const bool active = slot < bt.count;
+        char *mem = (char *)lds + (size_t)slot * LineLdsBytes(la.n, la.hi - la.lo + 1, false);
+        PlainLine<S, 6, true, K>(la, mdl, active ? bt.first + slot : 0, tt, bt.T, mem, active, memory);
+        __syncthreads();
     }
+}
+
+template <int S>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rk_batch_routed(
+    const BatchTile *tiles, int ntiles, const LineArgs *args, FluxModel mdl, LineHybrid hy, const double *first)
+{
+    extern __shared__ double lds[];
+    const bool memory = first && *first == 1.0;     // the march's first operator: ghosts as memory holds them
+    __shared__ unsigned long long tally[kTallies];
+    __shared__ float bias[3 * artra::kHidden];
+    for (int e = threadIdx.x; e < 3 * artra::kHidden; e += blockDim.x) bias[e] = hy.bias[e];
+    if (threadIdx.x < kTallies) tally[threadIdx.x] = 0ull;
     for (long w = blockIdx.x; w < ntiles; w += gridDim.x) {
         const BatchTile bt = tiles[w];
         const LineArgs &la = args[bt.c];
         // loaded per tile (L2 hits, issued ahead of the field loads) so that
         // they hold no registers past the tile's classification; an opaque
         // memory effect keeps the loads from being hoisted out of the loop
-        if (HYB) asm volatile("" ::: "memory");
+        asm volatile("" ::: "memory");
         artra::MlpWave frags;
-        if (HYB) artra::mlp_wave_fragments(hy.W1, hy.W2, frags);
+        artra::mlp_wave_fragments(hy.W1, hy.W2, frags);
         const int slot = threadIdx.x / bt.T, tt = threadIdx.x % bt.T;
         const bool write = slot < bt.count;
         const long line = bt.first + (write ? slot : bt.count - 1);
-        char *mem = (char *)lds + (size_t)slot * LineLdsBytes(la.n, la.hi - la.lo + 1, HYB);
-        LineBody<S, NS, true, HYB, 1>(la, mdl, hy, line, tt, bt.T, mem, write, tally, bias, frags);
+        char *mem = (char *)lds + (size_t)slot * LineLdsBytes(la.n, la.hi - la.lo + 1, true);
+        RoutedLine<S, 1>(la, mdl, hy, line, tt, bt.T, mem, write, memory, tally, bias, frags);
         __syncthreads();
     }
-    if (HYB && threadIdx.x == 0) {
+    if (threadIdx.x == 0) {
         unsigned long long *slot = hy.counts + (blockIdx.x % kCountSlots) * kCountStride;
         atomicAdd(slot, tally[0]);
         atomicAdd(slot + 1, tally[1]);
@@ -2209,9 +2330,10 @@ __device__ __forceinline__ double AdvanceClock(const double d[3], double cfl, co
 // Time step of every case of a batch; half[c] receives dt / 2, the step of
 // each Strang-split directional operator.
 __global__ void dt_batch(const BatchCase *cases, int C, const unsigned long long *vmax, double *clock, double *dt,
-                         double *half)
+                         double *half, double *stepNo)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c == 0) *stepNo = *stepNo + 1.0;            // read by the launches behind this one only
     if (c >= C) return;
     const BatchCase &bc = cases[c];
     const double h = AdvanceClock(bc.d, bc.cfl, vmax + 3 * c, clock + kClock * c);
@@ -2409,8 +2531,11 @@ struct ArtraDevice {
         int ok = 0;
         int count = 0;
         int dst[kLineRules], src[kLineRules];
-        double given[2][6];
+        double state[2][5];
+        int wall[2];
+        double wallT[2];
     } lines[3];
+    int deferFill = 0;              // the steps being enqueued leave their last fill to the end of the march
     // timing
     bool timing = false;
     double ms[ARTRA_T_COUNT] = {0.0, 0.0, 0.0, 0.0};
@@ -2703,12 +2828,45 @@ int TreatBoundary(ArtraDevice *dev, int level, int mode = 0)
     return 0;
 }
 
-// Launch shape of rk_line for axis p: threads, interior nodes per thread, LDS bytes.
+// Launch shape of the fused lines along axis p: threads and interior nodes
+// per thread of a line, lines and threads of a block, LDS bytes of a block.
 struct LineShape {
     int T = 0, K = 0;
+    int perBlock = 0, threads = 0;
     size_t lds = 0;
     long lines = 0;
 };
+
+// Threads of a plain line and lines of a block for lines of F faces and n
+// nodes: a thread per face (two faces each beyond 256), and of the numbers
+// of lines that fit 256 threads the one that keeps most lanes of the
+// resident wavefronts busy.  A line rounded up to whole wavefronts of its
+// own leaves half the lanes idle on 32-node and a third on 150-node lines;
+// packed, 95-98 % of them work.
+void PlainShape(int n, int F, LineShape &sh)
+{
+    sh.K = (F <= 256) ? 1 : 2;
+    sh.T = (F + sh.K - 1) / sh.K;
+    if (sh.T > 256) {
+        sh = LineShape{};
+        return;
+    }
+    double best = 0.0;
+    const size_t line = LineLdsBytes(n, F, false);
+    for (int P = 1; P * sh.T <= 256; ++P) {
+        if (P * line > 64 * 1024) break;
+        const int waves = (P * sh.T + 63) / 64;
+        const int blocks = std::min(12 / waves, (int)(160 * 1024 / (P * line)));     // resident, three wavefronts per SIMD
+        const double busy = (double)(P * F) / (64.0 * waves * sh.K) * (waves * blocks);
+        if (busy > 1.001 * best) {
+            best = busy;
+            sh.perBlock = P;
+            sh.threads = 64 * waves;
+            sh.lds = P * line;
+        }
+    }
+    if (!sh.perBlock) sh = LineShape{};
+}
 
 LineShape LineShapeOf(const ArtraDevice *dev, int p, bool hyb)
 {
@@ -2718,36 +2876,43 @@ LineShape LineShapeOf(const ArtraDevice *dev, int p, bool hyb)
     LineShape sh;
     const int interior = g.hi[p] - g.lo[p];
     if (interior <= 0) return sh;
-    sh.K = (interior <= 256) ? 1 : 2;
-    const int per = (interior + sh.K - 1) / sh.K;
-    sh.T = ((per + 63) / 64) * 64;
-    if (sh.T > 256) return LineShape{};
     const int F = interior + 1;
-    sh.lds = LineLdsBytes(ext[p], F, hyb);
+    if (hyb) {
+        // whole wavefronts of one line: the routing is per wavefront
+        sh.K = (interior <= 256) ? 1 : 2;
+        const int per = (interior + sh.K - 1) / sh.K;
+        sh.T = sh.threads = ((per + 63) / 64) * 64;
+        if (sh.T > 256) return LineShape{};
+        sh.perBlock = 1;
+        sh.lds = LineLdsBytes(ext[p], F, true);
+    } else {
+        PlainShape(ext[p], F, sh);
+        if (!sh.T) return sh;
+    }
     sh.lines = (long)(g.hi[t1] - g.lo[t1]) * (g.hi[t2] - g.lo[t2]);
     return sh;
 }
 
-// Whether one directional operator along p can run as one fused rk_line launch.
+// Whether one directional operator along p can run as one fused launch.
 bool LineEligible(const ArtraDevice *dev, int p, bool hyb)
 {
     if (!dev->fused || !dev->lines[p].ok || !dev->allFluid) return false;
     if (dev->layerStart.back() != 0) return false;               // immersed-boundary ghosts present
     if (dev->mdl.refMu > 0.0 || dev->par.multidim != 0) return false;
-    if (!dev->gatherResolved || !dev->useGather || !dev->partialFill) return false;
+    if (!dev->useGather || !dev->partialFill) return false;
+    if (hyb && !dev->gatherResolved) return false;               // walls are not routed
     const LineShape sh = LineShapeOf(dev, p, hyb);
     return sh.T > 0 && sh.lines > 0 && sh.lds <= 64 * 1024;
 }
 
-template <int S, int NS, bool FAST, bool HYB>
-void LaunchLineK(ArtraDevice *dev, const LineShape &sh, const LineArgs &la, const LineHybrid &hy)
+template <int S, int NS, bool FAST>
+void LaunchPlain(ArtraDevice *dev, const LineShape &sh, const LineArgs &la)
 {
+    const dim3 grid((unsigned)((sh.lines + sh.perBlock - 1) / sh.perBlock)), block(sh.threads);
     if (sh.K == 1) {
-        hipLaunchKernelGGL((rk_line<S, NS, FAST, HYB, 1>), dim3((unsigned)sh.lines), dim3(sh.T), sh.lds, dev->stream,
-                           la, dev->mdl, hy);
+        hipLaunchKernelGGL((rk_line<S, NS, FAST, 1>), grid, block, sh.lds, dev->stream, la, dev->mdl, sh.T, sh.perBlock);
     } else {
-        hipLaunchKernelGGL((rk_line<S, NS, FAST, HYB, 2>), dim3((unsigned)sh.lines), dim3(sh.T), sh.lds, dev->stream,
-                           la, dev->mdl, hy);
+        hipLaunchKernelGGL((rk_line<S, NS, FAST, 2>), grid, block, sh.lds, dev->stream, la, dev->mdl, sh.T, sh.perBlock);
     }
 }
 
@@ -2756,12 +2921,18 @@ void LaunchLineS(ArtraDevice *dev, const LineShape &sh, const LineArgs &la, cons
 {
     const bool fast = !dev->exact;
     if (dev->par.sScheme == 1) {
-        if (dev->hybrid) LaunchLineK<S, 6, true, true>(dev, sh, la, hy);
-        else if (fast) LaunchLineK<S, 6, true, false>(dev, sh, la, hy);
-        else LaunchLineK<S, 6, false, false>(dev, sh, la, hy);
+        if (dev->hybrid) {
+            const dim3 grid((unsigned)sh.lines), block(sh.T);
+            if (sh.K == 1) hipLaunchKernelGGL((rk_routed<S, 1>), grid, block, sh.lds, dev->stream, la, dev->mdl, hy);
+            else hipLaunchKernelGGL((rk_routed<S, 2>), grid, block, sh.lds, dev->stream, la, dev->mdl, hy);
+        } else if (fast) {
+            LaunchPlain<S, 6, true>(dev, sh, la);
+        } else {
+            LaunchPlain<S, 6, false>(dev, sh, la);
+        }
     } else {
-        if (fast) LaunchLineK<S, 4, true, false>(dev, sh, la, hy);
-        else LaunchLineK<S, 4, false, false>(dev, sh, la, hy);
+        if (fast) LaunchPlain<S, 4, true>(dev, sh, la);
+        else LaunchPlain<S, 4, false>(dev, sh, la);
     }
 }
 
@@ -2783,12 +2954,11 @@ void LaunchLean(ArtraDevice *dev, const LineShape &sh, const LineArgs &la, const
                        dev->deferList, dev->deferCount);
 }
 
-// All RK stages of the directional operator along p in one launch; the
-// result lands in TO, whose full boundary fill follows.
-int LineSweep(ArtraDevice *dev, double dt, int p)
+// The arguments of the fused lines along axis p that do not change from
+// step to step.
+LineArgs LineArgsOf(ArtraDevice *dev, int p)
 {
     const Grid &g = dev->g;
-    const LineShape sh = LineShapeOf(dev, p, dev->hybrid != 0);
     const int ext[3] = {g.nx, g.ny, g.nz};
     const int stride[3] = {1, g.nx, g.nx * g.ny};
     const int t1 = (p == 0) ? 1 : 0, t2 = (p == 2) ? 1 : 2;
@@ -2798,11 +2968,13 @@ int LineSweep(ArtraDevice *dev, double dt, int p)
     la.lo = g.lo[p];
     la.hi = g.hi[p];
     la.n1 = g.hi[t1] - g.lo[t1];
+    la.lines = la.n1 * (g.hi[t2] - g.lo[t2]);
     la.lo1 = g.lo[t1];
     la.lo2 = g.lo[t2];
     la.stride = stride[p];
     la.stride1 = stride[t1];
     la.stride2 = stride[t2];
+    la.operators = 1;
     if (dev->par.tScheme == 0) {
         la.stages = 2;
         la.a[0] = 0.0; la.b[0] = 1.0;
@@ -2813,17 +2985,36 @@ int LineSweep(ArtraDevice *dev, double dt, int p)
         la.a[1] = 3.0 / 4.0; la.b[1] = 1.0 / 4.0;
         la.a[2] = 1.0 / 3.0; la.b[2] = 2.0 / 3.0;
     }
-    la.r = dt * dev->par.dd[p];
-    la.dt = dev->stepDev;
     la.dd = dev->par.dd[p];
     la.gamma = dev->par.gamma;
+    la.gasR = dev->par.gasR;
     const ArtraDevice::LineRules &R = dev->lines[p];
     la.nrules = R.count;
     for (int e = 0; e < R.count; ++e) {
         la.rdst[e] = R.dst[e];
         la.rsrc[e] = R.src[e];
+        if (R.src[e] >= 0) la.reach = std::max(la.reach, 1 + std::min(R.src[e] - la.lo, la.hi - 1 - R.src[e]));
     }
-    memcpy(la.given, R.given, sizeof la.given);
+    memcpy(la.state, R.state, sizeof la.state);
+    memcpy(la.wall, R.wall, sizeof la.wall);
+    memcpy(la.wallT, R.wallT, sizeof la.wallT);
+    return la;
+}
+
+// `operators` directional operators along p in one launch; the result lands
+// in the interior of TO.  `first`: the step's first operator, which starts
+// from the ghosts in memory where the step is the call's first.
+int LineSweep(ArtraDevice *dev, double dt, int p, int operators, bool first)
+{
+    const LineShape sh = LineShapeOf(dev, p, dev->hybrid != 0);
+    LineArgs la = LineArgsOf(dev, p);
+    la.operators = operators;
+    la.r = dt * dev->par.dd[p];
+    la.dt = dev->stepDev;
+    if (first) {
+        la.memoryGhosts = dev->stepDev ? 2 : 1;
+        la.steps = dev->stepDev ? dev->stepDev + 1 : nullptr;    // the march's step words: dt, dt / 2, step number
+    }
     LineHybrid hy{};
     if (dev->hybrid) {
         hy.W1 = dev->mlpW1;
@@ -2857,89 +3048,105 @@ int LineSweep(ArtraDevice *dev, double dt, int p)
     return End(dev, slot);
 }
 
-// Per-line copy rules of the between-stage fill along axis p, read off the
-// resolved gather of the faces normal to p: every interior line must see the
-// same rules (destination position along the line <- source position on the
-// same line, or a constant state), covering every ghost the stencil reads.
-void DeriveLineRules(ArtraDevice *dev, const ArtraBcGather *gt)
+// Per-line copy rules of the fill along axis p, read off the resolved gather
+// of the faces normal to p: every interior line must see the same rules
+// (destination position along the line <- source position on the same line,
+// or a constant state), covering every ghost the stencil reads.
+void DeriveLineRules(ArtraDevice *dev, int p, long entries, const int *dst, const int *srcs)
 {
     const Grid &g = dev->g;
     const int ext[3] = {g.nx, g.ny, g.nz};
     const int half = (dev->par.sScheme == 1) ? 3 : 2;
-    for (int p = 0; p < 3; ++p) {
-        ArtraDevice::LineRules &R = dev->lines[p];
-        R = ArtraDevice::LineRules{};
-        if (!gt->resolved || g.hi[p] - g.lo[p] <= 0) continue;
-        const int t1 = (p == 0) ? 1 : 0, t2 = (p == 2) ? 1 : 2;
-        const long n1 = g.hi[t1] - g.lo[t1], n2 = g.hi[t2] - g.lo[t2];
-        if (n1 <= 0 || n2 <= 0) continue;
-        std::vector<std::vector<std::pair<int, int>>> per((size_t)(n1 * n2));
-        int faces[2] = {-1, -1}, nfaces = 0;
-        bool ok = true;
-        for (long e = 0; e < gt->axis_count[p] && ok; ++e) {
-            const int d = gt->axis_dst[p][e], q = gt->axis_src[p][e];
-            const int c[3] = {d % g.nx, (d / g.nx) % g.ny, d / (g.nx * g.ny)};
-            if (c[t1] < g.lo[t1] || c[t1] >= g.hi[t1] || c[t2] < g.lo[t2] || c[t2] >= g.hi[t2]) continue;
-            int src;
-            if (q >= 0) {
-                const int cq[3] = {q % g.nx, (q / g.nx) % g.ny, q / (g.nx * g.ny)};
-                if (cq[t1] != c[t1] || cq[t2] != c[t2] || cq[p] < g.lo[p] || cq[p] >= g.hi[p]) ok = false;
-                src = cq[p];
-            } else {
-                const int face = -3 - q;
-                int slot = -1;
-                for (int k = 0; k < nfaces; ++k)
-                    if (faces[k] == face) slot = k;
-                if (slot < 0) {
-                    if (nfaces == 2) {
-                        ok = false;
-                        break;
-                    }
-                    slot = nfaces;
-                    faces[nfaces++] = face;
-                }
-                src = -1 - slot;
+    ArtraDevice::LineRules &R = dev->lines[p];
+    R = ArtraDevice::LineRules{};
+    if (g.hi[p] - g.lo[p] <= 0) return;
+    const int t1 = (p == 0) ? 1 : 0, t2 = (p == 2) ? 1 : 2;
+    const long n1 = g.hi[t1] - g.lo[t1], n2 = g.hi[t2] - g.lo[t2];
+    if (n1 <= 0 || n2 <= 0) return;
+    std::vector<std::vector<std::pair<int, int>>> per((size_t)(n1 * n2));
+    int faces[2] = {-1, -1}, nfaces = 0;
+    for (long e = 0; e < entries; ++e) {
+        const int d = dst[e], q = srcs[e];
+        const int c[3] = {d % g.nx, (d / g.nx) % g.ny, d / (g.nx * g.ny)};
+        if (c[t1] < g.lo[t1] || c[t1] >= g.hi[t1] || c[t2] < g.lo[t2] || c[t2] >= g.hi[t2]) continue;
+        int src;
+        if (q >= 0) {
+            const int cq[3] = {q % g.nx, (q / g.nx) % g.ny, q / (g.nx * g.ny)};
+            if (cq[t1] != c[t1] || cq[t2] != c[t2] || cq[p] < g.lo[p] || cq[p] >= g.hi[p]) return;
+            src = cq[p];
+        } else {
+            const int face = -3 - q;
+            int slot = -1;
+            for (int k = 0; k < nfaces; ++k)
+                if (faces[k] == face) slot = k;
+            if (slot < 0) {
+                if (nfaces == 2) return;
+                slot = nfaces;
+                faces[nfaces++] = face;
             }
-            per[(size_t)((c[t1] - g.lo[t1]) + n1 * (c[t2] - g.lo[t2]))].emplace_back(c[p], src);
+            src = -1 - slot;
         }
-        if (!ok) continue;
-        for (auto &v : per) std::sort(v.begin(), v.end());
-        const auto &ref = per[0];
-        for (const auto &v : per) {
-            if (v != ref) {
-                ok = false;
-                break;
-            }
-        }
-        if (!ok || (int)ref.size() > kLineRules) continue;
-        // copy rules read interior nodes, each feeding at most kRefillPerNode
-        // ghosts (the owner of a node refills them when it updates it)
-        for (const auto &r : ref) {
-            if (r.second < 0) continue;
-            int feeds = 0;
-            for (const auto &o : ref) feeds += (o.second == r.second);
-            ok = ok && r.second >= g.lo[p] && r.second < g.hi[p] && feeds <= kRefillPerNode;
-        }
-        if (!ok) continue;
-        for (int pos = g.lo[p] - half; pos < g.hi[p] + half; ++pos) {
-            if (pos >= g.lo[p] && pos < g.hi[p]) continue;
-            bool hit = pos >= 0 && pos < ext[p];
-            if (hit) {
-                hit = false;
-                for (const auto &r : ref) hit = hit || r.first == pos;
-            }
-            ok = ok && hit;
-        }
-        if (!ok) continue;
-        R.count = (int)ref.size();
-        for (int e = 0; e < R.count; ++e) {
-            R.dst[e] = ref[e].first;
-            R.src[e] = ref[e].second;
-        }
-        for (int k = 0; k < nfaces; ++k)
-            for (int v = 0; v < 6; ++v) R.given[k][v] = dev->par.varBC[faces[k]][v];
-        R.ok = 1;
+        per[(size_t)((c[t1] - g.lo[t1]) + n1 * (c[t2] - g.lo[t2]))].emplace_back(c[p], src);
     }
+    for (auto &v : per) std::sort(v.begin(), v.end());
+    const auto &ref = per[0];
+    for (const auto &v : per) {
+        if (v != ref) return;
+    }
+    if ((int)ref.size() > kLineRules) return;
+    // copy rules read interior nodes (the owner of a node refills the ghosts
+    // that copy it when it updates it)
+    for (const auto &rule : ref) {
+        if (rule.second >= 0 && (rule.second < g.lo[p] || rule.second >= g.hi[p])) return;
+    }
+    for (int pos = g.lo[p] - half; pos < g.hi[p] + half; ++pos) {
+        if (pos >= g.lo[p] && pos < g.hi[p]) continue;
+        bool hit = false;
+        for (const auto &rule : ref) hit = hit || rule.first == pos;
+        if (!hit || pos < 0 || pos >= ext[p]) return;
+    }
+    R.count = (int)ref.size();
+    for (int e = 0; e < R.count; ++e) {
+        R.dst[e] = ref[e].first;
+        R.src[e] = ref[e].second;
+    }
+    for (int k = 0; k < nfaces; ++k) Conservative(dev->par.gamma, dev->par.varBC[faces[k]], R.state[k]);
+    R.ok = 1;
+}
+
+// The rules of an axis with a wall at one end or both, from the face types:
+// an interior line's ghosts along its own axis come from its own axis's
+// faces alone (boundary_treatment.c:66-185): the wall's mirror states, the
+// prescribed state in every layer, or the boundary neighbour's in every layer.
+void DeriveWallRules(ArtraDevice *dev, int p)
+{
+    const Grid &g = dev->g;
+    const int ext[3] = {g.nx, g.ny, g.nz};
+    const int half = (dev->par.sScheme == 1) ? 3 : 2;
+    ArtraDevice::LineRules &R = dev->lines[p];
+    R = ArtraDevice::LineRules{};
+    const int lo = g.lo[p], hi = g.hi[p];
+    // the mirrored nodes of the farthest ghost are interior
+    if (hi - lo < half || lo - half < 0 || hi + half > ext[p]) return;
+    ArtraDevice::LineRules N{};
+    int states = 0;
+    for (int side = 0; side < 2; ++side) {
+        const int face = 1 + 2 * p + side, type = dev->par.typeBC[face];
+        if (type == 2 || type == 3) {
+            N.wall[side] = type;
+            N.wallT[side] = dev->par.varBC[face][5];
+            continue;
+        }
+        if (type != 0 && type != 1) return;
+        for (int q = 0; q < half; ++q) {
+            N.dst[N.count] = side ? hi + q : lo - 1 - q;
+            N.src[N.count++] = (type == 0) ? -1 - states : side ? hi - 1 : lo;
+        }
+        if (type == 0) Conservative(dev->par.gamma, dev->par.varBC[face], N.state[states++]);
+    }
+    if (!N.wall[0] && !N.wall[1]) return;
+    R = N;
+    R.ok = 1;
 }
 
 // Runge-Kutta stages of one directional operator (fluid_dynamics.c:121-148).
@@ -2954,16 +3161,59 @@ int Stages(ArtraDevice *dev, double dt, int p, int next)
     const int lazy = (p < 3 && !(dev->mdl.refMu > 0.0) && dev->partialFill);
     const int mid = lazy ? 1 + p : 0;
     const int last = lazy ? next : 0;
-    if (p < 3 && LineEligible(dev, p, dev->hybrid != 0)) return LineSweep(dev, dt, p) || TreatBoundary(dev, 0, last);
     if (dev->hybrid) return Fail("the learned indicator is on but axis %d cannot run fused", p);
     if (dev->par.tScheme == 0) {
         if (Sweep(dev, dt, 0.0, 1.0, 0, 0, 1, p) || TreatBoundary(dev, 1, mid)) return 1;
-        if (Sweep(dev, dt, 1.0 / 2.0, 1.0 / 2.0, 0, 1, 0, p) || TreatBoundary(dev, 0, last)) return 1;
-        return 0;
+        return Sweep(dev, dt, 1.0 / 2.0, 1.0 / 2.0, 0, 1, 0, p) || TreatBoundary(dev, 0, last);
     }
     if (Sweep(dev, dt, 0.0, 1.0, 0, 0, 1, p) || TreatBoundary(dev, 1, mid)) return 1;
     if (Sweep(dev, dt, 3.0 / 4.0, 1.0 / 4.0, 0, 1, 2, p) || TreatBoundary(dev, 2, mid)) return 1;
-    if (Sweep(dev, dt, 1.0 / 3.0, 2.0 / 3.0, 0, 2, 0, p) || TreatBoundary(dev, 0, last)) return 1;
+    return Sweep(dev, dt, 1.0 / 3.0, 2.0 / 3.0, 0, 2, 0, p) || TreatBoundary(dev, 0, last);
+}
+
+// The axes of the split step's operators in order, by collapse flag
+// (fluid_dynamics.c:60-110); -1 ends the list.
+constexpr int kSplitOrder[9][6] = {{2, 1, 0, 0, 1, 2},    {2, 1, 1, 2, -1, -1},   {2, 0, 0, 2, -1, -1},
+                                   {1, 0, 0, 1, -1, -1},  {-1, -1, -1, -1, -1, -1}, {2, 2, -1, -1, -1, -1},
+                                   {-1, -1, -1, -1, -1, -1}, {1, 1, -1, -1, -1, -1}, {0, 0, -1, -1, -1, -1}};
+
+// Whether every operator of a step runs fused: no fill is read within it.
+bool AllFused(const ArtraDevice *dev)
+{
+    const int c = dev->par.collapse;
+    if (dev->par.multidim == 1 || c < 0 || c > 8 || kSplitOrder[c][0] < 0) return false;
+    for (int q = 0; q < 6 && kSplitOrder[c][q] >= 0; ++q) {
+        if (!LineEligible(dev, kSplitOrder[c][q], dev->hybrid != 0)) return false;
+    }
+    return true;
+}
+
+// The split operators of one step.  A fused operator reads and writes line
+// interiors only; the fill after it covers what a stage-by-stage operator
+// behind it reads, or everything at the end of the step (unless the march
+// fills once behind its last step).
+int SplitStep(ArtraDevice *dev, double h)
+{
+    const int c = dev->par.collapse;
+    if (c < 0 || c > 8 || kSplitOrder[c][0] < 0) return Fail("unsupported collapse flag %d", c);
+    const int *order = kSplitOrder[c];
+    for (int q = 0; q < 6 && order[q] >= 0;) {
+        const int p = order[q];
+        if (!LineEligible(dev, p, dev->hybrid != 0)) {
+            const int more = (q + 1 < 6 && order[q + 1] >= 0);
+            if (Stages(dev, h, p, more ? 1 + order[q + 1] : 0)) return 1;
+            ++q;
+            continue;
+        }
+        const int run = (!dev->hybrid && q + 1 < 6 && order[q + 1] == p) ? 2 : 1;
+        if (LineSweep(dev, h, p, run, q == 0 && !dev->par.sState)) return 1;
+        q += run;
+        if (q < 6 && order[q] >= 0) {
+            if (!LineEligible(dev, order[q], dev->hybrid != 0) && TreatBoundary(dev, 0, 1 + order[q])) return 1;
+        } else if (!dev->deferFill && !dev->par.sState && TreatBoundary(dev, 0, 0)) {
+            return 1;
+        }
+    }
     return 0;
 }
 
@@ -2999,16 +3249,22 @@ int SourceStage(ArtraDevice *dev, double dt, double a, double b, int to, int tn,
 }
 
 // Runge-Kutta stages of the gravity source operator (fluid_dynamics.c:121-148
-// with s = PHI), each followed by the full boundary fill as in the reference.
-int SourceStages(ArtraDevice *dev, double dt)
+// with s = PHI), each followed by the full boundary fill as in the reference
+// unless nothing reads one: the operator itself reads interior nodes only,
+// and so do fused operators (`last`: the step ends here).
+int SourceStages(ArtraDevice *dev, double dt, bool last)
 {
+    const bool none = AllFused(dev);
+    const auto fill = [&](int level) { return none ? 0 : TreatBoundary(dev, level); };
     if (dev->par.tScheme == 0) {
-        if (SourceStage(dev, dt, 0.0, 1.0, 0, 0, 1) || TreatBoundary(dev, 1)) return 1;
-        return SourceStage(dev, dt, 1.0 / 2.0, 1.0 / 2.0, 0, 1, 0) || TreatBoundary(dev, 0);
+        if (SourceStage(dev, dt, 0.0, 1.0, 0, 0, 1) || fill(1)) return 1;
+        if (SourceStage(dev, dt, 1.0 / 2.0, 1.0 / 2.0, 0, 1, 0) || fill(0)) return 1;
+    } else {
+        if (SourceStage(dev, dt, 0.0, 1.0, 0, 0, 1) || fill(1)) return 1;
+        if (SourceStage(dev, dt, 3.0 / 4.0, 1.0 / 4.0, 0, 1, 2) || fill(2)) return 1;
+        if (SourceStage(dev, dt, 1.0 / 3.0, 2.0 / 3.0, 0, 2, 0) || fill(0)) return 1;
     }
-    if (SourceStage(dev, dt, 0.0, 1.0, 0, 0, 1) || TreatBoundary(dev, 1)) return 1;
-    if (SourceStage(dev, dt, 3.0 / 4.0, 1.0 / 4.0, 0, 1, 2) || TreatBoundary(dev, 2)) return 1;
-    return SourceStage(dev, dt, 1.0 / 3.0, 2.0 / 3.0, 0, 2, 0) || TreatBoundary(dev, 0);
+    return (none && last && !dev->deferFill) ? TreatBoundary(dev, 0, 0) : 0;
 }
 
 // The lean pass's per-axis policy, from the lines it deferred since the
@@ -3154,8 +3410,9 @@ int MarchSteps(ArtraDevice *dev, const MarchScratch &ms, double clock[kMarchCloc
     head[kMarchClock] = head[kMarchClock + 1] = head[kMarchClock + 2] = 0.0;
     HIP_TRY(hipMemcpyAsync(ms.clock, head, sizeof head, hipMemcpyHostToDevice, dev->stream));
     hipGraphExec_t graph = nullptr;
-    if (allowGraph && StepGraph(dev, ms, floor, cfl, &graph)) return 1;
-    int rc = 0;
+    // nothing reads the fill between fused steps: one behind the last
+    dev->deferFill = AllFused(dev);
+    int rc = (allowGraph && StepGraph(dev, ms, floor, cfl, &graph)) ? 1 : 0;
     if (graph) {
         for (int i = 0; i < steps && !rc; ++i) {
             if (hipGraphLaunch(graph, dev->stream) != hipSuccess) rc = Fail("step graph launch failed");
@@ -3165,6 +3422,8 @@ int MarchSteps(ArtraDevice *dev, const MarchScratch &ms, double clock[kMarchCloc
         for (int i = 0; i < steps && !rc; ++i) rc = EnqueueStep(dev, ms, floor, cfl);
         dev->stepDev = nullptr;
     }
+    if (!rc && dev->deferFill) rc = TreatBoundary(dev, 0, 0);
+    dev->deferFill = 0;
     if (rc) return 1;
     HIP_TRY(hipMemcpyAsync(clock, ms.clock, kMarchClock * sizeof(double), hipMemcpyDeviceToHost, dev->stream));
     HIP_TRY(hipMemcpyAsync(dts, ms.hist, (size_t)steps * sizeof(double), hipMemcpyDeviceToHost, dev->stream));
@@ -3350,8 +3609,11 @@ int artra_dev_set_gather(ArtraDevice *dev, const ArtraBcGather *gt)
         dev->gCount[m] = 0;
     }
     dev->gatherResolved = 0;
-    for (int s = 0; s < 3; ++s) dev->axisGather[s] = 0;
-    DeriveLineRules(dev, gt);
+    for (int s = 0; s < 3; ++s) {
+        dev->axisGather[s] = 0;
+        dev->lines[s] = ArtraDevice::LineRules{};
+        if (gt->resolved) DeriveLineRules(dev, s, gt->axis_count[s], gt->axis_dst[s], gt->axis_src[s]);
+    }
     if (!gt->resolved) return 0;
     for (int m = 0; m < 4; ++m) {
         const long n = (m == 0) ? gt->count : gt->axis_count[m - 1];
@@ -3379,7 +3641,11 @@ int artra_dev_set_axis_gather(ArtraDevice *dev, int s, const ArtraBcGather *gt)
     dev->gDst[m] = dev->gSrc[m] = nullptr;
     dev->gCount[m] = 0;
     dev->axisGather[s] = 0;
-    if (!gt->resolved) return 0;
+    if (!gt->resolved) {
+        DeriveWallRules(dev, s);
+        return 0;
+    }
+    DeriveLineRules(dev, s, gt->count, gt->dst, gt->src);
     const long n = gt->count;
     if (n > 0) {
         HIP_TRY(hipMalloc(&dev->gDst[m], n * sizeof(int)));
@@ -3634,21 +3900,13 @@ int artra_dev_evolve(ArtraDevice *dev, double dt)
 {
     const double h = 0.5 * dt;
     // gravity source half-steps around the fluid operators (fluid_dynamics.c:57-59, 112-114)
-    if (dev->par.sState && SourceStages(dev, h)) return 1;
+    if (dev->par.sState && SourceStages(dev, h, false)) return 1;
     if (dev->par.multidim == 1) {
         if (Stages(dev, h, 3, 0) || Stages(dev, h, 3, 0)) return 1;
-    } else {
-        static const int order[9][6] = {{2, 1, 0, 0, 1, 2},    {2, 1, 1, 2, -1, -1},   {2, 0, 0, 2, -1, -1},
-                                        {1, 0, 0, 1, -1, -1},  {-1, -1, -1, -1, -1, -1}, {2, 2, -1, -1, -1, -1},
-                                        {-1, -1, -1, -1, -1, -1}, {1, 1, -1, -1, -1, -1}, {0, 0, -1, -1, -1, -1}};
-        const int c = dev->par.collapse;
-        if (c < 0 || c > 8 || order[c][0] < 0) return Fail("unsupported collapse flag %d", c);
-        for (int q = 0; q < 6 && order[c][q] >= 0; ++q) {
-            const int more = (q + 1 < 6 && order[c][q + 1] >= 0);
-            if (Stages(dev, h, order[c][q], more ? 1 + order[c][q + 1] : 0)) return 1;
-        }
+    } else if (SplitStep(dev, h)) {
+        return 1;
     }
-    if (dev->par.sState && SourceStages(dev, h)) return 1;
+    if (dev->par.sState && SourceStages(dev, h, true)) return 1;
     if (dev->timing && dev->evUsed > 4096) return Harvest(dev);
     return 0;
 }
@@ -3718,9 +3976,7 @@ int artra_dev_set_indicator(ArtraDevice *dev, const float *params, float thresho
     }
     if (dev->par.sScheme != 1) return Fail("the learned indicator routes WENO5 faces; this case uses WENO3");
     if (dev->exact) return Fail("the learned indicator runs with the fast arithmetic only");
-    static const int order[9][6] = {{2, 1, 0, 0, 1, 2},    {2, 1, 1, 2, -1, -1},   {2, 0, 0, 2, -1, -1},
-                                    {1, 0, 0, 1, -1, -1},  {-1, -1, -1, -1, -1, -1}, {2, 2, -1, -1, -1, -1},
-                                    {-1, -1, -1, -1, -1, -1}, {1, 1, -1, -1, -1, -1}, {0, 0, -1, -1, -1, -1}};
+    const auto &order = kSplitOrder;
     const int c = dev->par.collapse;
     for (int q = 0; c >= 0 && c <= 8 && q < 6 && order[c][q] >= 0; ++q) {
         if (!LineEligible(dev, order[c][q], true)) {
@@ -3887,6 +4143,7 @@ struct ArtraBatch {
     LineArgs *dArgs[3] = {nullptr, nullptr, nullptr};
     BatchTile *dTiles[3] = {nullptr, nullptr, nullptr};
     int ntiles[3] = {0, 0, 0};
+    int K[3] = {1, 1, 1};                   // faces per thread of the plain lines
     size_t lds[3] = {0, 0, 0};
     BatchCase *dCases = nullptr;
     CflChunk *dChunks = nullptr;
@@ -3896,6 +4153,7 @@ struct ArtraBatch {
     long gCount = 0;
     unsigned long long *vmax = nullptr;
     double *clock = nullptr, *dt = nullptr, *half = nullptr;
+    double *stepNo = nullptr;               // the step's number within the march call
     int hybrid = 0;
     LineHybrid hy{};
     float *mlpBias = nullptr;
@@ -3924,14 +4182,28 @@ int BatchBuildTiles(ArtraBatch *b, int p)
 {
     std::vector<BatchTile> tiles;
     size_t lds = 0;
+    b->K[p] = 1;
+    for (const ArtraDevice *dev : b->cases) {
+        if (dev->g.hi[p] - dev->g.lo[p] + 1 > 256) b->K[p] = 2;
+    }
     for (int c = 0; c < b->C; ++c) {
         const ArtraDevice *dev = b->cases[c];
         const Grid &g = dev->g;
         const int t1 = (p == 0) ? 1 : 0, t2 = (p == 2) ? 1 : 2;
         const long lines = (long)(g.hi[t1] - g.lo[t1]) * (g.hi[t2] - g.lo[t2]);
-        const int T = b->threads[c], P = 256 / T;
         const int ext[3] = {g.nx, g.ny, g.nz};
-        lds = std::max(lds, (size_t)P * LineLdsBytes(ext[p], g.hi[p] - g.lo[p] + 1, true));
+        const int F = g.hi[p] - g.lo[p] + 1;
+        const size_t line = LineLdsBytes(ext[p], F, b->hybrid != 0);
+        int T, P;
+        if (b->hybrid) {
+            T = b->threads[c];
+            P = 256 / T;
+        } else {
+            // a thread per face, as many lines as leave LDS to three blocks per compute unit
+            T = (F + b->K[p] - 1) / b->K[p];
+            P = std::max(1, std::min(256 / T, (int)(52 * 1024 / line)));
+        }
+        lds = std::max(lds, (size_t)P * line);
         for (long first = 0; first < lines; first += P) {
             BatchTile bt{};
             bt.c = c;
@@ -3952,41 +4224,52 @@ int BatchBuildTiles(ArtraBatch *b, int p)
     return 0;
 }
 
-void BatchLaunchLines(ArtraBatch *b, int p, hipStream_t st)
+// The lines of every case along p; `first`: the step's first operator.
+template <int S>
+void BatchLaunchAxis(ArtraBatch *b, bool first, hipStream_t st)
 {
-    const unsigned grid = (unsigned)std::max(1, std::min(b->grid, b->ntiles[p]));
-    const bool hyb = b->hybrid != 0;
+    const dim3 grid((unsigned)std::max(1, std::min(b->grid, b->ntiles[S]))), block(256);
     const FluxModel mdl = b->cases[0]->mdl;
-#define ARTRA_BATCH_LAUNCH(S)                                                                                   \
-    do {                                                                                                        \
-        if (hyb)                                                                                                \
-            hipLaunchKernelGGL((rk_batch<S, 6, true>), dim3(grid), dim3(256), b->lds[p], st, b->dTiles[p],      \
-                               b->ntiles[p], b->dArgs[p], mdl, b->hy);                                          \
-        else                                                                                                    \
-            hipLaunchKernelGGL((rk_batch<S, 6, false>), dim3(grid), dim3(256), b->lds[p], st, b->dTiles[p],     \
-                               b->ntiles[p], b->dArgs[p], mdl, b->hy);                                          \
-    } while (0)
-    if (p == 0) ARTRA_BATCH_LAUNCH(0);
-    else if (p == 1) ARTRA_BATCH_LAUNCH(1);
-    else ARTRA_BATCH_LAUNCH(2);
-#undef ARTRA_BATCH_LAUNCH
+    const double *step = first ? b->stepNo : nullptr;
+    if (b->hybrid) {
+        hipLaunchKernelGGL((rk_batch_routed<S>), grid, block, b->lds[S], st, b->dTiles[S], b->ntiles[S], b->dArgs[S], mdl,
+                           b->hy, step);
+    } else if (b->K[S] == 1) {
+        hipLaunchKernelGGL((rk_batch<S, 1>), grid, block, b->lds[S], st, b->dTiles[S], b->ntiles[S], b->dArgs[S], mdl, step);
+    } else {
+        hipLaunchKernelGGL((rk_batch<S, 2>), grid, block, b->lds[S], st, b->dTiles[S], b->ntiles[S], b->dArgs[S], mdl, step);
+    }
+}
+
+void BatchLaunchLines(ArtraBatch *b, int p, bool first, hipStream_t st)
+{
+    if (p == 0) BatchLaunchAxis<0>(b, first, st);
+    else if (p == 1) BatchLaunchAxis<1>(b, first, st);
+    else BatchLaunchAxis<2>(b, first, st);
+}
+
+// Every case's boundary fill.
+void BatchFill(ArtraBatch *b, hipStream_t st)
+{
+    if (b->gCount <= 0) return;
+    hipLaunchKernelGGL(gather_batch, dim3((unsigned)((b->gCount + 255) / 256)), dim3(256), 0, st, b->dGather, b->gCase,
+                       b->gDst, b->gSrc, b->gCount);
 }
 
 // One time step of every case: speeds, dt, then Z Y X X Y Z, each operator a
-// persistent launch over all cases' lines followed by every case's fill.
+// persistent launch over all cases' lines (plain x operators: both in one).
+// The lines start from their own interiors, so the fill of every case
+// follows once, behind a march's last step.
 int BatchStep(ArtraBatch *b, hipStream_t st)
 {
     hipLaunchKernelGGL(fill_u64, dim3((3 * b->C + 255) / 256), dim3(256), 0, st, b->vmax, 3 * b->C, 0ull);
     hipLaunchKernelGGL(cfl_batch, dim3((unsigned)std::min(b->nchunks, 4 * b->cus)), dim3(256), 0, st, b->dChunks,
                        b->nchunks, b->dCases, b->vmax);
     hipLaunchKernelGGL(dt_batch, dim3((b->C + 63) / 64), dim3(64), 0, st, b->dCases, b->C, b->vmax, b->clock, b->dt,
-                       b->half);
+                       b->half, b->stepNo);
     for (int q = 0; q < 6; ++q) {
-        BatchLaunchLines(b, kBatchOrder[q], st);
-        if (b->gCount > 0) {
-            hipLaunchKernelGGL(gather_batch, dim3((unsigned)((b->gCount + 255) / 256)), dim3(256), 0, st, b->dGather,
-                               b->gCase, b->gDst, b->gSrc, b->gCount);
-        }
+        if (!b->hybrid && q > 0 && kBatchOrder[q] == kBatchOrder[q - 1]) continue;
+        BatchLaunchLines(b, kBatchOrder[q], q == 0, st);
     }
     HIP_TRY(hipGetLastError());
     return 0;
@@ -4054,43 +4337,8 @@ int artra_dev_batch_create(ArtraDevice *const *devs, int count, const double *cl
     for (int p = 0; p < 3; ++p) {
         std::vector<LineArgs> args(count);
         for (int c = 0; c < count; ++c) {
-            ArtraDevice *dv = devs[c];
-            const Grid &g = dv->g;
-            const int ext[3] = {g.nx, g.ny, g.nz};
-            const int stride[3] = {1, g.nx, g.nx * g.ny};
-            const int t1 = (p == 0) ? 1 : 0, t2 = (p == 2) ? 1 : 2;
-            LineArgs la{};
-            la.U = Level(dv, 0);
-            la.n = ext[p];
-            la.lo = g.lo[p];
-            la.hi = g.hi[p];
-            la.n1 = g.hi[t1] - g.lo[t1];
-            la.lo1 = g.lo[t1];
-            la.lo2 = g.lo[t2];
-            la.stride = stride[p];
-            la.stride1 = stride[t1];
-            la.stride2 = stride[t2];
-            if (dv->par.tScheme == 0) {
-                la.stages = 2;
-                la.a[0] = 0.0; la.b[0] = 1.0;
-                la.a[1] = 1.0 / 2.0; la.b[1] = 1.0 / 2.0;
-            } else {
-                la.stages = 3;
-                la.a[0] = 0.0; la.b[0] = 1.0;
-                la.a[1] = 3.0 / 4.0; la.b[1] = 1.0 / 4.0;
-                la.a[2] = 1.0 / 3.0; la.b[2] = 2.0 / 3.0;
-            }
-            la.r = 0.0;
-            la.dd = dv->par.dd[p];
-            la.gamma = dv->par.gamma;
-            const ArtraDevice::LineRules &R = dv->lines[p];
-            la.nrules = R.count;
-            for (int e = 0; e < R.count; ++e) {
-                la.rdst[e] = R.dst[e];
-                la.rsrc[e] = R.src[e];
-            }
-            memcpy(la.given, R.given, sizeof la.given);
-            args[c] = la;
+            args[c] = LineArgsOf(devs[c], p);
+            args[c].operators = (p == 0) ? 2 : 1;   // x, x in the middle of the step (routed lines take one each)
         }
         if (hipMalloc(&b->dArgs[p], count * sizeof(LineArgs)) != hipSuccess) return fail(Fail("out of device memory"));
         hostArgs[p] = args;
@@ -4098,7 +4346,8 @@ int artra_dev_batch_create(ArtraDevice *const *devs, int count, const double *cl
     if (hipMalloc(&b->vmax, 3 * count * sizeof(unsigned long long)) != hipSuccess ||
         hipMalloc(&b->clock, kClock * count * sizeof(double)) != hipSuccess ||
         hipMalloc(&b->dt, count * sizeof(double)) != hipSuccess ||
-        hipMalloc(&b->half, count * sizeof(double)) != hipSuccess) {
+        hipMalloc(&b->half, count * sizeof(double)) != hipSuccess ||
+        hipMalloc(&b->stepNo, sizeof(double)) != hipSuccess) {
         return fail(Fail("out of device memory"));
     }
     for (int p = 0; p < 3; ++p) {
@@ -4189,6 +4438,7 @@ void artra_dev_batch_destroy(ArtraBatch *b)
     hipFree(b->clock);
     hipFree(b->dt);
     hipFree(b->half);
+    hipFree(b->stepNo);
     hipFree(b->mlpBias);
     hipFree(b->mlpW1);
     hipFree(b->mlpW2);
@@ -4202,6 +4452,9 @@ int artra_dev_batch_set_indicator(ArtraBatch *b, const float *params, float thre
     BatchDropGraph(b);
     if (!params) {
         b->hybrid = 0;
+        for (int p = 0; p < 3; ++p) {
+            if (BatchBuildTiles(b, p)) return 1;    // the plain lines' tiles
+        }
         return 0;
     }
     if (!b->mlpBias) {
@@ -4231,6 +4484,9 @@ int artra_dev_batch_set_indicator(ArtraBatch *b, const float *params, float thre
     b->hy.counts = b->counts;
     b->hy.smoothVariation = 1.0e-3f;
     b->hybrid = 1;
+    for (int p = 0; p < 3; ++p) {
+        if (BatchBuildTiles(b, p)) return 1;        // the routed lines' tiles
+    }
     return 0;
 }
 
@@ -4262,6 +4518,7 @@ int artra_dev_batch_march(ArtraBatch *b, int steps, int use_graph, double *ms)
         b->graphHybrid = b->hybrid;
     }
     HIP_TRY(hipEventRecord(e0, b->stream));
+    hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, b->stream, (unsigned long long *)b->stepNo, 1, 0ull);
     for (int q = 0; q < steps && !rc; ++q) {
         if (use_graph) {
             const hipError_t e = hipGraphLaunch(b->exec, b->stream);
@@ -4270,6 +4527,7 @@ int artra_dev_batch_march(ArtraBatch *b, int steps, int use_graph, double *ms)
             rc = BatchStep(b, b->stream);
         }
     }
+    if (steps > 0 && !rc) BatchFill(b, b->stream);
     HIP_TRY(hipEventRecord(e1, b->stream));
     HIP_TRY(hipEventSynchronize(e1));
     float el = 0.0f;
@@ -4349,6 +4607,7 @@ int artra_dev_batch_tune(ArtraBatch *b, int reps, int *threads_out, int *grid_ou
         if (std::find(lengths.begin(), lengths.end(), L) == lengths.end()) lengths.push_back(L);
     }
     const std::vector<int> saved = b->threads;
+    if (!b->hybrid) lengths.clear();                // plain lines take a thread per face: no shape to choose
     for (int L : lengths) {
         double best = 1e300;
         int bestT = 0;
@@ -4364,7 +4623,7 @@ int artra_dev_batch_tune(ArtraBatch *b, int reps, int *threads_out, int *grid_ou
             if (!ok) continue;
             HIP_TRY(hipEventRecord(e0, b->stream));
             for (int r = 0; r < reps; ++r)
-                for (int p = 0; p < 3; ++p) BatchLaunchLines(b, p, b->stream);
+                for (int p = 0; p < 3; ++p) BatchLaunchLines(b, p, false, b->stream);
             HIP_TRY(hipEventRecord(e1, b->stream));
             HIP_TRY(hipEventSynchronize(e1));
             HIP_TRY(hipGetLastError());

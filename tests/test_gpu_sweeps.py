@@ -71,3 +71,81 @@ def test_stage_sweeps_at_the_edges_of_their_tiles(tmp_path, oracle_mod, m, bcs, 
         assert np.array_equal(U, ref)
     for c in (slice(0, 1), slice(1, 4), slice(4, 5)):
         assert np.abs(U[c] - ref[c]).max() <= 1e-13 * np.abs(ref[c]).max()
+
+
+MIXED = [mc.inflow(1.1, 0.4, 0.1, 0, 1.2), mc.noslip(), mc.slip(), mc.OUTFLOW, mc.noslip(0.0033), mc.slip(0.0036)]
+# (nodes, boundaries, the axes that run as lines): lines of one node to one
+# past the two-node threads' first, several lines to a block with a rest, a
+# wavefront's and a block's faces more or less by one
+LINES = [((2, 3, 4), OPEN, "xyz"), ((4, 3, 3), RING, "xyz"), ((64, 63, 5), OPEN, "xyz"), ((4, 128, 7), RING, "xyz"),
+         ((256, 3, 5), OPEN, "xyz"), ((257, 5, 3), OPEN, "xyz"), ((3, 512, 3), OPEN, "xyz"), ((3, 3, 513), OPEN, "xy"),
+         ((11, 37, 16), WALLS, "xyz"), ((4, 258, 4), WALLS, "xyz"), ((21, 4, 66), MIXED, "xyz"),
+         ((2, 7, 2), WALLS, "y")]                # (a wall needs as many interior nodes as ghosts)
+
+
+@pytest.mark.parametrize("m, bcs, expected", LINES)
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("numerical", [(1, 1, 0, 0, 0, 0, 1), (0, 0, 0, 1, 1, 0, 1)])
+def test_lines_at_the_edges_of_their_blocks(tmp_path, oracle_mod, m, bcs, expected, exact, numerical):
+    """Whole operators on lines in local memory against the oracle: bit for
+    bit in exact arithmetic, rounding level (1e-13 of the largest value of a
+    group after two steps) in the fast one, with any kind of boundary at the
+    lines' ends."""
+    print(m, exact, numerical, flush=True)
+    U, ref, axes = against_oracle(oracle_mod, write_case(tmp_path, m, bcs, numerical), 2, exact)
+    print("axes", axes)
+    assert "".join("xyz"[a] for a in axes) == expected
+    if exact:
+        assert np.array_equal(U, ref)
+    for c in (slice(0, 1), slice(1, 4), slice(4, 5)):
+        assert np.abs(U[c] - ref[c]).max() <= 1e-13 * np.abs(ref[c]).max()
+
+
+@pytest.mark.parametrize("bcs", [OPEN, RING, MIXED])
+def test_a_step_on_lines_starts_from_the_ghosts_of_its_input(tmp_path, bcs):
+    """One step on a caller's field with ghosts of its own: the first operator
+    reads them as they are, on lines as stage by stage."""
+    from artracfd_amd import Case, Solver
+    directory = write_case(tmp_path, (9, 70, 6), bcs)
+    out = []
+    for fused in (True, False):
+        case = Case(directory)
+        solver = Solver(case, exact=True, fused=fused)
+        U = solver.field()
+        solver.set_field(0, U * (1.0 + 1e-3 * np.cos(np.arange(U.size)).reshape(U.shape)))
+        print(bcs[0], fused, flush=True)
+        solver.evolve(1e-4)
+        out.append(case.interior(solver.field()).copy())
+        solver.close()
+        case.close()
+    assert np.array_equal(out[0], out[1])
+
+
+def test_batched_lines_at_the_edges_of_their_blocks(tmp_path):
+    """Lines of 2 to 257 faces packed into one batch give what
+    the cases give alone, bit for bit."""
+    from artracfd_amd import Case, Solver
+    from artracfd_amd.batch import Batch
+    dirs = []
+    for q, m in enumerate([(2, 3, 4), (63, 5, 3), (255, 4, 3), (4, 257, 6)]):
+        (tmp_path / str(q)).mkdir()
+        dirs.append(write_case(tmp_path / str(q), m, OPEN if q % 2 else RING))
+    alone = []
+    for d in dirs:
+        case = Case(d)
+        solver = Solver(case)
+        solver.march(3)
+        alone.append(case.interior(solver.field()).copy())
+        solver.close()
+        case.close()
+    cases = [Case(d) for d in dirs]
+    solvers = [Solver(c) for c in cases]
+    print("batch", flush=True)
+    b = Batch(solvers)
+    b.march(3)
+    for q, (c, s) in enumerate(zip(cases, solvers)):
+        assert np.array_equal(c.interior(s.field()), alone[q]), q
+    b.close()
+    for s, c in zip(solvers, cases):
+        s.close()
+        c.close()
