@@ -1513,12 +1513,6 @@ __global__ __launch_bounds__(256) void geo_sphere(Grid g, GeoSetup gs, GeoBox b,
     }
 }
 
-// Pass 2 for a triangulated body (computational_geometry.c:463-506): one
-// wavefront per node; the lanes measure the facets that bounding spheres
-// (of 32-facet blocks, then of facets) cannot rule out, the lanes'
-// (distance, facet) pairs reduce to the lexicographic minimum (the first
-// facet at the global minimum, as the serial scan), and the pseudo-normal
-// at that facet decides.
 // Bounding spheres for the closest-facet search below: per facet its
 // centroid and radius, per block of 32 consecutive facets (a half-wavefront
 // here) the mean of their centroids and the farthest reach of their spheres
@@ -1563,45 +1557,6 @@ __global__ __launch_bounds__(256) void geo_spheres(ArtraPolyView pv, double4 *sp
 // (distance, facet) pairs reduce to the lexicographic minimum (the first
 // facet at the global minimum, as the serial scan), and the pseudo-normal
 // at that facet decides.
-// A bounding sphere per facet (centroid, radius) for the closest-facet
-// search below.
-__global__ __launch_bounds__(256) void geo_spheres(ArtraPolyView pv, double4 *sph)
-{
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= pv.faceN) return;
-    const double *v0 = pv.v[pv.f[n][0]], *v1 = pv.v[pv.f[n][1]], *v2 = pv.v[pv.f[n][2]];
-    double c[3], r2 = 0.0;
-    for (int s = 0; s < 3; ++s) c[s] = (v0[s] + v1[s] + v2[s]) / 3.0;
-    const double *vs[3] = {v0, v1, v2};
-    for (int q = 0; q < 3; ++q) {
-        const double d[3] = {vs[q][0] - c[0], vs[q][1] - c[1], vs[q][2] - c[2]};
-        r2 = fmax(r2, d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-    }
-    sph[n] = make_double4(c[0], c[1], c[2], sqrt(r2));
-}
-
-// A bounding sphere per block of 32 consecutive facets: the mean of their
-// centroids and the farthest reach of their spheres from it.
-__global__ __launch_bounds__(64) void geo_blocks(int faceN, const double4 *sph, double4 *bsph)
-{
-    const int bk = blockIdx.x * blockDim.x + threadIdx.x;
-    const int first = bk * 32, last = min(first + 32, faceN);
-    if (first >= faceN) return;
-    double c[3] = {0.0, 0.0, 0.0};
-    for (int n = first; n < last; ++n) {
-        c[0] += sph[n].x;
-        c[1] += sph[n].y;
-        c[2] += sph[n].z;
-    }
-    for (int s = 0; s < 3; ++s) c[s] /= (double)(last - first);
-    double r = 0.0;
-    for (int n = first; n < last; ++n) {
-        const double d[3] = {sph[n].x - c[0], sph[n].y - c[1], sph[n].z - c[2]};
-        r = fmax(r, sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]) + sph[n].w);
-    }
-    bsph[bk] = make_double4(c[0], c[1], c[2], r);
-}
-
 __global__ __launch_bounds__(256) void geo_mesh(Grid g, GeoSetup gs, GeoBox b, int *did, int *fid, ArtraPolyView pv,
                                                 const double4 *sph, const double4 *bsph, int body)
 {
@@ -1732,7 +1687,12 @@ __global__ __launch_bounds__(256) void geo_interface(Grid g, GeoSetup gs, GeoBox
 // over fluid nodes for an image-point ghost, radius 1 around itself over
 // the previous layer's ghosts of the body otherwise, growing to 3).
 constexpr int kGhostSlot = 343;
-constexpr int kGeoCounters = 16;    // ghost-table build counters: taken, overflow, layer ends
+// Box nodes of a wavefront: its ghosts' searches follow one another, and
+// 32 nodes of a row hold a few ghosts of a layer.  (The layers of a
+// triangulated sphere in 96^3 nodes take 52, 41 and 41 us with 16, 32 and
+// 64; with one search for any radius 57, 50 and 53.)
+constexpr int kGhostNodes = 32;
+constexpr int kGeoCounters = 16;    // ghost-table build counters: overflow, each layer's entries
 
 struct GhostBuildArgs {
     Grid g;
@@ -1761,21 +1721,69 @@ __device__ __forceinline__ double GbDist2(const double a[3], const double b[3])
     return GcDot(d, d);
 }
 
-__global__ __launch_bounds__(256) void ib_build(GhostBuildArgs a, GeoBox b, int r, GhostBody body, const int *did,
-                                                const int *fid, const int *gst, GhostDev *ghosts, int *snode,
-                                                double *sw, int *counter, int *overflow)
+// The nodes of the (2 R + 1)^3 box around ns that a ghost's stencil takes,
+// with their weights for the centre cs, by the whole wavefront; returns their
+// number.  Candidate c of the box is (kh, jh, ih) in k-j-i order, and the
+// found nodes take consecutive entries in that order (a ballot prefix), as
+// the serial search appends them.  A constant radius: no more chunks than
+// the box has, and no division by a variable width.
+template <int R>
+__device__ __forceinline__ int SearchBox(const GhostBuildArgs &a, const int ns[3], const double cs[3], int want, int layer,
+                                         const int *did, const int *gst, int *snode, double *sw)
 {
-    // each wavefront covers 64 nodes of the box and searches their ghosts'
-    // stencils one at a time, the lanes scanning a search box together:
-    // candidate c of the (2 rr + 1)^3 box is (kh, jh, ih) in k-j-i order,
-    // and the found nodes take consecutive entries in that order (a ballot
-    // prefix), as the serial search appends them
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr int w = 2 * R + 1, cand = w * w * w, kChunks = (cand + 63) / 64;
     const Grid &g = a.g;
     const int lane = __lane_id();
+    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    // every chunk's flags are loaded before the first ballot, so the loads of
+    // a search overlap
+    int qv[kChunks];
+    bool hv[kChunks];
+#pragma unroll
+    for (int ch = 0; ch < kChunks; ++ch) {
+        const int cc = ch * 64 + lane;
+        const int x = ns[0] + cc % w - R, y = ns[1] + (cc / w) % w - R, z = ns[2] + cc / (w * w) - R;
+        qv[ch] = -1;
+        if (cc < cand && z >= g.lo[2] && z < g.hi[2] && y >= g.lo[1] && y < g.hi[1] && x >= g.lo[0] && x < g.hi[0])
+            qv[ch] = (int)(((long)z * g.ny + y) * g.nx + x);
+    }
+#pragma unroll
+    for (int ch = 0; ch < kChunks; ++ch) {
+        hv[ch] = false;
+        if (qv[ch] < 0) continue;
+        const int dq = did[qv[ch]], gq = gst[qv[ch]];
+        hv[ch] = (want == dq) && (layer == 0 || layer == gq);
+    }
+    int count = 0;
+#pragma unroll
+    for (int ch = 0; ch < kChunks; ++ch) {
+        const unsigned long long hits = __ballot(hv[ch]);
+        if (hv[ch]) {
+            const int cc = ch * 64 + lane;
+            const int x = ns[0] + cc % w - R, y = ns[1] + (cc / w) % w - R, z = ns[2] + cc / (w * w) - R;
+            double ph[3];
+            GeoPoint(a.gs, x, y, z, ph);
+            const int pos = count + __popcll(hits & below);
+            snode[pos] = qv[ch];
+            sw[pos] = GbInverse(a.tinyL, GbDist2(cs, ph));
+        }
+        count += __popcll(hits);
+    }
+    return count;
+}
+
+__global__ __launch_bounds__(256) void ib_build(GhostBuildArgs a, GeoBox b, int r, GhostBody body, const int *did,
+                                                const int *fid, const int *gst, GhostDev *ghosts, int *snode,
+                                                double *sw, int *counters)
+{
+    // each wavefront covers kGhostNodes nodes of the box and searches their
+    // ghosts' stencils one at a time, the lanes scanning a search box together
+    const Grid &g = a.g;
+    const int lane = __lane_id();
+    const long t = (((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kGhostNodes + lane;
     int i = 0, j = 0, k = 0;
     bool mine = false;
-    if (t < b.count) {
+    if (lane < kGhostNodes && t < b.count) {
         const long q = GeoNode(g, b, t, i, j, k);
         mine = (r == gst[q] && body.body + 1 == did[q]);
     }
@@ -1797,12 +1805,15 @@ __global__ __launch_bounds__(256) void ib_build(GhostBuildArgs a, GeoBox b, int 
             for (int s = 0; s < 3; ++s) c[s] = pG[s];
         }
     }
-    const int h = image ? 2 : 1, want = image ? 0 : body.body + 1, layer = image ? 0 : r - 1;
+    const int want = image ? 0 : body.body + 1, layer = image ? 0 : r - 1;
     unsigned long long todo = __ballot(mine);
-    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     // the wavefront's ghosts take consecutive entries from one reservation
-    int e = 0;
-    if (lane == 0 && todo) e = atomicAdd(counter, __popcll(todo));
+    // behind the entries of the layers before (counts complete by now)
+    int e = 0, *overflow = counters;
+    if (lane == 0 && todo) {
+        e = atomicAdd(counters + r, __popcll(todo));
+        for (int before = 1; before < r; ++before) e += counters[before];
+    }
     e = __shfl(e, 0) - 1;
     int myEntry = -1, myCount = 0;
     while (todo) {
@@ -1821,50 +1832,10 @@ __global__ __launch_bounds__(256) void ib_build(GhostBuildArgs a, GeoBox b, int 
         }
         const int first = e * kGhostSlot;
         int count = 0;
-        bool lost = false;
-        for (int rr = h; 0 == count; ++rr) {
-            if (rr > 3) {
-                lost = true;
-                break;
-            }
-            const int w = 2 * rr + 1, cand = w * w * w;
-            // every chunk's flags are loaded before the first ballot, so the
-            // loads of a search overlap
-            constexpr int kChunks = (kGhostSlot + 63) / 64;
-            int qv[kChunks];
-            bool hv[kChunks];
-#pragma unroll
-            for (int ch = 0; ch < kChunks; ++ch) {
-                const int cc = ch * 64 + lane;
-                hv[ch] = false;
-                qv[ch] = -1;
-                if (cc < cand) {
-                    const int x = ns[0] + cc % w - rr, y = ns[1] + (cc / w) % w - rr, z = ns[2] + cc / (w * w) - rr;
-                    if (z >= g.lo[2] && z < g.hi[2] && y >= g.lo[1] && y < g.hi[1] && x >= g.lo[0] && x < g.hi[0])
-                        qv[ch] = (int)(((long)z * g.ny + y) * g.nx + x);
-                }
-                if (qv[ch] >= 0) {
-                    const int dq = did[qv[ch]], gq2 = gst[qv[ch]];
-                    hv[ch] = (want == dq) && (layer == 0 || layer == gq2);
-                }
-            }
-#pragma unroll
-            for (int ch = 0; ch < kChunks; ++ch) {
-                if (ch * 64 >= cand) break;
-                const unsigned long long hits = __ballot(hv[ch]);
-                if (hv[ch]) {
-                    const int cc = ch * 64 + lane;
-                    const int x = ns[0] + cc % w - rr, y = ns[1] + (cc / w) % w - rr, z = ns[2] + cc / (w * w) - rr;
-                    double ph[3];
-                    GeoPoint(a.gs, x, y, z, ph);
-                    const int pos = count + __popcll(hits & below);
-                    snode[first + pos] = qv[ch];
-                    sw[first + pos] = GbInverse(a.tinyL, GbDist2(cs, ph));
-                }
-                count += __popcll(hits);
-            }
-        }
-        if (lost) {
+        if (!image) count = SearchBox<1>(a, ns, cs, want, layer, did, gst, snode + first, sw + first);
+        if (0 == count) count = SearchBox<2>(a, ns, cs, want, layer, did, gst, snode + first, sw + first);
+        if (0 == count) count = SearchBox<3>(a, ns, cs, want, layer, did, gst, snode + first, sw + first);
+        if (0 == count) {                           // beyond radius 3
             if (lane == 0) atomicOr(overflow, 1);
             continue;
         }
@@ -1901,72 +1872,68 @@ __global__ __launch_bounds__(256) void ib_build(GhostBuildArgs a, GeoBox b, int 
 // The surface-force table of one body on the device (the host's
 // artra_build_force_table over the device's flags): one workgroup scans the
 // body's node box in k-j-i order and appends its layer-2 ghosts in that
-// order (a block-wide prefix of ballots), with the normal, arm and distance
-// of each; it counts the body's interfacial layer-2 nodes.  counters[0] is
-// the table's running end, counters[1 + 2 slot] and [2 + 2 slot] the
-// body's ghost and interfacial counts.
+// order (a block-wide prefix of ballots); it counts the body's interfacial
+// layer-2 nodes.  The scan is one workgroup's, for the order, and bound by
+// the latency of its loads: 79 us for a sphere in 96^3 nodes, 124 with a
+// prefix for every 1024 nodes and the geometry in the same workgroup.
+// counters[0] is the table's running end, counters[1 + 2 slot] and
+// [2 + 2 slot] the body's ghost and interfacial counts.
 constexpr int kForceBuildThreads = 1024;
+constexpr int kForceChunks = 8;     // nodes a thread reads before a prefix: their loads overlap
 
-__global__ __launch_bounds__(kForceBuildThreads) void force_build(Grid g, GeoSetup gs, GeoBox b, GhostBody body,
-                                                                  int slot, int viscous, const int *did,
-                                                                  const int *fid, const int *lid, const int *gst,
-                                                                  ArtraForceNode *nodes, ArtraForceBody *bodies,
-                                                                  int cap, int *counters)
+__global__ __launch_bounds__(kForceBuildThreads) void force_build(Grid g, GeoBox b, GhostBody body, int slot,
+                                                                  int viscous, const int *did, const int *lid,
+                                                                  const int *gst, ArtraForceNode *nodes,
+                                                                  ArtraForceBody *bodies, int cap, int *counters)
 {
-    __shared__ int waveHits[kForceBuildThreads / 64];
+    constexpr int kWaves = kForceBuildThreads / 64;
+    __shared__ int waveHits[kForceChunks][kWaves];
     __shared__ int lidCount;
     const int tid = threadIdx.x, lane = __lane_id(), wave = tid >> 6;
     const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const int first = counters[0];
     if (tid == 0) lidCount = 0;
-    __syncthreads();
-    int end = first;
-    for (long start = 0; start < b.count; start += kForceBuildThreads) {
-        const long t = start + tid;
-        bool hit = false;
-        long q = 0;
-        if (t < b.count) {
+    int end = first, interfacial = 0;
+    for (long start = 0; start < b.count; start += kForceChunks * kForceBuildThreads) {
+        int q[kForceChunks], d[kForceChunks];
+        unsigned long long m[kForceChunks];
+#pragma unroll
+        for (int u = 0; u < kForceChunks; ++u) {
+            const long t = start + u * kForceBuildThreads + tid;
             int i, j, k;
-            q = GeoNode(g, b, t, i, j, k);
-            const int d = did[q];
-            if (body.body + 1 == d) {
-                hit = (2 == gst[q]);
-                if (2 == lid[q]) atomicAdd(&lidCount, 1);
-            }
+            q[u] = (t < b.count) ? (int)GeoNode(g, b, t, i, j, k) : -1;
+            d[u] = (q[u] < 0) ? 0 : did[q[u]];
         }
-        const unsigned long long m = __ballot(hit);
-        __syncthreads();                            // the last chunk's prefix is read
-        if (lane == 0) waveHits[wave] = __popcll(m);
+        int ghost[kForceChunks], near[kForceChunks];
+#pragma unroll
+        for (int u = 0; u < kForceChunks; ++u) {
+            const bool own = body.body + 1 == d[u];
+            ghost[u] = own ? gst[q[u]] : 0;
+            near[u] = own ? lid[q[u]] : 0;
+        }
+        __syncthreads();                            // the last pass's prefix is read
+#pragma unroll
+        for (int u = 0; u < kForceChunks; ++u) {
+            m[u] = __ballot(2 == ghost[u]);
+            interfacial += __popcll(__ballot(2 == near[u]));
+            if (lane == 0) waveHits[u][wave] = __popcll(m[u]);
+        }
         __syncthreads();
-        int before = end, total = 0;
-        for (int w = 0; w < kForceBuildThreads / 64; ++w) {
-            if (w < wave) before += waveHits[w];
-            total += waveHits[w];
+        for (int u = 0; u < kForceChunks; ++u) {
+            int before = end, total = 0;
+            for (int w = 0; w < kWaves; ++w) {
+                if (w < wave) before += waveHits[u][w];
+                total += waveHits[u][w];
+            }
+            if (2 == ghost[u]) {
+                const int pos = before + __popcll(m[u] & below);
+                if (pos < cap) nodes[pos].node = q[u];  // its geometry is force_geometry's
+            }
+            end += total;
         }
-        if (hit) {
-            const int pos = before + __popcll(m & below);
-            if (pos < cap) nodes[pos].node = (int)q;    // the geometry once every entry is placed
-        }
-        end += total;
     }
+    if (lane == 0 && interfacial) atomicAdd(&lidCount, interfacial);
     __syncthreads();
-    // each entry's normal, arm and distance, all entries at once
-    for (int e = first + tid; e < end && e < cap; e += kForceBuildThreads) {
-        const long q = nodes[e].node;
-        const int i = (int)(q % g.nx), j = (int)((q / g.nx) % g.ny), k = (int)(q / ((long)g.nx * g.ny));
-        double pG[3], pO[3], pI[3], N[3];
-        GeoPoint(gs, i, j, k, pG);
-        GcGeometricData(pG, fid[q], &body.pv, body.O, body.r, pO, pI, N);
-        ArtraForceNode rec;
-        rec.node = (int)q;
-        rec.body = slot;
-        for (int s = 0; s < 3; ++s) {
-            rec.N[s] = N[s];
-            rec.r[s] = pO[s] - body.O[s];
-        }
-        rec.dist = sqrt(GbDist2(pG, pO));
-        nodes[e] = rec;
-    }
     if (tid == 0) {
         counters[0] = end;
         counters[1 + 2 * slot] = end - first;
@@ -1984,6 +1951,30 @@ __global__ __launch_bounds__(kForceBuildThreads) void force_build(Grid g, GeoSet
     }
 }
 
+// The normal, arm and distance of the entries that force_build placed for
+// the body of `slot`.
+__global__ __launch_bounds__(256) void force_geometry(Grid g, GeoSetup gs, GhostBody body, int slot, const int *fid,
+                                                      ArtraForceNode *nodes, const ArtraForceBody *bodies, int cap)
+{
+    const int first = bodies[slot].first, end = min(first + bodies[slot].count, cap);
+    for (int e = first + blockIdx.x * blockDim.x + threadIdx.x; e < end; e += gridDim.x * blockDim.x) {
+        const long q = nodes[e].node;
+        const int i = (int)(q % g.nx), j = (int)((q / g.nx) % g.ny), k = (int)(q / ((long)g.nx * g.ny));
+        double pG[3], pO[3], pI[3], N[3];
+        GeoPoint(gs, i, j, k, pG);
+        GcGeometricData(pG, fid[q], &body.pv, body.O, body.r, pO, pI, N);
+        ArtraForceNode rec;
+        rec.node = (int)q;
+        rec.body = slot;
+        for (int s = 0; s < 3; ++s) {
+            rec.N[s] = N[s];
+            rec.r[s] = pO[s] - body.O[s];
+        }
+        rec.dist = sqrt(GbDist2(pG, pO));
+        nodes[e] = rec;
+    }
+}
+
 // A table of filled nodes on the device with its stencil entries; the
 // buffers grow as needed and are reused when the table is rebuilt.
 struct IbTable {
@@ -1993,6 +1984,23 @@ struct IbTable {
     int count = 0;
     int ghostCap = 0, stencilCap = 0;
 };
+
+// acc + x[0] + x[W] + ... + x[(m - 1) W], added in that order; sixteen reads
+// at a time are in flight ahead of the additions.
+template <int W>
+__device__ __forceinline__ double SumColumn(const double *x, int m, double acc)
+{
+    int e = 0;
+    for (; e + 16 <= m; e += 16) {
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = x[(e + u) * W];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) acc = acc + v[u];
+    }
+    for (; e < m; ++e) acc = acc + x[e * W];
+    return acc;
+}
 
 // The ghost node's state from the weighted sums of its stencil's primitive
 // states (Uo) and weights (wsum): for a first-layer ghost the boundary
@@ -2042,39 +2050,48 @@ __device__ __forceinline__ void IbFinish(double *U, const GhostDev &gh, double U
     StoreNode(U, gh.node, out);
 }
 
-// One 64-lane block per filled node: the lanes load and convert 64 stencil
-// entries at a time into LDS (the loop's memory latency overlapped), then
-// lane c < 6 sums component c of the weighted primitive states and lane 6
-// the weights, each over the entries in stencil order: the same operations
-// as a loop over the stencil (immersed_boundary.c:393-440), so the node's
-// state is bit for bit the reference's.  Grid: one block per entry of
-// [begin, end).
+// One 64-lane block per filled node: the lanes load, convert and weight 128
+// stencil entries at a time into LDS (two to a lane, both asked for before
+// either is waited for), then lane c < 6 sums component c of the weighted
+// primitive states and lane 6 the weights, each over the entries in stencil
+// order: the same operations as a loop over the stencil
+// (immersed_boundary.c:393-440), so the node's state is bit for bit the
+// reference's.  Bound by latency: the sums are chains of as many additions
+// as the stencil has entries, so their reads go ahead of them sixteen at a
+// time.  (A sphere in 96^3 nodes: 18 us a fill, 30 with 64 entries at a time
+// and each read in front of its addition.)
+// Grid: one block per entry of [begin, end).
 __global__ __launch_bounds__(64) void ib_fill(double *U, const GhostDev *ghosts, int begin, const int *snode,
                                               const double *sw, double gamma, double gasR)
 {
-    __shared__ double stage[64 * 7];
+    constexpr int kStage = 128;
+    __shared__ double stage[kStage * 7];
     __shared__ double part[7];
     const int lane = threadIdx.x;
     const GhostDev gh = ghosts[begin + blockIdx.x];
     double acc = 0.0;                               // lane c < 6: Uo[c]; lane 6: the weight sum
     const int last = gh.first + gh.count;
-    for (int base = gh.first; base < last; base += 64) {
-        const int q = base + lane;
-        if (q < last) {
-            double Uh[5], Uoh[6];
-            LoadNode(U, snode[q], Uh);
-            Primitive(gamma, gasR, Uh, Uoh);
+    for (int base = gh.first; base < last; base += kStage) {
+        double Uh[kStage / 64][5], w[kStage / 64];
 #pragma unroll
-            for (int c = 0; c < 6; ++c) stage[lane * 7 + c] = Uoh[c];
-            stage[lane * 7 + 6] = sw[q];
+        for (int h = 0; h < kStage / 64; ++h) {
+            const int q = base + 64 * h + lane;
+            if (q >= last) continue;
+            LoadNode(U, snode[q], Uh[h]);
+            w[h] = sw[q];
+        }
+#pragma unroll
+        for (int h = 0; h < kStage / 64; ++h) {
+            if (base + 64 * h + lane >= last) continue;
+            double Uoh[6], *to = stage + (64 * h + lane) * 7;
+            Primitive(gamma, gasR, Uh[h], Uoh);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) to[c] = Uoh[c] * w[h];
+            to[6] = w[h];
         }
         __syncthreads();
-        const int m = min(64, last - base);
-        if (lane < 6) {
-            for (int e = 0; e < m; ++e) acc = acc + stage[e * 7 + lane] * stage[e * 7 + 6];
-        } else if (lane == 6) {
-            for (int e = 0; e < m; ++e) acc = acc + stage[e * 7 + 6];
-        }
+        const int m = min(kStage, last - base);
+        if (lane < 7) acc = SumColumn<7>(stage + lane, m, acc);
         __syncthreads();
     }
     if (lane < 7) part[lane] = acc;
@@ -2135,38 +2152,67 @@ __global__ __launch_bounds__(256) void force_terms(const double *U, const ArtraF
     o[9] = Uo[4];
 }
 
+// One node's addition of force_sum: the term, the pressure less p0 (after =
+// p0; 0 elsewhere, where the subtraction changes nothing), or the square.
+__device__ __forceinline__ double AddTerm(double acc, double x, bool square, double p0, double after)
+{
+    const double d = x - p0;
+    return acc + (square ? d * d : x) - after;
+}
+
 // Per body, the sums of its nodes' terms in table order (the reference's
 // loop order, so the sums are those of its serial loop) and the pressure
 // statistics: fvar = (p of the first node, sum (p - p0), sum (p - p0)^2).
-// One 64-lane block per body: 64 nodes' terms at a time are staged in LDS,
-// then lane q < 9 sums term q and lanes 9 and 10 the two statistics, each
-// over the nodes in table order (the serial loop's additions, without its
-// memory latency per node).
-__global__ __launch_bounds__(64) void force_sum(const ArtraForceBody *bodies, int nbody, const double *terms,
-                                                double *sums)
+// One block per body: the terms of 256 nodes at a time are staged in LDS by
+// coalesced loads, the next ones asked for before these are summed; then
+// lane q < 9 sums term q and lanes 9 and 10 the two statistics, each over
+// the nodes in table order (the serial loop's additions).  Bound by those
+// chains of additions, one or (lane 9) two to a node.  (A sphere in
+// 96^3 nodes: 74 us, 150 with 64 nodes at a time and the three kinds of sum
+// one after the other.)
+constexpr int kForceStage = 256;
+
+__global__ __launch_bounds__(kForceStage) void force_sum(const ArtraForceBody *bodies, int nbody, const double *terms,
+                                                         double *sums)
 {
-    __shared__ double stage[64 * 10];
+    __shared__ double stage[kForceStage * 10];
     const int b = blockIdx.x;
     if (b >= nbody) return;                         // uniform over the block
     const int lane = threadIdx.x;
     const ArtraForceBody bd = bodies[b];
-    const int last = bd.first + bd.count;
-    const double p0 = (bd.count > 0) ? terms[(size_t)bd.first * 10 + 9] : 0.0;
-    double acc = 0.0;
-    for (int base = bd.first; base < last; base += 64) {
-        const int t = base + lane;
-        if (t < last) {
+    const long words = (long)bd.count * 10;
+    const double *from = terms + (size_t)bd.first * 10;
+    const double p0 = (bd.count > 0) ? from[9] : 0.0;
+    // lanes below 9 add the term itself, lane 9 the pressure and then -p0,
+    // lane 10 the square of their difference
+    const double after = (lane == 9) ? p0 : 0.0;
+    const int column = min(lane, 9);
+    double acc = 0.0, v[10];
 #pragma unroll
-            for (int q = 0; q < 10; ++q) stage[lane * 10 + q] = terms[(size_t)t * 10 + q];
-        }
+    for (int u = 0; u < 10; ++u) {
+        const long q = lane + (long)kForceStage * u;
+        v[u] = (q < words) ? from[q] : 0.0;
+    }
+    for (int base = 0; base < bd.count; base += kForceStage) {
+#pragma unroll
+        for (int u = 0; u < 10; ++u) stage[lane + kForceStage * u] = v[u];
         __syncthreads();
-        const int m = min(64, last - base);
-        if (lane < 9) {
-            for (int e = 0; e < m; ++e) acc = acc + stage[e * 10 + lane];
-        } else if (lane == 9) {
-            for (int e = 0; e < m; ++e) acc = acc + stage[e * 10 + 9] - p0;
-        } else if (lane == 10) {
-            for (int e = 0; e < m; ++e) acc = acc + (stage[e * 10 + 9] - p0) * (stage[e * 10 + 9] - p0);
+#pragma unroll
+        for (int u = 0; u < 10; ++u) {
+            const long q = (long)(base + kForceStage) * 10 + lane + (long)kForceStage * u;
+            v[u] = (q < words) ? from[q] : 0.0;
+        }
+        const int m = min(kForceStage, bd.count - base);
+        if (lane < 11) {
+            int e = 0;
+            for (; e + 16 <= m; e += 16) {
+                double x[16];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) x[u] = stage[(e + u) * 10 + column];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) acc = AddTerm(acc, x[u], lane == 10, p0, after);
+            }
+            for (; e < m; ++e) acc = AddTerm(acc, stage[e * 10 + column], lane == 10, p0, after);
         }
         __syncthreads();
     }
@@ -3645,7 +3691,9 @@ int artra_dev_set_axis_gather(ArtraDevice *dev, int s, const ArtraBcGather *gt)
         DeriveWallRules(dev, s);
         return 0;
     }
-    DeriveLineRules(dev, s, gt->count, gt->dst, gt->src);
+    // (with bodies in the grid no line runs fused: their 30 ms on 512 x 512
+    // lines would be for nothing)
+    if (dev->allFluid) DeriveLineRules(dev, s, gt->count, gt->dst, gt->src);
     const long n = gt->count;
     if (n > 0) {
         HIP_TRY(hipMalloc(&dev->gDst[m], n * sizeof(int)));
@@ -3842,7 +3890,7 @@ int artra_dev_surface_force(ArtraDevice *dev, double *sums)
                            dev->par.gamma, dev->par.gasR, dev->par.refMu, dev->par.refT, dev->forceTerms);
         HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL(force_sum, dim3(dev->forceBodyCount), dim3(64), 0, dev->stream, dev->forceBodies,
+    hipLaunchKernelGGL(force_sum, dim3(dev->forceBodyCount), dim3(kForceStage), 0, dev->stream, dev->forceBodies,
                        dev->forceBodyCount, dev->forceTerms, dev->forceSums);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(sums, dev->forceSums, (size_t)dev->forceBodyCount * 12 * sizeof(double),
@@ -4859,7 +4907,7 @@ int artra_dev_build_ghosts(ArtraDevice *dev, const ArtraGeoBody *bodies, int nbo
     }
     if (!dev->geoCounters) HIP_TRY(hipMalloc(&dev->geoCounters, kGeoCounters * sizeof(int)));
     if (!dev->geoCountsHost) HIP_TRY(hipHostMalloc(&dev->geoCountsHost, kGeoCounters * sizeof(int)));
-    HIP_TRY(hipMemsetAsync(dev->geoCounters, 0, 2 * sizeof(int), dev->stream));
+    HIP_TRY(hipMemsetAsync(dev->geoCounters, 0, kGeoCounters * sizeof(int), dev->stream));
     GhostBuildArgs a;
     a.g = g;
     a.gs = dev->geo;
@@ -4899,26 +4947,24 @@ int artra_dev_build_ghosts(ArtraDevice *dev, const ArtraGeoBody *bodies, int nbo
             gbody.cf = bd.cf;
             gbody.T = bd.T;
             gbody.body = n;
-            hipLaunchKernelGGL(ib_build, dim3((unsigned)((bb.count + 255) / 256)), dim3(256), 0, dev->stream, a, bb, r,
-                               gbody, did, fid, gst, tb.ghosts, tb.snode, tb.sw, dev->geoCounters,
-                               dev->geoCounters + 1);
+            const long perBlock = 4 * kGhostNodes;
+            hipLaunchKernelGGL(ib_build, dim3((unsigned)((bb.count + perBlock - 1) / perBlock)), dim3(256), 0,
+                               dev->stream, a, bb, r, gbody, did, fid, gst, tb.ghosts, tb.snode, tb.sw,
+                               dev->geoCounters);
             HIP_TRY(hipGetLastError());
         }
-        // the table's end after layer r, kept on the device until all are built
-        HIP_TRY(hipMemcpyAsync(dev->geoCounters + 2 + r, dev->geoCounters, sizeof(int), hipMemcpyDeviceToDevice,
-                               dev->stream));
     }
     int *c = dev->geoCountsHost;
-    HIP_TRY(hipMemcpyAsync(c, dev->geoCounters, (size_t)(layers + 3) * sizeof(int), hipMemcpyDeviceToHost,
+    HIP_TRY(hipMemcpyAsync(c, dev->geoCounters, (size_t)(layers + 1) * sizeof(int), hipMemcpyDeviceToHost,
                            dev->stream));
     HIP_TRY(hipStreamSynchronize(dev->stream));
-    if (c[1] || c[0] > tb.ghostCap) {
-        tb.count = std::min(c[0], tb.ghostCap);  // the next build allocates room for them
+    std::vector<int> layerEnd(layers + 1, 0);
+    for (int r = 1; r <= layers; ++r) layerEnd[r] = layerEnd[r - 1] + c[r];
+    if (c[0] || layerEnd[layers] > tb.ghostCap) {
+        tb.count = std::min(layerEnd[layers], tb.ghostCap);  // the next build allocates room for them
         *fallback = 1;
         return 0;
     }
-    std::vector<int> layerEnd(layers + 1, 0);
-    for (int r = 1; r <= layers; ++r) layerEnd[r] = c[2 + r];
     tb.count = layerEnd[layers];
     dev->layerStart.assign(layerEnd.begin(), layerEnd.end());
     dev->ibImageOnly = (ibmLayer >= layers);
@@ -4987,9 +5033,11 @@ int artra_dev_build_force_table(ArtraDevice *dev, const ArtraGeoBody *bodies, in
             gbody.cf = bd.cf;
             gbody.T = bd.T;
             gbody.body = n;
-            hipLaunchKernelGGL(force_build, dim3(1), dim3(kForceBuildThreads), 0, dev->stream, dev->g, dev->geo, bb,
-                               gbody, b, viscous[b], did, fid, lid, gst, dev->forceNodes, dev->forceBodies,
-                               dev->forceNodeCap, dev->forceCounters);
+            hipLaunchKernelGGL(force_build, dim3(1), dim3(kForceBuildThreads), 0, dev->stream, dev->g, bb, gbody, b,
+                               viscous[b], did, lid, gst, dev->forceNodes, dev->forceBodies, dev->forceNodeCap,
+                               dev->forceCounters);
+            hipLaunchKernelGGL(force_geometry, dim3(64), dim3(256), 0, dev->stream, dev->g, dev->geo, gbody, b, fid,
+                               dev->forceNodes, dev->forceBodies, dev->forceNodeCap);
             HIP_TRY(hipGetLastError());
         }
         int *c = dev->forceCountsHost;
