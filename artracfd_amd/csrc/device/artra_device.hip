@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1475,16 +1476,37 @@ __device__ __forceinline__ void GeoPoint(const GeoSetup &gs, int i, int j, int k
     p[2] = gs.smin[2] + (k - gs.ng[2]) * gs.d[2];
 }
 
+// The result of a classification for the host: the number of changed nodes,
+// per body the lowest and highest i, j, k of its nodes (lowest > highest: it
+// has none), then a record per changed node, in no order: its place in the
+// region in k-j-i order, its did, fid, lid, gst and previous domain field.
+// A half-step moves a body by a fraction of a cell, so few nodes change
+// while the region's flags are megabytes: the host reads and writes what
+// changed only.
+__host__ __device__ __forceinline__ long GeoHeader(int nbody)
+{
+    return 1 + 6l * nbody;
+}
+
+constexpr int kGeoRecord = ARTRA_GEO_RECORD;
+
 // Pass 1 (immersed_boundary.c:72-113): keep the domain field in gst, clear
 // the fluid nodes' face links, release the interfacial nodes of moving bodies.
+// The flags that pass 3 compares with go to `before` (fid, then gst), and
+// the list of changes (GeoChange) starts empty.
 __global__ __launch_bounds__(256) void geo_reset(Grid g, GeoBox b, int *did, int *fid, const int *lid, int *gst,
-                                                 const int *moving, int nbody)
+                                                 const int *moving, int nbody, int *before, int *changes)
 {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    for (long e = t; e < GeoHeader(nbody); e += (long)gridDim.x * blockDim.x) {
+        changes[e] = (e == 0) ? 0 : ((e - 1) % 6 < 3) ? INT_MAX : INT_MIN;
+    }
     if (t >= b.count) return;
     int i, j, k;
     const long q = GeoNode(g, b, t, i, j, k);
     const int gid = did[q];
+    before[t] = fid[q];
+    before[b.count + t] = gst[q];
     gst[q] = gid;
     if (0 == gid) {
         fid[q] = 0;
@@ -1655,29 +1677,56 @@ __device__ int GeoInterState(const Grid &g, const GeoSetup &gs, const int *didv,
 }
 
 // Pass 3's interfacial states (immersed_boundary.c:183-225, which read did
-// only), the sweeps' fluid flags, and the region's flags packed for the host:
-// packed[0..4][t] = did, fid, lid, gst and the previous domain field.
-__global__ __launch_bounds__(256) void geo_interface(Grid g, GeoSetup gs, GeoBox b, const int *did, const int *fid,
-                                                     int *lid, int *gst, uint8_t *fluid, int *packed)
+// only), the sweeps' fluid flags, the changes for the host and the boxes of
+// the moving bodies' nodes.  A node that a body uncovered gets the mark of a
+// reconstructed node (fid -1, as on the host).
+__global__ __launch_bounds__(256) void geo_interface(Grid g, GeoSetup gs, GeoBox b, const int *did, int *fid,
+                                                     int *lid, int *gst, uint8_t *fluid, const int *moving, int nbody,
+                                                     const int *before, int *changes)
 {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= b.count) return;
-    int i, j, k;
-    const long q = GeoNode(g, b, t, i, j, k);
-    const int dq = did[q];
-    int l = 0, s = 0;
-    if (0 != dq) {
-        l = GeoInterState(g, gs, did, k, j, i, dq, false);
-        if (0 < l) s = GeoInterState(g, gs, did, k, j, i, 0, true);
+    bool changed = false;
+    int i = 0, j = 0, k = 0, dq = 0, f = 0, l = 0, s = 0, prev = 0;
+    if (t < b.count) {
+        const long q = GeoNode(g, b, t, i, j, k);
+        dq = did[q];
+        f = fid[q];
+        prev = gst[q];                              // the previous domain field (pass 1)
+        if (0 != dq) {
+            l = GeoInterState(g, gs, did, k, j, i, dq, false);
+            if (0 < l) s = GeoInterState(g, gs, did, k, j, i, 0, true);
+        }
+        changed = dq != prev || f != before[t] || l != lid[q] || s != before[b.count + t];
+        if (0 == dq && dq != prev) fid[q] = -1;
+        lid[q] = l;
+        gst[q] = s;
+        fluid[q] = (0 == dq);
     }
-    packed[t] = dq;
-    packed[b.count + t] = fid[q];
-    packed[2 * b.count + t] = l;
-    packed[3 * b.count + t] = s;
-    packed[4 * b.count + t] = gst[q];               // the previous domain field (pass 1)
-    lid[q] = l;
-    gst[q] = s;
-    fluid[q] = (0 == dq);
+    const int lane = __lane_id();
+    const unsigned long long m = __ballot(changed);
+    int e = 0;
+    if (lane == 0 && m) e = atomicAdd(changes, __popcll(m));
+    e = __shfl(e, 0) + __popcll(m & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))));
+    if (changed) {
+        int *rec = changes + GeoHeader(nbody) + (long)e * kGeoRecord;
+        rec[0] = (int)t;
+        rec[1] = dq;
+        rec[2] = f;
+        rec[3] = l;
+        rec[4] = s;
+        rec[5] = prev;
+    }
+    // the words only widen: a node inside what it reads there adds nothing
+    if (0 < dq && dq <= nbody && moving[dq - 1]) {
+        int *box = changes + 1 + 6 * (dq - 1);
+        const int c[3] = {i, j, k};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (c[d] < __hip_atomic_load(box + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(box + d, c[d]);
+            if (c[d] > __hip_atomic_load(box + 3 + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                atomicMax(box + 3 + d, c[d]);
+        }
+    }
 }
 
 // The ghost table on the device (immersed_boundary.c:270-487 via
@@ -2542,9 +2591,10 @@ struct ArtraDevice {
     // the node classification of moving bodies (did, fid, lid, gst), kept
     // on the device and reclassified there after every move
     int *geoFlags = nullptr;        // [4][N]
-    int *geoPacked = nullptr;       // [5][region nodes] for the host's copy
-    int *geoPackedHost = nullptr;   // that copy (pinned)
-    long geoPackedCap = 0;
+    int *geoBefore = nullptr;       // [2][region nodes] flags before a classification
+    int *geoChanges = nullptr;      // its result for the host (GeoHeader)
+    int *geoChangesHost = nullptr;  // the host's copy (pinned)
+    long geoRegionCap = 0;          // region nodes these hold
     int *geoMoving = nullptr;       // [bodies]: 1 for a body that moves
     int *geoCounters = nullptr;     // ghost-table build: entries taken, overflow, each layer's end
     int *geoCountsHost = nullptr;   // their pinned host copy
@@ -3573,8 +3623,9 @@ void artra_dev_destroy(ArtraDevice *dev)
     hipFree(dev->fluid);
     hipFree(dev->flagStage);
     hipFree(dev->geoFlags);
-    hipFree(dev->geoPacked);
-    hipHostFree(dev->geoPackedHost);
+    hipFree(dev->geoBefore);
+    hipFree(dev->geoChanges);
+    hipHostFree(dev->geoChangesHost);
     hipFree(dev->geoMoving);
     hipFree(dev->geoCounters);
     hipHostFree(dev->geoCountsHost);
@@ -4744,6 +4795,7 @@ int artra_dev_geo_init(ArtraDevice *dev, const ArtraGeoSetup *setup, const int *
         dev->geoBodies.assign(nbody, GeoBodyDev());
         hipFree(dev->geoMoving);
         dev->geoMoving = nullptr;
+        dev->geoRegionCap = 0;                      // the changes' header grows with the bodies
         HIP_TRY(hipMalloc(&dev->geoMoving, (size_t)(nbody > 0 ? nbody : 1) * sizeof(int)));
     }
     dev->geo = *setup;
@@ -4751,10 +4803,9 @@ int artra_dev_geo_init(ArtraDevice *dev, const ArtraGeoSetup *setup, const int *
 }
 
 int artra_dev_geo_classify(ArtraDevice *dev, const ArtraGeoBody *bodies, int nbody, const int region[3][2],
-                           const int **packed, long *count)
+                           ArtraGeoResult *result)
 {
-    *count = 0;
-    *packed = nullptr;
+    *result = ArtraGeoResult{};
     if (!dev->geoFlags || nbody != (int)dev->geoBodies.size()) return Fail("moving-body classification not set up");
     ++dev->configGen;
     dev->allFluid = 0;                              // bodies present: the stage-by-stage sweeps
@@ -4819,19 +4870,22 @@ int artra_dev_geo_classify(ArtraDevice *dev, const ArtraGeoBody *bodies, int nbo
         rb.count *= rb.n[s];
     }
     if (rb.count == 0) return 0;
-    if (5 * rb.count > dev->geoPackedCap) {
-        hipFree(dev->geoPacked);
-        hipHostFree(dev->geoPackedHost);
-        dev->geoPacked = nullptr;
-        dev->geoPackedHost = nullptr;
-        dev->geoPackedCap = 0;
-        HIP_TRY(hipMalloc(&dev->geoPacked, (size_t)5 * rb.count * sizeof(int)));
-        HIP_TRY(hipHostMalloc(&dev->geoPackedHost, (size_t)5 * rb.count * sizeof(int)));
-        dev->geoPackedCap = 5 * rb.count;
+    const long header = GeoHeader(nbody);
+    if (rb.count > dev->geoRegionCap) {
+        hipFree(dev->geoBefore);
+        hipFree(dev->geoChanges);
+        hipHostFree(dev->geoChangesHost);
+        dev->geoBefore = dev->geoChanges = dev->geoChangesHost = nullptr;
+        dev->geoRegionCap = 0;
+        const size_t list = (size_t)(header + kGeoRecord * rb.count) * sizeof(int);
+        HIP_TRY(hipMalloc(&dev->geoBefore, (size_t)2 * rb.count * sizeof(int)));
+        HIP_TRY(hipMalloc(&dev->geoChanges, list));
+        HIP_TRY(hipHostMalloc(&dev->geoChangesHost, list));
+        dev->geoRegionCap = rb.count;
     }
     const GeoSetup gs = dev->geo;
     hipLaunchKernelGGL(geo_reset, dim3((unsigned)((rb.count + 255) / 256)), dim3(256), 0, dev->stream, g, rb, did, fid,
-                       lid, gst, dev->geoMoving, nbody);
+                       lid, gst, dev->geoMoving, nbody, dev->geoBefore, dev->geoChanges);
     HIP_TRY(hipGetLastError());
     for (int n = 0; n < nbody; ++n) {
         const ArtraGeoBody &bd = bodies[n];
@@ -4865,13 +4919,26 @@ int artra_dev_geo_classify(ArtraDevice *dev, const ArtraGeoBody *bodies, int nbo
         HIP_TRY(hipGetLastError());
     }
     hipLaunchKernelGGL(geo_interface, dim3((unsigned)((rb.count + 255) / 256)), dim3(256), 0, dev->stream, g, gs, rb,
-                       did, fid, lid, gst, dev->fluid, dev->geoPacked);
+                       did, fid, lid, gst, dev->fluid, dev->geoMoving, nbody, dev->geoBefore, dev->geoChanges);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(dev->geoPackedHost, dev->geoPacked, (size_t)5 * rb.count * sizeof(int),
+    // the header with the first records, the rest if there are more
+    int *host = dev->geoChangesHost;
+    const long guess = std::min(rb.count, 1024l);
+    HIP_TRY(hipMemcpyAsync(host, dev->geoChanges, (size_t)(header + kGeoRecord * guess) * sizeof(int),
                            hipMemcpyDeviceToHost, dev->stream));
     HIP_TRY(hipStreamSynchronize(dev->stream));
-    *packed = dev->geoPackedHost;
-    *count = rb.count;
+    const long changes = host[0];
+    if (changes > guess) {
+        const long from = header + kGeoRecord * guess;
+        HIP_TRY(hipMemcpyAsync(host + from, dev->geoChanges + from,
+                               (size_t)(kGeoRecord * (changes - guess)) * sizeof(int), hipMemcpyDeviceToHost,
+                               dev->stream));
+        HIP_TRY(hipStreamSynchronize(dev->stream));
+    }
+    result->nodes = rb.count;
+    result->changes = changes;
+    result->extent = (const int (*)[2][DIMS])(host + 1);
+    result->change = (const int (*)[ARTRA_GEO_RECORD])(host + header);
     return 0;
 }
 

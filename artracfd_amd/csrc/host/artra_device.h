@@ -131,13 +131,25 @@ int artra_dev_build_force_table(ArtraDevice *dev, const ArtraGeoBody *bodies, in
 
 /* The flags did, fid, lid, gst ([4][N], host order) onto the device. */
 int artra_dev_geo_init(ArtraDevice *dev, const ArtraGeoSetup *setup, const int *flags, int nbody);
+/* What a classification changed: per changed node of the region its place in
+ * k-j-i order, did, fid, lid, gst and previous domain field, in no order
+ * (the host's flags equal the device's before it); per body the lowest and
+ * highest i, j, k of its nodes if it moves (lowest > highest without any). */
+enum { ARTRA_GEO_RECORD = 6 };
+
+typedef struct {
+    long nodes;                     /* of the region */
+    long changes;
+    const int (*change)[ARTRA_GEO_RECORD];
+    const int (*extent)[2][DIMS];
+} ArtraGeoResult;
+
 /* ComputeGeometricField's three passes (immersed_boundary.c:65-264) over
  * region on the device (the domain field over each moving body's box), the
- * sweeps' fluid flags updated; *packed points to [5][*count] ints, the
- * region's new did, fid, lid, gst and previous domain field in k-j-i order,
- * held by the device until its next classification. */
+ * sweeps' fluid flags updated; *result points to memory held by the device
+ * until its next classification. */
 int artra_dev_geo_classify(ArtraDevice *dev, const ArtraGeoBody *bodies, int nbody, const int region[DIMS][LIMIT],
-                           const int **packed, long *count);
+                           ArtraGeoResult *result);
 
 /* replay the device march's step from a captured graph (1, the default) or
  * launch its kernels one by one (0) */

@@ -124,13 +124,13 @@ int artra_compute_geometric_field(Space *space, const Model *model, ArtraGhostTa
  * artra_scope_update refreshes the scope from the new classification (the
  * moving bodies' nodes all lie inside that region).
  */
-/* The host's copy of a classification made on the device over region:
- * packed[5][count] = did, fid, lid, gst and the previous domain field of
- * the region's nodes in k-j-i order (artra_dev_geo_classify).  The nodes a
- * body uncovered are listed in joins (artra_add_join, on the flags as the
+/* The host's copy of a classification made on the device over a region of
+ * `count` nodes, from its changes: change[] = place in the region in k-j-i
+ * order, did, fid, lid, gst and previous domain field.  The nodes a body
+ * uncovered are listed in joins (artra_add_join, on the flags as the
  * reference's interfacial pass finds them) and marked fid = -1. */
-int artra_apply_classification(Space *space, const int region[DIMS][LIMIT], const int *packed, long count,
-                               ArtraGhostTable *joins);
+int artra_apply_classification(Space *space, const int region[DIMS][LIMIT], const int (*change)[6], long changes,
+                               long count, ArtraGhostTable *joins);
 
 typedef struct {
     int bodies;
@@ -142,6 +142,10 @@ void artra_scope_free(ArtraGeometryScope *scope);
 void artra_scope_region(const Space *space, const ArtraGeometryScope *scope, int region[DIMS][LIMIT]);
 void artra_scope_update(const Space *space, ArtraGeometryScope *scope, const ArtraGhostTable *joins,
                         const int region[DIMS][LIMIT]);
+/* the same from the boxes that a classification found: extent[body] = lowest
+ * and highest i, j, k (NULL: no moving body has nodes) */
+void artra_scope_extents(const Space *space, ArtraGeometryScope *scope, const ArtraGhostTable *joins,
+                         const int (*extent)[2][DIMS]);
 void artra_identify_geometry_state(Geometry *geo);
 
 /* ------------------------------------------------- device-side tables */

@@ -672,6 +672,16 @@ void artra_scope_region(const Space *space, const ArtraGeometryScope *sc, int re
     AddBox(region, (const int (*)[LIMIT])sc->join);
 }
 
+static void ScopeJoins(const Partition *part, ArtraGeometryScope *sc, const ArtraGhostTable *joins)
+{
+    EmptyBox(sc->join);
+    for (int q = 0; joins && q < joins->nghost; ++q) {
+        const int idx = joins->ghosts[q].node;
+        const int i = idx % part->n[X], j = (idx / part->n[X]) % part->n[Y], k = idx / (part->n[X] * part->n[Y]);
+        AddNode(sc->join, k, j, i);
+    }
+}
+
 void artra_scope_update(const Space *space, ArtraGeometryScope *sc, const ArtraGhostTable *joins,
                         const int region[DIMS][LIMIT])
 {
@@ -691,52 +701,75 @@ void artra_scope_update(const Space *space, ArtraGeometryScope *sc, const ArtraG
                 const int did = space->node[artra_index(k, j, i, part->n[Y], part->n[X])].did;
                 if (0 < did && did <= geo->totN && 1 != geo->poly[did - 1].state) AddNode(sc->extent[did - 1], k, j, i);
             }
-    EmptyBox(sc->join);
-    for (int q = 0; joins && q < joins->nghost; ++q) {
-        const int idx = joins->ghosts[q].node;
-        const int i = idx % part->n[X], j = (idx / part->n[X]) % part->n[Y], k = idx / (part->n[X] * part->n[Y]);
-        AddNode(sc->join, k, j, i);
-    }
+    ScopeJoins(part, sc, joins);
 }
 
-int artra_apply_classification(Space *space, const int region[DIMS][LIMIT], const int *packed, long count,
-                               ArtraGhostTable *joins)
+void artra_scope_extents(const Space *space, ArtraGeometryScope *sc, const ArtraGhostTable *joins,
+                         const int (*extent)[LIMIT][DIMS])
+{
+    const Geometry *geo = &space->geo;
+    for (int n = 0; n < geo->totN; ++n) {
+        if (1 == geo->poly[n].state) continue;
+        EmptyBox(sc->extent[n]);
+        if (NULL == extent || extent[n][MIN][X] > extent[n][MAX][X]) continue;
+        AddNode(sc->extent[n], extent[n][MIN][Z], extent[n][MIN][Y], extent[n][MIN][X]);
+        AddNode(sc->extent[n], extent[n][MAX][Z], extent[n][MAX][Y], extent[n][MAX][X]);
+    }
+    ScopeJoins(&space->part, sc, joins);
+}
+
+static int ByPlace(const void *a, const void *b)
+{
+    const int p = **(const int *const *)a, q = **(const int *const *)b;
+    return (p > q) - (p < q);
+}
+
+int artra_apply_classification(Space *space, const int region[DIMS][LIMIT], const int (*change)[6], long changes,
+                               long count, ArtraGhostTable *joins)
 {
     const Partition *part = &space->part;
     Node *node = space->node;
-    int lo[DIMS], hi[DIMS];
+    int lo[DIMS], n[DIMS];
     long span = 1;
     for (int s = 0; s < DIMS; ++s) {
         lo[s] = (region[s][MIN] > part->ns[PIN][s][MIN]) ? region[s][MIN] : part->ns[PIN][s][MIN];
-        hi[s] = (region[s][MAX] < part->ns[PIN][s][MAX]) ? region[s][MAX] : part->ns[PIN][s][MAX];
-        span *= (hi[s] > lo[s]) ? hi[s] - lo[s] : 0;
+        const int hi = (region[s][MAX] < part->ns[PIN][s][MAX]) ? region[s][MAX] : part->ns[PIN][s][MAX];
+        n[s] = (hi > lo[s]) ? hi - lo[s] : 0;
+        span *= n[s];
     }
     if (span != count) return artra_set_error(1, "classification of %ld nodes for a region of %ld", count, span);
+    if (0 == changes) return 0;
     /* the flags as the reference's interfacial pass finds them: the new
-     * domain field, gst still holding the previous one */
-    long t = 0;
-    for (int k = lo[Z]; k < hi[Z]; ++k)
-        for (int j = lo[Y]; j < hi[Y]; ++j)
-            for (int i = lo[X]; i < hi[X]; ++i, ++t) {
-                Node *nd = node + artra_index(k, j, i, part->n[Y], part->n[X]);
-                nd->did = packed[t];
-                nd->fid = packed[count + t];
-                nd->gst = packed[4 * count + t];
-            }
-    for (int k = lo[Z]; k < hi[Z]; ++k)
-        for (int j = lo[Y]; j < hi[Y]; ++j)
-            for (int i = lo[X]; i < hi[X]; ++i) {
-                const Node *nd = node + artra_index(k, j, i, part->n[Y], part->n[X]);
-                if (nd->gst != nd->did && 0 == nd->did && artra_add_join(space, k, j, i, joins)) return 1;
-            }
+     * domain field, gst still holding the previous one (a node that did not
+     * change is fluid with gst 0 in both, or in a body, which no stencil of
+     * a reconstruction takes) */
+    const int **uncovered = malloc((size_t)changes * sizeof *uncovered);
+    if (NULL == uncovered) return artra_set_error(1, "out of host memory for %ld changed nodes", changes);
+    long joined = 0;
+    for (long e = 0; e < changes; ++e) {
+        const int *c = change[e];
+        const int i = lo[X] + c[0] % n[X], j = lo[Y] + (c[0] / n[X]) % n[Y], k = lo[Z] + c[0] / (n[X] * n[Y]);
+        Node *nd = node + artra_index(k, j, i, part->n[Y], part->n[X]);
+        nd->did = c[1];
+        nd->fid = c[2];
+        nd->gst = c[5];
+        if (c[5] != c[1] && 0 == c[1]) uncovered[joined++] = c;
+    }
+    qsort(uncovered, (size_t)joined, sizeof *uncovered, ByPlace);
+    int rc = 0;
+    for (long e = 0; e < joined && !rc; ++e) {
+        const int t = *uncovered[e];
+        rc = artra_add_join(space, lo[Z] + t / (n[X] * n[Y]), lo[Y] + (t / n[X]) % n[Y], lo[X] + t % n[X], joins);
+    }
+    free(uncovered);
+    if (rc) return 1;
     for (int q = 0; q < joins->nghost; ++q) node[joins->ghosts[q].node].fid = NONE;
-    t = 0;
-    for (int k = lo[Z]; k < hi[Z]; ++k)
-        for (int j = lo[Y]; j < hi[Y]; ++j)
-            for (int i = lo[X]; i < hi[X]; ++i, ++t) {
-                Node *nd = node + artra_index(k, j, i, part->n[Y], part->n[X]);
-                nd->lid = packed[2 * count + t];
-                nd->gst = packed[3 * count + t];
-            }
+    for (long e = 0; e < changes; ++e) {
+        const int *c = change[e];
+        const int i = lo[X] + c[0] % n[X], j = lo[Y] + (c[0] / n[X]) % n[Y], k = lo[Z] + c[0] / (n[X] * n[Y]);
+        Node *nd = node + artra_index(k, j, i, part->n[Y], part->n[X]);
+        nd->lid = c[3];
+        nd->gst = c[4];
+    }
     return 0;
 }

@@ -327,15 +327,17 @@ static ArtraGeoBody *GeoBodies(const Space *space)
 }
 
 /* ComputeGeometricField over region on the device, the host's flags
- * updated from it and the uncovered nodes listed in joins. */
+ * updated from it, the uncovered nodes listed in joins and the scope
+ * refreshed. */
 static int ClassifyOnDevice(ArtraHipSolver *s, const int region[DIMS][LIMIT], const ArtraGeoBody *bodies,
                             ArtraGhostTable *joins)
 {
     Space *space = s->space;
-    const int *packed = NULL;
-    long count = 0;
-    if (artra_dev_geo_classify(s->dev, bodies, space->geo.totN, region, &packed, &count)) return artra_dev_failed();
-    return artra_apply_classification(space, region, packed, count, joins);
+    ArtraGeoResult result;
+    if (artra_dev_geo_classify(s->dev, bodies, space->geo.totN, region, &result)) return artra_dev_failed();
+    if (artra_apply_classification(space, region, result.change, result.changes, result.nodes, joins)) return 1;
+    artra_scope_extents(space, &s->scope, joins, result.extent);
+    return 0;
 }
 
 /* The surface-force table built on the device from its flags
@@ -447,7 +449,6 @@ int artra_solid_step(ArtraHipSolver *s, Real now, Real dt)
     ArtraGeoBody *bodies = GeoBodies(space);
     int rc = bodies ? 0 : artra_set_error(1, "out of host memory");
     if (!rc) rc = ClassifyOnDevice(s, (const int (*)[LIMIT])region, bodies, &joins);
-    if (!rc) artra_scope_update(space, &s->scope, &joins, (const int (*)[LIMIT])region);
     if (!rc) rc = TablesOnDevice(s, bodies);
     free(bodies);
     if (!rc && artra_dev_reconstruct(s->dev, TO, &joins)) rc = artra_dev_failed();

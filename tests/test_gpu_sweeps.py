@@ -149,3 +149,40 @@ def test_batched_lines_at_the_edges_of_their_blocks(tmp_path):
     for s, c in zip(solvers, cases):
         s.close()
         c.close()
+
+
+@pytest.mark.parametrize("m, r, steps", [(64, 0.41, 3), (24, 0.2, 4)])
+def test_flags_of_a_moving_body_reach_the_host(tmp_path, m, r, steps):
+    """The host's flags after half-steps that change thousands of nodes (more
+    than one copy of the changes holds) and few: the domain field is the
+    sphere at its last position, interfacial layer 1 its nodes with a fluid
+    neighbour, ghosts exactly the body's interfacial nodes."""
+    from artracfd_amd import Case, Solver
+    d = tmp_path / "case"
+    d.mkdir()
+    (d / "artracfd.case").write_text(mc.case_text(((-0.5, -0.5, -0.5), (0.5, 0.5, 0.5), (m, m, m)),
+                                                  (0, 1e9, 0.6, 0, 1, 0), (1, 1, 0, 0, 0, 1, 1), mc.INVISCID, mc.REF1,
+                                                  ("1", "0", "0", "0", "1"), [mc.OUTFLOW] * 6))
+    (d / "artracfd.geo").write_text(mc.moving_geo_text(spheres=[
+        dict(O=(-0.02, 0.01, 0.0), r=r, V=(3.0, 1.0, 0.5), rho=50.0, mid=2)]))
+    case = Case(str(d))
+    solver = Solver(case)
+    before = case.interior(case.flags()).copy()
+    print(m, r, flush=True)
+    done, _ = solver.march(steps)
+    flags, O = case.interior(case.flags()), case.bodies()[0, :3]
+    assert done == steps and np.isfinite(case.interior(solver.field())).all()
+    x = [-0.5 + (np.arange(*case.pin[s]) - (case.n[s] - m - 1) // 2) / m - O[s] for s in range(3)]
+    d2 = x[2][:, None, None] ** 2 + x[1][None, :, None] ** 2 + x[0][None, None, :] ** 2
+    inside = flags[0] == 1
+    assert (inside == (d2 <= r * r))[np.abs(d2 - r * r) > 1e-12].all()
+    near = np.zeros_like(inside)
+    for axis in range(3):
+        for shift in (1, -1):
+            near |= np.roll(~inside, shift, axis)
+    assert np.array_equal(flags[2] == 1, inside & near)
+    assert np.array_equal(flags[3] == 1, inside & near)
+    if m == 64:
+        assert (flags != before).any(axis=0).sum() > 1024
+    solver.close()
+    case.close()
