@@ -2436,10 +2436,12 @@ __global__ void dt_batch(const BatchCase *cases, int C, const unsigned long long
     half[c] = 0.5 * h;
 }
 
-// Cell sizes and CFL number of a single-case device march.
+// Cell sizes, CFL number and the words that the speed maxima start from (the
+// body speeds' floors) of a single-case device march.
 struct StepGeometry {
     double d[3];
     double cfl;
+    unsigned long long floor[3];
 };
 
 // Time step of a single case on the device: step[0] = dt, step[1] = dt / 2
@@ -2451,7 +2453,9 @@ struct StepGeometry {
 // accumulated time reaches the interval, or the loop ends) clock[6] is set
 // and later steps leave the clock as it is, so that the host writes the
 // output of exactly that state.
-__global__ void dt_single(StepGeometry sg, const unsigned long long *vmax, double *clock, double *step, double *hist)
+// The maxima are left at their floors for the next step's reduction (a
+// launch less in every step: 3 us of 95 on 256 x 4 x 4 nodes).
+__global__ void dt_single(StepGeometry sg, unsigned long long *vmax, double *clock, double *step, double *hist)
 {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
     double h = 0.0;
@@ -2466,6 +2470,7 @@ __global__ void dt_single(StepGeometry sg, const unsigned long long *vmax, doubl
             if (due) clock[6] = 1.0;
         }
     }
+    for (int s = 0; s < 3; ++s) vmax[s] = sg.floor[s];
     step[0] = h;
     step[1] = 0.5 * h;
     hist[(int)step[2]] = h;
@@ -3386,18 +3391,31 @@ int UpdateLeanPolicy(ArtraDevice *dev)
     return 0;
 }
 
-// Per-axis speed maxima of level TO folded with the floors (body speeds),
-// into vmax on the device (solve.c:108-153).
-int EnqueueSpeeds(ArtraDevice *dev, const double floor[3], unsigned long long *vmax)
+// The words that speed maxima with the given floors (body speeds) start from.
+void SpeedFloors(const double floor[3], unsigned long long words[3])
 {
-    unsigned long long init[3];
     for (int s = 0; s < 3; ++s) {
         const double f = (floor[s] > 0.0) ? floor[s] : 0.0;
-        memcpy(init + s, &f, sizeof f);
+        memcpy(words + s, &f, sizeof f);
     }
+}
+
+// vmax on the device set to the floors.
+int EnqueueFloors(ArtraDevice *dev, const double floor[3], unsigned long long *vmax)
+{
+    unsigned long long init[3];
+    SpeedFloors(floor, init);
+    hipLaunchKernelGGL(init_speeds, dim3(1), dim3(1), 0, dev->stream, vmax, init[0], init[1], init[2]);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+// Per-axis speed maxima of level TO folded into vmax on the device
+// (solve.c:108-153).
+int EnqueueSpeeds(ArtraDevice *dev, unsigned long long *vmax)
+{
     int slot;
     if (Begin(dev, ARTRA_T_CFL, &slot)) return 1;
-    hipLaunchKernelGGL(init_speeds, dim3(1), dim3(1), 0, dev->stream, vmax, init[0], init[1], init[2]);
     const Grid &g = dev->g;
     const long total = (long)(g.hi[0] - g.lo[0]) * (g.hi[1] - g.lo[1]) * (g.hi[2] - g.lo[2]);
     long blocks = (total + 255) / 256;
@@ -3439,7 +3457,8 @@ int EnqueueStep(ArtraDevice *dev, const MarchScratch &ms, const double floor[3],
     StepGeometry sg;
     for (int s = 0; s < 3; ++s) sg.d[s] = dev->par.d[s];
     sg.cfl = cfl;
-    if (EnqueueSpeeds(dev, floor, ms.vmax)) return 1;
+    SpeedFloors(floor, sg.floor);
+    if (EnqueueSpeeds(dev, ms.vmax)) return 1;
     hipLaunchKernelGGL(dt_single, dim3(1), dim3(1), 0, dev->stream, sg, ms.vmax, ms.clock, ms.step, ms.hist);
     if (hipGetLastError() != hipSuccess) return Fail("dt_single launch failed");
     return artra_dev_evolve(dev, 0.0);
@@ -3505,6 +3524,7 @@ int MarchSteps(ArtraDevice *dev, const MarchScratch &ms, double clock[kMarchCloc
     memcpy(head, clock, kMarchClock * sizeof(double));
     head[kMarchClock] = head[kMarchClock + 1] = head[kMarchClock + 2] = 0.0;
     HIP_TRY(hipMemcpyAsync(ms.clock, head, sizeof head, hipMemcpyHostToDevice, dev->stream));
+    if (EnqueueFloors(dev, floor, ms.vmax)) return 1;
     hipGraphExec_t graph = nullptr;
     // nothing reads the fill between fused steps: one behind the last
     dev->deferFill = AllFused(dev);
@@ -3888,7 +3908,7 @@ int artra_dev_treat_immersed(ArtraDevice *dev, int level)
 
 int artra_dev_max_speed(ArtraDevice *dev, const double floor[3], double vmax[3])
 {
-    if (EnqueueSpeeds(dev, floor, dev->vmax)) return 1;
+    if (EnqueueFloors(dev, floor, dev->vmax) || EnqueueSpeeds(dev, dev->vmax)) return 1;
     unsigned long long host[3];
     HIP_TRY(hipMemcpyAsync(host, dev->vmax, sizeof host, hipMemcpyDeviceToHost, dev->stream));
     HIP_TRY(hipStreamSynchronize(dev->stream));
