@@ -1165,8 +1165,8 @@ __device__ __forceinline__ void RoutedLine(const LineArgs &la, const FluxModel &
 
 // Plain lines, as many per block as its threads hold: `perLine` threads a
 // line, one per face up to 256 faces (K = 1), two faces each beyond (K = 2).
-// Bound by FP64 vector issue (534 of 675 vector instructions a stage and
-// node; 75-80 % of the issue cycles are taken at three wavefronts per SIMD).
+// Bound by FP64 vector issue (535 of 600-626 vector instructions a stage and
+// node; 78-85 % of the issue cycles are taken at three wavefronts per SIMD).
 // At 256^3 an operator takes 1.17 ms along y, 1.14 along z, the two along x
 // in one launch 2.12 (one line to a block of whole wavefronts, component by
 // component loads, a launch per operator: 1.28, 1.25, 1.23 each with the same

@@ -20,7 +20,7 @@ Prints one JSON line.  The roofline object is for the dominant kernel family
 timed region.  Algorithmic bytes per cell-stage are those of a stage-by-stage
 sweep (80 B for the first RK3 stage: read U_tn, write U_tm; 120 B for the
 other two, which also read U_to; 106.7 B on average); a fused launch covers
-three cell-stages per cell.
+three cell-stages per cell, or six where two like operators share it.
 """
 import argparse
 import json
@@ -40,8 +40,8 @@ FP64_PEAK_TFLOPS = 78.6
 # WRITE_SIZE, scale factors from a 1 GiB copy kernel) and FP64 flops per
 # cell-stage of the plain WENO5 flux and update (FMA = 2, from the FP64
 # instruction counters).
-TRAFFIC_B_PER_CELL_STAGE = 25.9
-FP64_FLOP_PER_CELL_STAGE = 914.0
+TRAFFIC_B_PER_CELL_STAGE = 22.4
+FP64_FLOP_PER_CELL_STAGE = 812.0
 # the stage-by-stage sweeps (profiles/sweep_shockvortex256.md)
 UNFUSED_TRAFFIC_B_PER_CELL_STAGE = 112.3
 METRIC = "Mcell-stage updates/s (256³ WENO5-RK3) + learned-hybrid vs plain at ≤1e-3 L1"
@@ -159,12 +159,12 @@ def reference_rate(name, steps):
 # (case, timed steps, CPU sample case, CPU sample steps, dominant kernel family,
 # measured HBM bytes per cell-stage of its sweeps, profiles/sweep_tgv128_cylinder.md)
 SIDE_WORKLOADS = (
-    ("tgv128", 20, "tgv64", 4, "sweep_tile with the viscous flux (stage-by-stage sweeps)", 176.6),
+    ("tgv128", 20, "tgv64", 4, "sweep_tile with the viscous flux (stage-by-stage sweeps)", 120.1),
     ("cylinder", 40, "cyl64", 100, "sweep_tile with the immersed-boundary fill (stage-by-stage sweeps)",
-     126.0),
+     125.5),
     ("cylinder_moving", 40, "cyl64_moving", 10,
      "sweep_tile with the immersed-boundary fill; solid half-steps (surface force, kinematics, motion, "
-     "reclassification, ghost tables) between the fluid steps", 126.0),
+     "reclassification, ghost tables) between the fluid steps", 125.5),
 )
 
 
@@ -413,7 +413,7 @@ def main():
         "data": "synthetic",
         "config": {"workload": describe(case_dir, args.case, cells), "parallelism": "single GPU",
                    "fused_axes": fused_axes},
-        "roofline": {"bound": "hbm", "limiter": "FP64 vector issue (fp64 below); HBM traffic is a quarter of the "
+        "roofline": {"bound": "hbm", "limiter": "FP64 vector issue (fp64 below); HBM traffic is a fifth of the "
                                                 "algorithmic bytes", "achieved": round(achieved, 2),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
