@@ -1360,6 +1360,9 @@ struct BatchTile {
     long first;                     // first line of the tile
 };
 
+// A block per plain tile: blocks that walk the list in strides leave their
+// last round uneven (four for each CU where three fit: 16 cases of 32 to 128
+// nodes a side took 60.5 ms for ten steps, 55.2 with a block per tile).
 template <int S, int K>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rk_batch(const BatchTile *tiles,
                                                                                          int ntiles,
@@ -1367,16 +1370,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
                                                                                          FluxModel mdl, const double *first)
 {
     extern __shared__ double lds[];
+    if (blockIdx.x >= ntiles) return;
     const bool memory = first && *first == 1.0;     // the march's first operator: ghosts as memory holds them
-    for (long w = blockIdx.x; w < ntiles; w += gridDim.x) {
-        const BatchTile bt = tiles[w];
-        const LineArgs &la = args[bt.c];
-        const int slot = threadIdx.x / bt.T, tt = threadIdx.x - slot * bt.T;
-        const bool active = slot < bt.count;
-        char *mem = (char *)lds + (size_t)slot * LineLdsBytes(la.n, la.hi - la.lo + 1, false);
-        PlainLine<S, 6, true, K>(la, mdl, active ? bt.first + slot : 0, tt, bt.T, mem, active, memory);
-        __syncthreads();
-    }
+    const BatchTile bt = tiles[blockIdx.x];
+    const LineArgs &la = args[bt.c];
+    const int slot = threadIdx.x / bt.T, tt = threadIdx.x - slot * bt.T;
+    const bool active = slot < bt.count;
+    char *mem = (char *)lds + (size_t)slot * LineLdsBytes(la.n, la.hi - la.lo + 1, false);
+    PlainLine<S, 6, true, K>(la, mdl, active ? bt.first + slot : 0, tt, bt.T, mem, active, memory);
 }
 
 template <int S>
@@ -4347,7 +4348,8 @@ int BatchBuildTiles(ArtraBatch *b, int p)
 template <int S>
 void BatchLaunchAxis(ArtraBatch *b, bool first, hipStream_t st)
 {
-    const dim3 grid((unsigned)std::max(1, std::min(b->grid, b->ntiles[S]))), block(256);
+    const int blocks = b->hybrid ? std::min(b->grid, b->ntiles[S]) : b->ntiles[S];
+    const dim3 grid((unsigned)std::max(1, blocks)), block(256);
     const FluxModel mdl = b->cases[0]->mdl;
     const double *step = first ? b->stepNo : nullptr;
     if (b->hybrid) {
@@ -4764,7 +4766,7 @@ int artra_dev_batch_tune(ArtraBatch *b, int reps, int *threads_out, int *grid_ou
         if (BatchBuildTiles(b, p)) return 1;
     double bestG = 1e300;
     int grid = b->grid;
-    for (int m = 2; m <= 8; m *= 2) {
+    for (int m = 2; b->hybrid && m <= 8; m *= 2) {  // (plain tiles: a block each)
         b->grid = m * b->cus;
         HIP_TRY(hipEventRecord(e0, b->stream));
         for (int r = 0; r < reps; ++r)
