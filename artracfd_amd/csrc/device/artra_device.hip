@@ -821,17 +821,30 @@ __device__ __forceinline__ bool FromMemory(const LineArgs &la)
     return la.memoryGhosts == 1 || (la.memoryGhosts == 2 && *la.steps == 1.0);
 }
 
-// The ghost node g of 2 half (low end, then high end) of a line: its
-// position, and in U its state by the line's rules or as memory holds it;
-// false where neither gives one (a wall's, which WallGhosts makes).
-__device__ __forceinline__ bool GhostNode(const LineArgs &la, long base, int g, int half, bool memory, int &pos, double U[5])
+// The position of ghost node g of 2 half (low end, then high end) of a line.
+__device__ __forceinline__ int GhostPosition(const LineArgs &la, int g, int half)
 {
-    pos = (g < half) ? la.lo - half + g : la.hi + g - half;
-    int src = memory ? pos : -3;
+    return (g < half) ? la.lo - half + g : la.hi + g - half;
+}
+
+// What the rules make of the node at pos: `none` where they say nothing.
+__device__ __forceinline__ int RuleSource(const LineArgs &la, int pos, int none)
+{
+    int src = none;
 #pragma unroll
     for (int e = 0; e < kLineRules; ++e) {
-        if (!memory && e < la.nrules && la.rdst[e] == pos) src = la.rsrc[e];
+        if (e < la.nrules && la.rdst[e] == pos) src = la.rsrc[e];
     }
+    return src;
+}
+
+// The ghost node g: its position, and in U its state by the line's rules or
+// as memory holds it; false where neither gives one (a wall's, which
+// WallGhosts makes).
+__device__ __forceinline__ bool GhostNode(const LineArgs &la, long base, int g, int half, bool memory, int &pos, double U[5])
+{
+    pos = GhostPosition(la, g, half);
+    const int src = memory ? pos : RuleSource(la, pos, -3);
     if (src >= 0) {
         LoadNode(la.U, base + (long)src * la.stride, U);
     } else {
@@ -839,6 +852,20 @@ __device__ __forceinline__ bool GhostNode(const LineArgs &la, long base, int g, 
         for (int c = 0; c < 5; ++c) U[c] = (src == -1) ? la.state[0][c] : la.state[1][c];
     }
     return src > -3;
+}
+
+// The prescribed states into their ghosts, for a line that started from the
+// ghosts in memory: the fill behind its first stage, which Refill (copies)
+// and WallGhosts (walls) leave to this.  Nothing changes them afterwards.
+// Between the first stage's fluxes and the barrier that ends its update.
+__device__ __forceinline__ void PrescribedGhosts(const LineArgs &la, int half, double *st, int tt, int T)
+{
+    for (int g = tt; g < 2 * half; g += T) {
+        const int pos = GhostPosition(la, g, half), src = RuleSource(la, pos, 0);
+        if (src >= 0) continue;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) st[pos * 5 + c] = (src == -1) ? la.state[0][c] : la.state[1][c];
+    }
 }
 
 // A line into LDS by its T threads, one interior node each with K = 1 and
@@ -977,7 +1004,6 @@ __device__ __forceinline__ void PlainLine(const LineArgs &la, const FluxModel &m
             if (active) WallGhosts<S>(la, SL + 1, st, tt, T);
             __syncthreads();
         }
-        memory = false;
         double FL[5];
 #pragma nounroll
         for (int k = 0; k < K; ++k) {
@@ -1029,6 +1055,8 @@ __device__ __forceinline__ void PlainLine(const LineArgs &la, const FluxModel &m
             Refill(la, i, v, st);
         }
         if (todo == 1) return;
+        if (memory && active) PrescribedGhosts(la, SL + 1, st, tt, T);
+        memory = false;
         __syncthreads();
         s = (s + 1 == la.stages) ? 0 : s + 1;
     }
@@ -1159,6 +1187,7 @@ __device__ __forceinline__ void RoutedLine(const LineArgs &la, const FluxModel &
             for (int c = 0; c < 5; ++c) st[i * 5 + c] = v[c];
             Refill(la, i, v, st);
         }
+        if (memory && s == 0) PrescribedGhosts(la, 3, st, tt, T);
         if (s + 1 < la.stages) __syncthreads();
     }
 }
@@ -1234,7 +1263,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 
     artra::MlpWave frags;
     artra::mlp_wave_fragments(hy.W1, hy.W2, frags);
     for (int e = tt; e < 3 * artra::kHidden; e += T) bias[e] = hy.bias[e];
-    LoadRoutedLine<1>(la, base, tt, T, FromMemory(la), mdl.gamma, st, nodeRP);
+    const bool memory = FromMemory(la);
+    LoadRoutedLine<1>(la, base, tt, T, memory, mdl.gamma, st, nodeRP);
     const int i = la.lo + tt;                       // this thread's node
     const bool own = i < la.hi;
     if (tt == 0) troubledAny = 0;
@@ -1297,6 +1327,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 
                 Refill(la, i, v, st);
             }
         }
+        if (memory && s == 0) PrescribedGhosts(la, 3, st, tt, T);
         if (s + 1 < la.stages) __syncthreads();
     }
 }

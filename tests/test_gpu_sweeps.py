@@ -8,6 +8,7 @@ import sys
 import numpy as np
 import pytest
 
+import mlp_oracle as M
 from conftest import ROOT
 
 sys.path.insert(0, os.path.join(ROOT, "cases"))
@@ -119,6 +120,113 @@ def test_a_step_on_lines_starts_from_the_ghosts_of_its_input(tmp_path, bcs):
         solver.close()
         case.close()
     assert np.array_equal(out[0], out[1])
+
+
+IN_LOW, IN_HIGH = mc.inflow(1.1, 0.1, 0.2, 0.4, 1.2), mc.inflow(0.9, -0.2, 0.1, -0.3, 0.8)
+INFLOWS = {"low": [mc.OUTFLOW] * 4 + [IN_LOW, mc.OUTFLOW], "high": [mc.OUTFLOW] * 4 + [mc.OUTFLOW, IN_HIGH],
+           "both": [mc.OUTFLOW, IN_HIGH, IN_LOW, IN_HIGH, IN_LOW, IN_HIGH],
+           "wall": [IN_LOW, mc.slip(), IN_LOW, mc.noslip(), IN_LOW, mc.noslip(0.0033)],
+           "x": [IN_LOW, mc.OUTFLOW] + [mc.OUTFLOW] * 4, "y": [mc.OUTFLOW] * 2 + [mc.OUTFLOW, IN_HIGH] + [mc.OUTFLOW] * 2}
+
+
+def with_ghosts_of_its_own(solver, scale=1e-3):
+    """Every node's state changed, the ghosts' too: they no longer are what a
+    boundary fill makes of the interior."""
+    U = solver.field()
+    solver.set_field(0, U * (1.0 + scale * np.cos(np.arange(U.size)).reshape(U.shape)))
+
+
+def run_once(directory, steps, start=with_ghosts_of_its_own, params=None, threshold=0.0, gate=0.0, **options):
+    """Interior after evolve() (steps 0) or a march, from the field `start` makes."""
+    from artracfd_amd import Case, Solver
+    case = Case(directory)
+    solver = Solver(case, **options)
+    if params is not None:
+        solver.set_indicator(params, threshold, smooth_variation=gate)
+    start(solver)
+    if steps:
+        assert solver.march(steps)[0] == steps
+    else:
+        solver.evolve(1e-4)
+    U = case.interior(solver.field()).copy()
+    solver.close()
+    case.close()
+    return U
+
+
+# the first operator runs along z in three dimensions, along y with z
+# collapsed, along the one axis of a tube (both operators in one launch)
+@pytest.mark.parametrize("m, kind", [((6, 5, 70), "low"), ((6, 5, 70), "high"), ((6, 5, 70), "both"),
+                                     ((5, 6, 40), "wall"), ((4, 4, 300), "both"), ((40, 30, 1), "y"),
+                                     ((40, 30, 1), "both"), ((70, 1, 1), "x"), ((1, 1, 70), "low"),
+                                     ((1, 70, 1), "y")])
+@pytest.mark.parametrize("steps", [0, 3])
+@pytest.mark.parametrize("numerical", [(1, 1, 0, 0, 0, 0, 1), (0, 0, 0, 1, 1, 0, 1)])
+def test_prescribed_states_are_back_after_the_first_stage(tmp_path, m, kind, steps, numerical):
+    """A call that starts from a caller's own ghosts reads them in its first
+    stage only: from then on an inflow end holds its prescribed state, on
+    lines as stage by stage."""
+    directory = write_case(tmp_path, m, INFLOWS[kind], numerical)
+    print(m, kind, steps, flush=True)
+    fused = run_once(directory, steps, exact=True)
+    assert np.array_equal(fused, run_once(directory, steps, exact=True, fused=False))
+
+
+@pytest.mark.parametrize("m, kind", [((4, 3, 70), "both"), ((3, 3, 300), "low"), ((70, 1, 1), "x")])
+@pytest.mark.parametrize("steps", [0, 3])
+def test_prescribed_states_on_routed_lines(tmp_path, m, kind, steps):
+    """The same with the indicator: every face on the full flux is the plain
+    solver bit for bit (lines deferred by the lean pass and, beyond 256
+    nodes, lines that never take it)."""
+    directory = write_case(tmp_path, m, INFLOWS[kind])
+    print(m, kind, steps, flush=True)
+    plain = run_once(directory, steps)
+    assert np.array_equal(plain, run_once(directory, steps, params=M.init_params(3), threshold=-1e30))
+
+
+def test_prescribed_states_on_lean_lines(tmp_path):
+    """A smooth line stays in the lean pass; the same line with a jump at its
+    far end is deferred and routed.  Near the inflow both take the linear flux
+    and agree bit for bit, from ghosts of their own."""
+    directory = write_case(tmp_path, (1, 1, 200), INFLOWS["low"])
+    out = []
+    for jump in (0.0, 0.5):
+        def start(solver):
+            U = np.ones_like(solver.field()) * np.array([1.1, 0.11, 0.22, 0.44, 3.2])[:, None, None, None]
+            U *= 1.0 + 2e-4 * np.cos(np.arange(U.size)).reshape(U.shape)
+            U[:, 160:] *= 1.0 + jump
+            solver.set_field(0, U)
+        print("jump", jump, flush=True)
+        out.append(run_once(directory, 0, start, params=M.init_params(3), threshold=-1e30, gate=1e-2)[:, :60])
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("routed", [False, True])
+def test_batched_lines_start_from_the_ghosts_of_their_input(tmp_path, routed):
+    """A batch started from ghosts of its own gives what its cases give alone."""
+    from artracfd_amd import Case, Solver
+    from artracfd_amd.batch import Batch
+    dirs = []
+    for q, (m, kind) in enumerate([((5, 4, 70), "both"), ((12, 11, 40), "low"), ((6, 5, 256), "high")]):
+        (tmp_path / str(q)).mkdir()
+        dirs.append(write_case(tmp_path / str(q), m, INFLOWS[kind]))
+    cases = [Case(d) for d in dirs]
+    solvers = [Solver(c) for c in cases]
+    for s in solvers:
+        with_ghosts_of_its_own(s)
+    print("batch", routed, flush=True)
+    b = Batch(solvers)
+    if routed:
+        b.set_indicator(M.init_params(3), -1e30)
+    b.march(3)
+    got = [c.interior(s.field()).copy() for c, s in zip(cases, solvers)]
+    b.close()
+    for s, c in zip(solvers, cases):
+        s.close()
+        c.close()
+    alone = dict(params=M.init_params(3), threshold=-1e30, gate=1e-3) if routed else {}
+    for q, d in enumerate(dirs):
+        assert np.array_equal(got[q], run_once(d, 3, **alone)), q
 
 
 def test_batched_lines_at_the_edges_of_their_blocks(tmp_path):
