@@ -29,6 +29,7 @@
 
 #include "flux.hpp"
 #include "indicator.hpp"
+#include "tiles.hpp"
 
 extern "C" {
 #include "artra_device.h"
@@ -36,6 +37,13 @@ extern "C" {
 #include "geomcore.h"
 
 using artra::FluxModel;
+using artra::kTileIn;
+using artra::kTileOut;
+using artra::kTileThreads;
+using artra::SweepTile;
+using artra::TileDoubles;
+using artra::TileOffset;
+using artra::TileSpare;
 
 namespace {
 
@@ -185,32 +193,6 @@ __device__ __forceinline__ long XcdLine(long b, long nb)
 // of 32 nodes per thread in a register window (y, z): those asked the L1 for
 // 30 to 70 strided 8-byte loads per face, and the marches left small grids
 // with a few hundred blocks.
-struct SweepTile {
-    int P;                          // lines per tile
-    int seg, nseg;                  // nodes per segment, segments per line
-    int groups, others;             // tiles across the line axis, extent of the third axis
-    int rows;                       // nodes per line in LDS: seg + 2 halo
-    int perPass;                    // x: threads per line; y and z: rows of the tile the block copies at a time
-    int threads;                    // of a block
-    int tiles;
-};
-
-constexpr int kTileThreads = 256;
-constexpr int kTileIn = 11, kTileOut = 6;            // doubles per thread of a tile's states and of its a-term
-
-// Doubles of LDS: node states, face fluxes, with the viscous flux the
-// transverse differences of every node a face touches and then, in their
-// place, the viscous fluxes, and the a-term's states.
-__host__ __device__ __forceinline__ int TileSpare(int P, int seg, bool visc)
-{
-    const int faces = P * (seg + 1), differences = (faces + P) * 4;
-    return !visc ? 0 : (differences > 5 * faces) ? differences : 5 * faces;
-}
-
-__host__ __device__ __forceinline__ size_t TileDoubles(int P, int seg, int rows, bool visc)
-{
-    return (size_t)5 * P * (rows + (seg + 1) + seg) + TileSpare(P, seg, visc);
-}
 
 // The transverse differences of node idx (see viscous_flux): components S
 // and the tangential one along each tangential axis.
@@ -299,7 +281,7 @@ __device__ __forceinline__ void TileFetch(const Grid &g, const double *U, const 
 {
     const int stride = (S == 2) ? g.nx * g.ny : g.nx;                        // between rows
     const double *base = U + ((long)t.first - (long)before * ((S == 0) ? 1 : stride)) * 5;
-    const unsigned at = (unsigned)(h.row * stride * 5 + h.col) * 8u;
+    const unsigned at = TileOffset(h.row, stride, h.col);
     const long step = (S == 0) ? h.perPass : (long)h.perPass * stride * 5;
     const bool on = h.on && ((S == 0) ? h.row < t.lines : h.col < 5 * t.lines);
     const int end = (S == 0) ? 5 * n - h.col : n - h.row;
@@ -431,7 +413,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(FA
     const double *v = vb + ((S == 0) ? h.row * F * 5 : 0) + shareAt;
     const double *u = vb + TileSpare(P, ts.seg, VISC) + ((S == 0) ? h.row * ts.seg * 5 : 0) + shareAt;
     const double *un = st + ((S == 0) ? (h.row * rows + halo) * 5 : halo * 5 * P) + shareAt;
-    const unsigned at = (unsigned)(h.row * rowStride * 5 + h.col) * 8u;
+    const unsigned at = TileOffset(h.row, rowStride, h.col);
     double *base = sa.Utm + (size_t)t.first * 5;
     const long pass = (S == 0) ? h.perPass : (long)h.perPass * rowStride * 5;
 #pragma unroll
@@ -2726,66 +2708,17 @@ int Harvest(ArtraDevice *dev)
     return 0;
 }
 
-// Tile of a stage sweep along s: of the shapes that fit a block of at most
-// kTileThreads, the one whose blocks cost least in all.  A wavefront's faces
-// cost about 650 issue slots, an element copied in or out 8 or 20 per
-// wavefront (instruction counts of the kernel), a cache line moved about 6;
-// idle lanes of a partly filled wavefront, the halo of a short segment and
-// the broken cache lines of a narrow tile show in these counts.
-SweepTile TileOf(const Grid &g, int s, int halo, bool visc, int longest)
-{
-    SweepTile best{};
-    double bestCost = 0.0;
-    const int line = (s == 0) ? 1 : 0, third = (s == 2) ? 1 : 2;
-    const int es = g.hi[s] - g.lo[s], across = g.hi[line] - g.lo[line], others = g.hi[third] - g.lo[third];
-    const int extra = visc ? 2 : 1;                  // threads per line beyond its nodes
-    for (int P = 1; P <= across && P <= kTileThreads / 2; ++P) {
-        int seg = std::min(es, kTileThreads / P - extra);
-        if (seg < 1) break;
-        if (s > 0 && longest > 0) seg = std::min(seg, longest);
-        const int nseg = (es + seg - 1) / seg;
-        seg = (es + nseg - 1) / nseg;
-        const int rows = seg + 2 * halo;
-        // x: enough threads per line for its faces and for kTileIn elements each
-        const int perLine = (s == 0) ? std::max(seg + extra, (5 * rows + kTileIn - 1) / kTileIn) : seg + extra;
-        const int faceWaves = (P * perLine + 63) / 64;
-        if (TileDoubles(P, seg, rows, visc) * sizeof(double) > 48 * 1024) continue;
-        for (int waves = faceWaves; 64 * waves <= kTileThreads; ++waves) {
-            // y and z: rows of 5 P doubles per pass of the block
-            if (s == 0 && waves > faceWaves) break;
-            const int perPass = (s == 0) ? perLine : 64 * waves / (5 * P);
-            if (perPass < 1) continue;
-            const int in = (((s == 0) ? 5 * rows : rows) + perPass - 1) / perPass;
-            const int out = (((s == 0) ? 5 * seg : seg) + perPass - 1) / perPass;
-            if (in > kTileIn || out > kTileOut) continue;
-            const double cacheLines = (s == 0) ? P * ((rows + 2 * seg) * 40.0 / 128.0 + 2.25)
-                                               : (rows + 2 * seg) * (P * 40.0 / 128.0 + 0.75);
-            const double tiles = (double)((across + P - 1) / P) * others * nseg;
-            const double cost = tiles * (650.0 * faceWaves + waves * (8.0 * in + 20.0 * out) + 6.0 * cacheLines);
-            if (best.P && cost >= bestCost) continue;
-            best.P = P;
-            best.seg = seg;
-            best.nseg = nseg;
-            best.groups = (across + P - 1) / P;
-            best.others = others;
-            best.rows = rows;
-            best.perPass = perPass;
-            best.threads = 64 * waves;
-            best.tiles = best.groups * others * nseg;
-            bestCost = cost;
-        }
-    }
-    return best;
-}
-
 template <int NS, bool VISC, bool FAST>
 void LaunchSweep(ArtraDevice *dev, int s, const StageArgs &sa)
 {
     const Grid &g = dev->g;
+    int interior[3];
     for (int q = 0; q < 3; ++q) {
-        if (g.hi[q] <= g.lo[q]) return;
+        interior[q] = g.hi[q] - g.lo[q];
+        if (interior[q] <= 0) return;
     }
-    const SweepTile ts = TileOf(g, s, NS / 2, VISC, dev->segment);
+    const int n[3] = {g.nx, g.ny, g.nz};
+    const SweepTile ts = artra::TileOf(n, interior, s, NS / 2, VISC, dev->segment);
     const size_t lds = TileDoubles(ts.P, ts.seg, ts.rows, VISC) * sizeof(double);
     const dim3 grid((unsigned)ts.tiles), block(ts.threads);
     if (s == 0) hipLaunchKernelGGL((sweep_tile<0, NS, VISC, FAST>), grid, block, lds, dev->stream, g, sa, dev->mdl, ts);

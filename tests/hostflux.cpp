@@ -3,8 +3,10 @@
 // Compiled by tests/test_flux_host.py with hipcc's host pass only: the
 // __host__ __device__ functions of flux.hpp and indicator.hpp run on the CPU,
 // so the closed-form and characteristic linear fluxes of the learned hybrid
-// and the fast WENO5 flux can be checked against the CPU oracle without a GPU.
+// and the fast WENO5 flux can be checked against the CPU oracle without a GPU;
+// likewise the tile shapes and offsets of the stage sweeps (tiles.hpp).
 #include "indicator.hpp"
+#include "tiles.hpp"
 
 namespace {
 
@@ -67,6 +69,20 @@ void host_weno_flux(int s, int roe, int sw, const double *st, double *F)
     if (s == 0) Weno<0>(roe, sw, w, F);
     else if (s == 1) Weno<1>(roe, sw, w, F);
     else Weno<2>(roe, sw, w, F);
+}
+
+// The tile of a stage sweep: P, seg, nseg, groups, others, rows, perPass,
+// threads, tiles.
+void host_tile(const int *n, const int *interior, int s, int halo, int visc, int longest, int *out)
+{
+    const artra::SweepTile t = artra::TileOf(n, interior, s, halo, visc != 0, longest);
+    const int v[9] = {t.P, t.seg, t.nseg, t.groups, t.others, t.rows, t.perPass, t.threads, t.tiles};
+    for (int q = 0; q < 9; ++q) out[q] = v[q];
+}
+
+unsigned host_tile_offset(int row, int stride, int col)
+{
+    return artra::TileOffset(row, stride, col);
 }
 
 }  // extern "C"

@@ -16,6 +16,9 @@ what the mathematics fixes:
   lambda* (U+ - U-) / 2, equals its characteristic form on any stencil;
 * the fast-arithmetic WENO5 flux of the plain sweeps agrees with the
   oracle's to round-off on random stencils.
+
+The tile shapes of the stage sweeps are checked there too: what a block's
+threads hold, and the kernel's 32-bit byte offsets against the exact ones.
 """
 import ctypes
 import os
@@ -147,3 +150,35 @@ def test_linear_flux_differs_from_weno5_where_the_data_are_not_smooth(hostflux, 
     ref = _face_flux(oracle_mod, list(st), 0, 1, 0, 0)
     F = linear_flux(hostflux, st, 0, 0, 0, 1)
     assert np.abs(F - ref).max() > 1e-3 * np.abs(ref).max()
+
+
+# grids of up to INT_MAX nodes: wide planes, planes of one line, long lines
+TILES = [(3450, 3450, 36), (4650, 4650, 22), (5200, 5200, 17), (12000, 12000, 2), (1, 400000, 20), (2, 3000000, 9),
+         (3, 9000, 9000), (20000000, 2, 1), (3000000, 5, 4), (1024, 1024, 1024), (96, 96, 96), (1, 1, 1)]
+
+
+@pytest.mark.parametrize("interior", TILES)
+@pytest.mark.parametrize("halo", [2, 3])
+@pytest.mark.parametrize("visc", [0, 1])
+def test_tiles_fit_their_blocks_and_their_offsets(hostflux, interior, halo, visc):
+    n = [v + 2 * halo for v in interior]
+    assert n[0] * n[1] * n[2] < 2 ** 31
+    hostflux.host_tile_offset.restype = ctypes.c_uint
+    for s in range(3):
+        out = (ctypes.c_int * 9)()
+        hostflux.host_tile((ctypes.c_int * 3)(*n), (ctypes.c_int * 3)(*interior), s, halo, visc, 0, out)
+        P, seg, nseg, groups, others, rows, per, threads, tiles = list(out)
+        across, third = interior[1 if s == 0 else 0], interior[1 if s == 2 else 2]
+        # every node is swept, every face of a segment has a thread
+        assert P >= 1 and seg * nseg >= interior[s] and P * groups >= across and others == third
+        assert tiles == nseg * groups * others and rows == seg + 2 * halo
+        assert threads <= 256 and P * (seg + 1 + visc) <= threads
+        # the doubles that a thread holds: 11 of the states, 6 of the level they are added to
+        assert (5 * rows if s == 0 else rows) <= 11 * per and (5 * seg if s == 0 else seg) <= 6 * per
+        assert (P if s == 0 else 5 * P) * per <= threads
+        # byte offsets of a pass's rows (x: of the tile's lines)
+        stride = n[0] * n[1] if s == 2 else n[0]
+        for row in {0, 1, (P if s == 0 else per) - 1}:
+            for col in (0, (per if s == 0 else 5 * P) - 1):
+                if row < (P if s == 0 else per):
+                    assert hostflux.host_tile_offset(row, stride, col) == (row * stride * 5 + col) * 8
