@@ -670,7 +670,8 @@ __global__ __launch_bounds__(256) void bc_gather(GatherArgs ga, const int *__res
 // them; only the first operator of a call takes its ghosts from memory, as
 // the caller left them.  Two operators along the same axis in a row (x, x in
 // the middle of the three-dimensional step) run in one launch.
-constexpr int kLineRules = 12;
+constexpr int kLineGhosts = 6;      // of a line, at most: half a stencil at either end
+constexpr int kWallGhost = -3;      // the source of a ghost that a wall mirrors
 // The face tallies of the indicator are spread over slots on separate
 // 128-byte lines (block b adds into slot b mod kCountSlots): one counter
 // pair taking an atomic from every block serialises tens of thousands of
@@ -697,10 +698,10 @@ struct LineArgs {
     double gamma, gasR;
     int memoryGhosts;               // the ghosts the line starts from: 0 by the rules, 1 as memory holds them, 2 as
     const double *steps;            // memory holds them in the first step of a march (*steps == 1)
-    int nrules;
-    int rdst[kLineRules], rsrc[kLineRules];   // src >= 0: line position, src < 0: constant state -1 - src
-    int reach;                      // the copied nodes are among the first or last `reach` of the interior
-    double state[2][5];             // conservative states of constant (inflow) rules
+    int src[kLineGhosts];           // per ghost, by position: the line position it copies, -1 - k for state k, or
+                                    // kWallGhost
+    unsigned prescribed;            // bit g: ghost g holds a state; bit 8 + g: it is state 1
+    const double *state;            // [2][5]: conservative states of prescribed (inflow) ends
     int wall[2];                    // low and high end: 0, or the wall type (2 slip, 3 no-slip) that mirrors there
     double wallT[2];                // its temperature (negative: adiabatic)
 };
@@ -809,13 +810,13 @@ __device__ __forceinline__ int GhostPosition(const LineArgs &la, int g, int half
     return (g < half) ? la.lo - half + g : la.hi + g - half;
 }
 
-// What the rules make of the node at pos: `none` where they say nothing.
-__device__ __forceinline__ int RuleSource(const LineArgs &la, int pos, int none)
+// The source of ghost g.
+__device__ __forceinline__ int GhostSource(const LineArgs &la, int g)
 {
-    int src = none;
+    int src = la.src[0];
 #pragma unroll
-    for (int e = 0; e < kLineRules; ++e) {
-        if (e < la.nrules && la.rdst[e] == pos) src = la.rsrc[e];
+    for (int e = 1; e < kLineGhosts; ++e) {
+        if (g == e) src = la.src[e];
     }
     return src;
 }
@@ -826,27 +827,25 @@ __device__ __forceinline__ int RuleSource(const LineArgs &la, int pos, int none)
 __device__ __forceinline__ bool GhostNode(const LineArgs &la, long base, int g, int half, bool memory, int &pos, double U[5])
 {
     pos = GhostPosition(la, g, half);
-    const int src = memory ? pos : RuleSource(la, pos, -3);
-    if (src >= 0) {
-        LoadNode(la.U, base + (long)src * la.stride, U);
-    } else {
-#pragma unroll
-        for (int c = 0; c < 5; ++c) U[c] = (src == -1) ? la.state[0][c] : la.state[1][c];
-    }
-    return src > -3;
+    const int src = memory ? pos : GhostSource(la, g);
+    LoadNode((src >= 0) ? la.U : la.state, (src >= 0) ? base + (long)src * la.stride : -1 - max(src, -2), U);
+    return src > kWallGhost;
 }
 
 // The prescribed states into their ghosts, for a line that started from the
 // ghosts in memory: the fill behind its first stage, which Refill (copies)
 // and WallGhosts (walls) leave to this.  Nothing changes them afterwards.
 // Between the first stage's fluxes and the barrier that ends its update.
+// (The states are read from memory here: as launch arguments they would hold
+// twenty scalar registers through every stage, 1.5 % of a step on 256^3.)
 __device__ __forceinline__ void PrescribedGhosts(const LineArgs &la, int half, double *st, int tt, int T)
 {
     for (int g = tt; g < 2 * half; g += T) {
-        const int pos = GhostPosition(la, g, half), src = RuleSource(la, pos, 0);
-        if (src >= 0) continue;
+        if (!((la.prescribed >> g) & 1u)) continue;
+        double v[5], *d = st + GhostPosition(la, g, half) * 5;
+        LoadNode(la.state, (la.prescribed >> (8 + g)) & 1u, v);
 #pragma unroll
-        for (int c = 0; c < 5; ++c) st[pos * 5 + c] = (src == -1) ? la.state[0][c] : la.state[1][c];
+        for (int c = 0; c < 5; ++c) d[c] = v[c];
     }
 }
 
@@ -877,15 +876,27 @@ __device__ __forceinline__ void LoadLine(const LineArgs &la, long base, int tt, 
     }
 }
 
-// The ghosts that copy interior node i, refilled with its new state v.
-__device__ __forceinline__ void Refill(const LineArgs &la, int i, const double v[5], double *st)
+// The ghosts that copy node i, a bit each, found once per line (looked for
+// in every stage they cost 5 % of a step on 20^3 nodes, 1 % on 200^3, both
+// in exact arithmetic).
+__device__ __forceinline__ unsigned FeedsOf(const LineArgs &la, int i)
 {
-    if (i - la.lo >= la.reach && la.hi - 1 - i >= la.reach) return;
+    unsigned feeds = 0;
 #pragma unroll
-    for (int e = 0; e < kLineRules; ++e) {
-        if (e >= la.nrules || la.rsrc[e] != i) continue;
+    for (int g = 0; g < kLineGhosts; ++g) feeds |= (unsigned)(la.src[g] == i) << g;
+    return feeds;
+}
+
+// The ghosts that a node feeds, refilled with its new state v.
+__device__ __forceinline__ void Refill(const LineArgs &la, int half, unsigned feeds, const double v[5], double *st)
+{
+    if (!feeds) return;
 #pragma unroll
-        for (int c = 0; c < 5; ++c) st[la.rdst[e] * 5 + c] = v[c];
+    for (int g = 0; g < kLineGhosts; ++g) {
+        if (!((feeds >> g) & 1u)) continue;
+        double *d = st + GhostPosition(la, g, half) * 5;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) d[c] = v[c];
     }
 }
 
@@ -978,6 +989,9 @@ __device__ __forceinline__ void PlainLine(const LineArgs &la, const FluxModel &m
     const long base = LineBase(la, line);
     const bool walls = la.wall[0] || la.wall[1];
     const double r = Uniform(la.dt ? *la.dt * la.dd : la.r);
+    unsigned feeds[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) feeds[k] = FeedsOf(la, la.lo + tt + T * k);
     if (active) LoadLine<K>(la, base, tt, T, SL + 1, memory, st);
     if (la.dt && *la.dt == 0.0) return;             // past the march's end: the same for the whole block
     __syncthreads();
@@ -1034,7 +1048,7 @@ __device__ __forceinline__ void PlainLine(const LineArgs &la, const FluxModel &m
             }
 #pragma unroll
             for (int c = 0; c < 5; ++c) st[i * 5 + c] = v[c];
-            Refill(la, i, v, st);
+            Refill(la, SL + 1, feeds[k], v, st);
         }
         if (todo == 1) return;
         if (memory && active) PrescribedGhosts(la, SL + 1, st, tt, T);
@@ -1093,6 +1107,9 @@ __device__ __forceinline__ void RoutedLine(const LineArgs &la, const FluxModel &
     double *u0 = fb + 5 * F;                        // [F - 1][5]
     float *nodeRP = (float *)(work + LineWorkPlainBytes(F));   // [2][n]
     const long base = LineBase(la, line);
+    unsigned feeds[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) feeds[k] = FeedsOf(la, la.lo + tt + T * k);
     LoadRoutedLine<K>(la, base, tt, T, memory, mdl.gamma, st, nodeRP);
     __syncthreads();
     const int M = (F + T - 1) / T;
@@ -1167,7 +1184,7 @@ __device__ __forceinline__ void RoutedLine(const LineArgs &la, const FluxModel &
             }
 #pragma unroll
             for (int c = 0; c < 5; ++c) st[i * 5 + c] = v[c];
-            Refill(la, i, v, st);
+            Refill(la, 3, feeds[k], v, st);
         }
         if (memory && s == 0) PrescribedGhosts(la, 3, st, tt, T);
         if (s + 1 < la.stages) __syncthreads();
@@ -1249,6 +1266,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 
     LoadRoutedLine<1>(la, base, tt, T, memory, mdl.gamma, st, nodeRP);
     const int i = la.lo + tt;                       // this thread's node
     const bool own = i < la.hi;
+    const unsigned feeds = FeedsOf(la, i);
     if (tt == 0) troubledAny = 0;
     __syncthreads();
     // classification: the faces q = tt and q = tt + T (same trip count on
@@ -1306,7 +1324,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MEAN ? 6 : 
             } else {
 #pragma unroll
                 for (int c = 0; c < 5; ++c) st[i * 5 + c] = v[c];
-                Refill(la, i, v, st);
+                Refill(la, 3, feeds, v, st);
             }
         }
         if (memory && s == 0) PrescribedGhosts(la, 3, st, tt, T);
@@ -2644,12 +2662,11 @@ struct ArtraDevice {
     int allFluid = 0;               // every interior node is fluid
     struct LineRules {
         int ok = 0;
-        int count = 0;
-        int dst[kLineRules], src[kLineRules];
-        double state[2][5];
+        int src[kLineGhosts];       // as in LineArgs
         int wall[2];
         double wallT[2];
     } lines[3];
+    double *lineStates = nullptr;   // [3][2][5]: each axis's prescribed states
     int deferFill = 0;              // the steps being enqueued leave their last fill to the end of the march
     // timing
     bool timing = false;
@@ -3055,13 +3072,11 @@ LineArgs LineArgsOf(ArtraDevice *dev, int p)
     la.gamma = dev->par.gamma;
     la.gasR = dev->par.gasR;
     const ArtraDevice::LineRules &R = dev->lines[p];
-    la.nrules = R.count;
-    for (int e = 0; e < R.count; ++e) {
-        la.rdst[e] = R.dst[e];
-        la.rsrc[e] = R.src[e];
-        if (R.src[e] >= 0) la.reach = std::max(la.reach, 1 + std::min(R.src[e] - la.lo, la.hi - 1 - R.src[e]));
+    memcpy(la.src, R.src, sizeof la.src);
+    la.state = dev->lineStates + 10 * p;
+    for (int e = 0; e < kLineGhosts; ++e) {
+        if (R.src[e] == -1 || R.src[e] == -2) la.prescribed |= ((R.src[e] == -2) ? 0x101u : 1u) << e;
     }
-    memcpy(la.state, R.state, sizeof la.state);
     memcpy(la.wall, R.wall, sizeof la.wall);
     memcpy(la.wallT, R.wallT, sizeof la.wallT);
     return la;
@@ -3114,21 +3129,32 @@ int LineSweep(ArtraDevice *dev, double dt, int p, int operators, bool first)
     return End(dev, slot);
 }
 
+// The states of the faces that prescribe one, in the order of the rules of
+// axis p, which are complete with them.
+int SetLineStates(ArtraDevice *dev, int p, int count, const int faces[2])
+{
+    double state[2][5] = {};
+    for (int k = 0; k < count; ++k) Conservative(dev->par.gamma, dev->par.varBC[faces[k]], state[k]);
+    HIP_TRY(hipMemcpy(dev->lineStates + 10 * p, state, sizeof state, hipMemcpyHostToDevice));
+    dev->lines[p].ok = 1;
+    return 0;
+}
+
 // Per-line copy rules of the fill along axis p, read off the resolved gather
 // of the faces normal to p: every interior line must see the same rules
 // (destination position along the line <- source position on the same line,
 // or a constant state), covering every ghost the stencil reads.
-void DeriveLineRules(ArtraDevice *dev, int p, long entries, const int *dst, const int *srcs)
+int DeriveLineRules(ArtraDevice *dev, int p, long entries, const int *dst, const int *srcs)
 {
     const Grid &g = dev->g;
     const int ext[3] = {g.nx, g.ny, g.nz};
     const int half = (dev->par.sScheme == 1) ? 3 : 2;
     ArtraDevice::LineRules &R = dev->lines[p];
     R = ArtraDevice::LineRules{};
-    if (g.hi[p] - g.lo[p] <= 0) return;
+    if (g.hi[p] - g.lo[p] <= 0) return 0;
     const int t1 = (p == 0) ? 1 : 0, t2 = (p == 2) ? 1 : 2;
     const long n1 = g.hi[t1] - g.lo[t1], n2 = g.hi[t2] - g.lo[t2];
-    if (n1 <= 0 || n2 <= 0) return;
+    if (n1 <= 0 || n2 <= 0) return 0;
     std::vector<std::vector<std::pair<int, int>>> per((size_t)(n1 * n2));
     int faces[2] = {-1, -1}, nfaces = 0;
     for (long e = 0; e < entries; ++e) {
@@ -3138,7 +3164,7 @@ void DeriveLineRules(ArtraDevice *dev, int p, long entries, const int *dst, cons
         int src;
         if (q >= 0) {
             const int cq[3] = {q % g.nx, (q / g.nx) % g.ny, q / (g.nx * g.ny)};
-            if (cq[t1] != c[t1] || cq[t2] != c[t2] || cq[p] < g.lo[p] || cq[p] >= g.hi[p]) return;
+            if (cq[t1] != c[t1] || cq[t2] != c[t2] || cq[p] < g.lo[p] || cq[p] >= g.hi[p]) return 0;
             src = cq[p];
         } else {
             const int face = -3 - q;
@@ -3146,7 +3172,7 @@ void DeriveLineRules(ArtraDevice *dev, int p, long entries, const int *dst, cons
             for (int k = 0; k < nfaces; ++k)
                 if (faces[k] == face) slot = k;
             if (slot < 0) {
-                if (nfaces == 2) return;
+                if (nfaces == 2) return 0;
                 slot = nfaces;
                 faces[nfaces++] = face;
             }
@@ -3157,34 +3183,32 @@ void DeriveLineRules(ArtraDevice *dev, int p, long entries, const int *dst, cons
     for (auto &v : per) std::sort(v.begin(), v.end());
     const auto &ref = per[0];
     for (const auto &v : per) {
-        if (v != ref) return;
+        if (v != ref) return 0;
     }
-    if ((int)ref.size() > kLineRules) return;
     // copy rules read interior nodes (the owner of a node refills the ghosts
     // that copy it when it updates it)
     for (const auto &rule : ref) {
-        if (rule.second >= 0 && (rule.second < g.lo[p] || rule.second >= g.hi[p])) return;
+        if (rule.second >= 0 && (rule.second < g.lo[p] || rule.second >= g.hi[p])) return 0;
     }
-    for (int pos = g.lo[p] - half; pos < g.hi[p] + half; ++pos) {
-        if (pos >= g.lo[p] && pos < g.hi[p]) continue;
+    for (int e = 0; e < 2 * half; ++e) {
+        const int pos = (e < half) ? g.lo[p] - half + e : g.hi[p] + e - half;
         bool hit = false;
-        for (const auto &rule : ref) hit = hit || rule.first == pos;
-        if (!hit || pos < 0 || pos >= ext[p]) return;
+        for (const auto &rule : ref) {
+            if (rule.first != pos) continue;
+            R.src[e] = rule.second;
+            hit = true;
+        }
+        if (!hit || pos < 0 || pos >= ext[p]) return 0;
     }
-    R.count = (int)ref.size();
-    for (int e = 0; e < R.count; ++e) {
-        R.dst[e] = ref[e].first;
-        R.src[e] = ref[e].second;
-    }
-    for (int k = 0; k < nfaces; ++k) Conservative(dev->par.gamma, dev->par.varBC[faces[k]], R.state[k]);
-    R.ok = 1;
+    for (int e = 2 * half; e < kLineGhosts; ++e) R.src[e] = kWallGhost;     // none
+    return SetLineStates(dev, p, nfaces, faces);
 }
 
 // The rules of an axis with a wall at one end or both, from the face types:
 // an interior line's ghosts along its own axis come from its own axis's
 // faces alone (boundary_treatment.c:66-185): the wall's mirror states, the
 // prescribed state in every layer, or the boundary neighbour's in every layer.
-void DeriveWallRules(ArtraDevice *dev, int p)
+int DeriveWallRules(ArtraDevice *dev, int p)
 {
     const Grid &g = dev->g;
     const int ext[3] = {g.nx, g.ny, g.nz};
@@ -3193,9 +3217,10 @@ void DeriveWallRules(ArtraDevice *dev, int p)
     R = ArtraDevice::LineRules{};
     const int lo = g.lo[p], hi = g.hi[p];
     // the mirrored nodes of the farthest ghost are interior
-    if (hi - lo < half || lo - half < 0 || hi + half > ext[p]) return;
+    if (hi - lo < half || lo - half < 0 || hi + half > ext[p]) return 0;
     ArtraDevice::LineRules N{};
-    int states = 0;
+    std::fill(N.src, N.src + kLineGhosts, kWallGhost);
+    int states = 0, faces[2] = {0, 0};
     for (int side = 0; side < 2; ++side) {
         const int face = 1 + 2 * p + side, type = dev->par.typeBC[face];
         if (type == 2 || type == 3) {
@@ -3203,16 +3228,13 @@ void DeriveWallRules(ArtraDevice *dev, int p)
             N.wallT[side] = dev->par.varBC[face][5];
             continue;
         }
-        if (type != 0 && type != 1) return;
-        for (int q = 0; q < half; ++q) {
-            N.dst[N.count] = side ? hi + q : lo - 1 - q;
-            N.src[N.count++] = (type == 0) ? -1 - states : side ? hi - 1 : lo;
-        }
-        if (type == 0) Conservative(dev->par.gamma, dev->par.varBC[face], N.state[states++]);
+        if (type != 0 && type != 1) return 0;
+        for (int q = 0; q < half; ++q) N.src[side * half + q] = (type == 0) ? -1 - states : side ? hi - 1 : lo;
+        if (type == 0) faces[states++] = face;
     }
-    if (!N.wall[0] && !N.wall[1]) return;
+    if (!N.wall[0] && !N.wall[1]) return 0;
     R = N;
-    R.ok = 1;
+    return SetLineStates(dev, p, states, faces);
 }
 
 // Runge-Kutta stages of one directional operator (fluid_dynamics.c:121-148).
@@ -3575,6 +3597,7 @@ int artra_dev_create(const ArtraDevParams *par, const uint8_t *fluid, ArtraDevic
     if (e == hipSuccess) e = hipMalloc(&dev->U, fieldBytes);
     if (e == hipSuccess) e = hipMalloc(&dev->fluid, (size_t)g.N);
     if (e == hipSuccess) e = hipMalloc(&dev->vmax, 4 * sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipMalloc(&dev->lineStates, 30 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&dev->marchBuf, MarchScratchBytes(kMarchChunk));
     if (e == hipSuccess) e = hipMemcpy(dev->fluid, fluid, (size_t)g.N, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -3618,6 +3641,7 @@ void artra_dev_destroy(ArtraDevice *dev)
         hipFree(b.f); hipFree(b.e); hipFree(b.block); hipHostFree(b.stage); hipFree(b.sph); hipFree(b.bsph);
     }
     hipFree(dev->vmax);
+    hipFree(dev->lineStates);
     hipFree(dev->marchBuf);
     hipFree(dev->forceNodes);
     hipFree(dev->forceBodies);
@@ -3694,7 +3718,7 @@ int artra_dev_set_gather(ArtraDevice *dev, const ArtraBcGather *gt)
     for (int s = 0; s < 3; ++s) {
         dev->axisGather[s] = 0;
         dev->lines[s] = ArtraDevice::LineRules{};
-        if (gt->resolved) DeriveLineRules(dev, s, gt->axis_count[s], gt->axis_dst[s], gt->axis_src[s]);
+        if (gt->resolved && DeriveLineRules(dev, s, gt->axis_count[s], gt->axis_dst[s], gt->axis_src[s])) return 1;
     }
     if (!gt->resolved) return 0;
     for (int m = 0; m < 4; ++m) {
@@ -3723,13 +3747,10 @@ int artra_dev_set_axis_gather(ArtraDevice *dev, int s, const ArtraBcGather *gt)
     dev->gDst[m] = dev->gSrc[m] = nullptr;
     dev->gCount[m] = 0;
     dev->axisGather[s] = 0;
-    if (!gt->resolved) {
-        DeriveWallRules(dev, s);
-        return 0;
-    }
+    if (!gt->resolved) return DeriveWallRules(dev, s);
     // (with bodies in the grid no line runs fused: their 30 ms on 512 x 512
     // lines would be for nothing)
-    if (dev->allFluid) DeriveLineRules(dev, s, gt->count, gt->dst, gt->src);
+    if (dev->allFluid && DeriveLineRules(dev, s, gt->count, gt->dst, gt->src)) return 1;
     const long n = gt->count;
     if (n > 0) {
         HIP_TRY(hipMalloc(&dev->gDst[m], n * sizeof(int)));
