@@ -24,7 +24,7 @@ def build():
     reference harness and the drop-in driver (the reference's objects linked
     with libartra_hip.so, which must be built first)."""
     subprocess.run(["make", "-s", "-C", HERE, "oracle"], check=True)
-    if os.path.isdir("/root/reference"):
+    if os.path.isfile("/root/reference/solve.c"):
         subprocess.run(["make", "-s", "-C", HERE, "ref", "-j8"], check=True)
         subprocess.run(["make", "-s", "-C", HERE, "dropin"], check=True)
 
