@@ -634,7 +634,9 @@ __host__ __device__ __forceinline__ void viscous_flux(const FluxModel &mdl, cons
     const double gSS = (velE[S] - velP[S]) * dd[S];
     const double gAS = (velE[TA] - velP[TA]) * dd[S], gBS = (velE[TB] - velP[TB]) * dd[S];
     const double Ts = 0.5 * (TP + TE) * mdl.refT;
-    const double mu = (mdl.refMu * 1.458e-6) * (Ts * root(Ts)) * reciprocal(Ts + 110.4);
+    // (root(0) is not a number: a face between nodes without pressure has no viscosity)
+    const double rTs = (Ts == 0.0) ? 0.0 : root(Ts);
+    const double mu = (mdl.refMu * 1.458e-6) * (Ts * rTs) * reciprocal(Ts + 110.4);
     const double heatK = mdl.gamma * mdl.cv * (1.0 / 0.71) * mu;
     const double divV = gSS + gAA + gBB;
     F[0] = 0.0;

@@ -74,6 +74,29 @@ def test_stage_sweeps_at_the_edges_of_their_tiles(tmp_path, oracle_mod, m, bcs, 
         assert np.abs(U[c] - ref[c]).max() <= 1e-13 * np.abs(ref[c]).max()
 
 
+def test_viscous_face_between_nodes_without_pressure(tmp_path):
+    """Two neighbours along z with E = rho w^2 / 2 exactly: their temperature
+    and Sutherland's viscosity at their face are zero in both arithmetics."""
+    from artracfd_amd import Case, Solver
+    directory = write_case(tmp_path, (7, 7, 7), RING, mu=0.02)
+    out = []
+    for exact in (True, False):
+        case = Case(directory)
+        solver = Solver(case, exact=exact)
+        U = solver.field()
+        U[:, 5, 6, 6] = [1.0, 0.0, 0.0, 0.5, 0.125]
+        U[:, 6, 6, 6] = [1.0, 0.0, 0.0, 0.25, 0.03125]
+        solver.set_field(0, U)
+        print(exact, flush=True)
+        solver.evolve(1e-6)
+        out.append(case.interior(solver.field()).copy())
+        solver.close()
+        case.close()
+    assert np.isfinite(out[0]).all()
+    for c in (slice(0, 1), slice(1, 4), slice(4, 5)):
+        assert np.abs(out[1][c] - out[0][c]).max() <= 1e-13 * np.abs(out[0][c]).max()
+
+
 MIXED = [mc.inflow(1.1, 0.4, 0.1, 0, 1.2), mc.noslip(), mc.slip(), mc.OUTFLOW, mc.noslip(0.0033), mc.slip(0.0036)]
 # (nodes, boundaries, the axes that run as lines): lines of one node to one
 # past the two-node threads' first, several lines to a block with a rest, a
