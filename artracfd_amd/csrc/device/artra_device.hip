@@ -972,8 +972,9 @@ __device__ __forceinline__ bool ClassifyFace(const LineHybrid &hy, const float *
 }
 
 // The operators on one line, run by T threads tt = 0 .. T - 1: thread tt
-// holds the nodes lo + tt + T k and the faces to their left (T covers the F
-// faces with K per thread).  Every thread of the block must call it with the
+// holds the nodes lo + tt + T k and the faces to their left (T covers the
+// nodes with K per thread; with K = 2 the one face beyond may take a pass of
+// its own).  Every thread of the block must call it with the
 // same stage counts, because the stages are separated by block barriers;
 // lines that are not `active` (past the last of the block) only keep the
 // barriers.
@@ -989,6 +990,7 @@ __device__ __forceinline__ void PlainLine(const LineArgs &la, const FluxModel &m
     const long base = LineBase(la, line);
     const bool walls = la.wall[0] || la.wall[1];
     const double r = Uniform(la.dt ? *la.dt * la.dd : la.r);
+    const int passes = (K == 1) ? 1 : (F + T - 1) / T;
     unsigned feeds[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) feeds[k] = FeedsOf(la, la.lo + tt + T * k);
@@ -1002,7 +1004,7 @@ __device__ __forceinline__ void PlainLine(const LineArgs &la, const FluxModel &m
         }
         double FL[5];
 #pragma nounroll
-        for (int k = 0; k < K; ++k) {
+        for (int k = 0; k < passes; ++k) {
             const int q = tt + T * k;               // face between nodes lo - 1 + q and lo + q
             if (!active || q >= F) continue;
             double Fx[5];
@@ -2921,8 +2923,9 @@ struct LineShape {
 };
 
 // Threads of a plain line and lines of a block for lines of F faces and n
-// nodes: a thread per face (two faces each beyond 256), and of the numbers
-// of lines that fit 256 threads the one that keeps most lanes of the
+// nodes: a thread per face (two faces each beyond 256; the 513th, of 512
+// nodes on 256 threads, is a third pass of one wavefront), and of the
+// numbers of lines that fit 256 threads the one that keeps most lanes of the
 // resident wavefronts busy.  A line rounded up to whole wavefronts of its
 // own leaves half the lanes idle on 32-node and a third on 150-node lines;
 // packed, 95-98 % of them work.
@@ -2930,6 +2933,7 @@ void PlainShape(int n, int F, LineShape &sh)
 {
     sh.K = (F <= 256) ? 1 : 2;
     sh.T = (F + sh.K - 1) / sh.K;
+    if (F == 513) sh.T = 256;
     if (sh.T > 256) {
         sh = LineShape{};
         return;

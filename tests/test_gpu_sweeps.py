@@ -99,10 +99,12 @@ def test_viscous_face_between_nodes_without_pressure(tmp_path):
 
 MIXED = [mc.inflow(1.1, 0.4, 0.1, 0, 1.2), mc.noslip(), mc.slip(), mc.OUTFLOW, mc.noslip(0.0033), mc.slip(0.0036)]
 # (nodes, boundaries, the axes that run as lines): lines of one node to one
-# past the two-node threads' first, several lines to a block with a rest, a
-# wavefront's and a block's faces more or less by one
+# past the two-node threads' first, the longest line and one longer, several
+# lines to a block with a rest, a wavefront's and a block's faces more or less
+# by one
 LINES = [((2, 3, 4), OPEN, "xyz"), ((4, 3, 3), RING, "xyz"), ((64, 63, 5), OPEN, "xyz"), ((4, 128, 7), RING, "xyz"),
-         ((256, 3, 5), OPEN, "xyz"), ((257, 5, 3), OPEN, "xyz"), ((3, 512, 3), OPEN, "xyz"), ((3, 3, 513), OPEN, "xy"),
+         ((256, 3, 5), OPEN, "xyz"), ((257, 5, 3), OPEN, "xyz"), ((3, 512, 3), OPEN, "xyz"), ((3, 3, 513), OPEN, "xyz"),
+         ((3, 511, 3), RING, "xyz"), ((3, 3, 514), OPEN, "xy"),
          ((11, 37, 16), WALLS, "xyz"), ((4, 258, 4), WALLS, "xyz"), ((21, 4, 66), MIXED, "xyz"),
          ((2, 7, 2), WALLS, "y")]                # (a wall needs as many interior nodes as ghosts)
 
