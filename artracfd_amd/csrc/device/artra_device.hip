@@ -2748,7 +2748,7 @@ void LaunchSweep(ArtraDevice *dev, int s, const StageArgs &sa)
         if (interior[q] <= 0) return;
     }
     const int n[3] = {g.nx, g.ny, g.nz};
-    const SweepTile ts = artra::TileOf(n, interior, s, NS / 2, VISC, dev->segment);
+    const SweepTile ts = artra::TileOf(n, interior, s, NS / 2, VISC, FAST, dev->segment);
     const size_t lds = TileDoubles(ts.P, ts.seg, ts.rows, VISC) * sizeof(double);
     const dim3 grid((unsigned)ts.tiles), block(ts.threads);
     const auto launch = [&](auto axis) {

@@ -63,10 +63,16 @@ inline int TileRows(int stride, int width)
 // issue slots, an element copied in or out 8 or 20 per wavefront
 // (instruction counts of the kernel), a cache line moved about 6; idle lanes
 // of a partly filled wavefront, the halo of a short segment and the broken
-// cache lines of a narrow tile show in these counts.  One row at a time and
-// a segment of kTileIn - 2 halo nodes or less always fits, so there is a
-// shape for every grid.
-inline SweepTile TileOf(const int n[3], const int interior[3], int s, int halo, bool visc, int longest)
+// cache lines of a narrow tile show in these counts.
+// In exact arithmetic, with its divisions and roots, the faces cost 2500,
+// and only eight wavefronts fit a compute unit: those a block leaves no room
+// for (two blocks of three) or holds for copies alone count half.  (A step
+// stage by stage on 127^3 nodes 3.10 -> 2.92 ms, on 199^3 11.50 -> 11.17, a
+// viscous one on 127 x 127 x 63 2.47 -> 2.19 against 650 alone; 2500 alone
+// takes 1.85 where this takes 1.60 on 511 x 511 x 3.)
+// One row at a time and a segment of kTileIn - 2 halo nodes or less always
+// fits, so there is a shape for every grid.
+inline SweepTile TileOf(const int n[3], const int interior[3], int s, int halo, bool visc, bool fast, int longest)
 {
     SweepTile best{};
     double bestCost = 0.0;
@@ -99,7 +105,8 @@ inline SweepTile TileOf(const int n[3], const int interior[3], int s, int halo, 
             const double cacheLines = (s == 0) ? P * ((rows + 2 * seg) * 40.0 / 128.0 + 2.25)
                                                : (rows + 2 * seg) * (P * 40.0 / 128.0 + 0.75);
             const double tiles = (double)((across + P - 1) / P) * others * nseg;
-            const double cost = tiles * (650.0 * faceWaves + waves * (8.0 * in + 20.0 * out) + 6.0 * cacheLines);
+            const double faces = fast ? 650.0 * faceWaves : 1250.0 * (faceWaves + 8.0 / (8 / waves));
+            const double cost = tiles * (faces + waves * (8.0 * in + 20.0 * out) + 6.0 * cacheLines);
             if (best.P && cost >= bestCost) continue;
             best.P = P;
             best.seg = seg;

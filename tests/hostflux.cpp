@@ -73,9 +73,10 @@ void host_weno_flux(int s, int roe, int sw, const double *st, double *F)
 
 // The tile of a stage sweep: P, seg, nseg, groups, others, rows, perPass,
 // threads, tiles.
-void host_tile(const int *n, const int *interior, int s, int halo, int visc, int longest, int *out)
+void host_tile(const int *n, const int *interior, int s, int halo, int visc, int fast, int longest,
+               int *out)
 {
-    const artra::SweepTile t = artra::TileOf(n, interior, s, halo, visc != 0, longest);
+    const artra::SweepTile t = artra::TileOf(n, interior, s, halo, visc != 0, fast != 0, longest);
     const int v[9] = {t.P, t.seg, t.nseg, t.groups, t.others, t.rows, t.perPass, t.threads, t.tiles};
     for (int q = 0; q < 9; ++q) out[q] = v[q];
 }

@@ -160,13 +160,14 @@ TILES = [(3450, 3450, 36), (4650, 4650, 22), (5200, 5200, 17), (12000, 12000, 2)
 @pytest.mark.parametrize("interior", TILES)
 @pytest.mark.parametrize("halo", [2, 3])
 @pytest.mark.parametrize("visc", [0, 1])
-def test_tiles_fit_their_blocks_and_their_offsets(hostflux, interior, halo, visc):
+@pytest.mark.parametrize("fast", [0, 1])
+def test_tiles_fit_their_blocks_and_their_offsets(hostflux, interior, halo, visc, fast):
     n = [v + 2 * halo for v in interior]
     assert n[0] * n[1] * n[2] < 2 ** 31
     hostflux.host_tile_offset.restype = ctypes.c_uint
     for s in range(3):
         out = (ctypes.c_int * 9)()
-        hostflux.host_tile((ctypes.c_int * 3)(*n), (ctypes.c_int * 3)(*interior), s, halo, visc, 0, out)
+        hostflux.host_tile((ctypes.c_int * 3)(*n), (ctypes.c_int * 3)(*interior), s, halo, visc, fast, 0, out)
         P, seg, nseg, groups, others, rows, per, threads, tiles = list(out)
         across, third = interior[1 if s == 0 else 0], interior[1 if s == 2 else 2]
         # every node is swept, every face of a segment has a thread
