@@ -2652,6 +2652,10 @@ struct ArtraDevice {
     std::vector<GeoBodyDev> geoBodies;
     std::vector<int> layerStart;
     FluxModel mdl{};
+    struct StageTile {              // of the stage sweeps along an axis, and the settings it was chosen for (the
+        SweepTile ts;               // grid, the schemes and the viscosity stay): 2 us of search a launch otherwise
+        int exact = -1, segment = -1;
+    } tiles[3];
     int segment = 0;                // longest segment of the y and z stage sweeps (0: as the tile allows)
     int exact = 0;                  // 1: reference operation order (bit-faithful), 0: fast arithmetic
     int partialFill = 1;            // axis-only fills between the stages of inviscid split sweeps
@@ -2747,8 +2751,14 @@ void LaunchSweep(ArtraDevice *dev, int s, const StageArgs &sa)
         interior[q] = g.hi[q] - g.lo[q];
         if (interior[q] <= 0) return;
     }
-    const int n[3] = {g.nx, g.ny, g.nz};
-    const SweepTile ts = artra::TileOf(n, interior, s, NS / 2, VISC, FAST, dev->segment);
+    ArtraDevice::StageTile &kept = dev->tiles[s];
+    if (kept.exact != dev->exact || kept.segment != dev->segment) {
+        const int n[3] = {g.nx, g.ny, g.nz};
+        kept.ts = artra::TileOf(n, interior, s, NS / 2, VISC, FAST, dev->segment);
+        kept.exact = dev->exact;
+        kept.segment = dev->segment;
+    }
+    const SweepTile &ts = kept.ts;
     const size_t lds = TileDoubles(ts.P, ts.seg, ts.rows, VISC) * sizeof(double);
     const dim3 grid((unsigned)ts.tiles), block(ts.threads);
     const auto launch = [&](auto axis) {
