@@ -1,6 +1,5 @@
-"""Batched cases: many independent cases advanced in lockstep, one
-persistent launch per directional operator over the lines of every case
-(artra_hip_batch_*), optionally replayed from a captured HIP graph.
+"""Batched cases: many independent cases advanced in lockstep, one launch per
+directional operator over the lines of every case (artra_hip_batch_*), optionally replayed from a captured HIP graph.
 
 The synthetic workload of the batched benchmark: oblique shocks running
 into randomly perturbed gas, cubic grids of uneven sizes, all drawn from one
@@ -57,7 +56,9 @@ class Batch:
         self._h = h
 
     def tune(self, reps=2):
-        """Autotune tile shapes and the persistent grid; returns (threads per line per case, grid)."""
+        """Autotune the routed lines' tile shapes and persistent grid; returns
+        (threads per line per case, grid).  Without the indicator there is
+        nothing to tune: they come back as they stand."""
         n = len(self.solvers)
         threads = (ctypes.c_int * n)()
         grid = ctypes.c_int()
@@ -65,7 +66,8 @@ class Batch:
         return list(threads), grid.value
 
     def set_threads(self, threads):
-        """Tile shape per case (threads per line) instead of the tuner's choice."""
+        """Tile shape per case (threads per routed line) instead of the tuner's
+        choice; no effect without the indicator."""
         n = len(self.solvers)
         t = (ctypes.c_int * n)(*[int(v) for v in threads])
         _check(_bind().artra_hip_batch_set_threads(self._h, t))

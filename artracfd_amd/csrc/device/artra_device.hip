@@ -1390,12 +1390,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
     }
 }
 
-// Many independent cases in one persistent launch: blocks of 256 threads
-// walk a tile list; a tile is 256 / T lines of one case, each run by T
-// threads.  Plain lines take a thread per face (K = 1; two faces each with
-// K = 2); with the indicator T is a multiple of the wavefront, the tile
-// shape picked per grid size, and lines past the case's end in its last tile
-// are computed on a copy of its last line and not stored.
+// Many independent cases in one launch over a list of tiles, a tile being
+// some lines of one case, each run by T of the block's 256 threads.  Plain
+// lines take a thread per face (K = 1; two faces each with K = 2), as many
+// lines a tile as its threads and 52 KB of LDS hold, and a block per tile.
+// With the indicator persistent blocks walk the list; T is a multiple of the
+// wavefront, the tile 256 / T lines, its shape picked per grid size, and
+// lines past the case's end in its last tile are computed on a copy of its
+// last line and not stored.
 struct BatchTile {
     int c;                          // case
     int T;                          // threads per line
@@ -4276,8 +4278,8 @@ struct ArtraBatch {
     std::vector<ArtraDevice *> cases;
     int C = 0;
     hipStream_t stream = nullptr;
-    std::vector<int> threads;               // threads per line of each case (tuned)
-    int grid = 0;                           // persistent blocks of the line launches
+    std::vector<int> threads;               // threads per routed line of each case (tuned)
+    int grid = 0;                           // persistent blocks of the routed lines' launches
     LineArgs *dArgs[3] = {nullptr, nullptr, nullptr};
     BatchTile *dTiles[3] = {nullptr, nullptr, nullptr};
     int ntiles[3] = {0, 0, 0};
@@ -4395,8 +4397,8 @@ void BatchFill(ArtraBatch *b, hipStream_t st)
                        b->gDst, b->gSrc, b->gCount);
 }
 
-// One time step of every case: speeds, dt, then Z Y X X Y Z, each operator a
-// persistent launch over all cases' lines (plain x operators: both in one).
+// One time step of every case: speeds, dt, then Z Y X X Y Z, each operator one
+// launch over all cases' lines (plain x operators: both in one).
 // The lines start from their own interiors, so the fill of every case
 // follows once, behind a march's last step.
 int BatchStep(ArtraBatch *b, hipStream_t st)
@@ -4684,8 +4686,9 @@ int artra_dev_batch_clock(ArtraBatch *b, double *clock)
     return 0;
 }
 
-// Tile shape of every case: threads[c] threads per line (64, 128 or 256, at
-// least the case's longest interior line, with 256 / T lines in LDS).
+// Tile shape of every case's routed lines: threads[c] threads per line (64,
+// 128 or 256, at least the case's longest interior line, with 256 / T lines
+// in LDS).
 int artra_dev_batch_set_threads(ArtraBatch *b, const int *threads)
 {
     for (int c = 0; c < b->C; ++c) {
@@ -4715,14 +4718,22 @@ int artra_dev_batch_set_clock(ArtraBatch *b, const double *clock)
     return 0;
 }
 
-// Autotuner: for every grid size in the batch (cases of equal line length)
-// time the three directional launches with each admissible threads-per-line
-// choice (the tile shape: 256 / T lines of T threads per block), keep the
-// fastest; then time whole steps for persistent grids of 2, 4 and 8 blocks
-// per compute unit.  The field is restored afterwards (the tuning steps run
-// on a scratch copy of level TO in level TN of every case).
+// Autotuner of the routed lines: for every grid size in the batch (cases of
+// equal line length) time the three directional launches with each
+// admissible threads-per-line choice (the tile shape: 256 / T lines of T
+// threads per block), keep the fastest; then time whole steps for persistent
+// grids of 2, 4 and 8 blocks per compute unit.  The field is restored
+// afterwards (the tuning steps run on a scratch copy of level TO in level TN
+// of every case).  Plain lines have no shape to choose (BatchBuildTiles), so
+// without the indicator nothing runs.
 int artra_dev_batch_tune(ArtraBatch *b, int reps, int *threads_out, int *grid_out)
 {
+    if (!b->hybrid) {
+        for (int c = 0; c < b->C; ++c)
+            if (threads_out) threads_out[c] = b->threads[c];
+        if (grid_out) *grid_out = b->grid;
+        return 0;
+    }
     if (reps < 1) reps = 1;
     // save TO of every case into TN, restore at the end
     for (ArtraDevice *dv : b->cases) {
@@ -4746,7 +4757,6 @@ int artra_dev_batch_tune(ArtraBatch *b, int reps, int *threads_out, int *grid_ou
         if (std::find(lengths.begin(), lengths.end(), L) == lengths.end()) lengths.push_back(L);
     }
     const std::vector<int> saved = b->threads;
-    if (!b->hybrid) lengths.clear();                // plain lines take a thread per face: no shape to choose
     for (int L : lengths) {
         double best = 1e300;
         int bestT = 0;
@@ -4784,7 +4794,7 @@ int artra_dev_batch_tune(ArtraBatch *b, int reps, int *threads_out, int *grid_ou
         if (BatchBuildTiles(b, p)) return 1;
     double bestG = 1e300;
     int grid = b->grid;
-    for (int m = 2; b->hybrid && m <= 8; m *= 2) {  // (plain tiles: a block each)
+    for (int m = 2; m <= 8; m *= 2) {
         b->grid = m * b->cus;
         HIP_TRY(hipEventRecord(e0, b->stream));
         for (int r = 0; r < reps; ++r)

@@ -232,8 +232,8 @@ int artra_mlp_gradient_dev(const float *params, const float *feat, const float *
 int artra_mlp_infer_dev(const float *params, const float *feat, long n, float *logit);
 const char *artra_mlp_error(void);
 
-/* batched cases: many independent cases advanced together, one persistent
- * launch per directional operator over the lines of every case */
+/* batched cases: many independent cases advanced together, one launch per
+ * directional operator over the lines of every case */
 typedef struct ArtraBatch ArtraBatch;
 /* clock[c] = {now, end, rcInt, tmInt, stepC, stepN} of case c (6 doubles);
  * cfl[c] its CFL number */
@@ -245,6 +245,7 @@ int artra_dev_batch_counts(ArtraBatch *b, unsigned long long counts[ARTRA_HYBRID
 int artra_dev_batch_march(ArtraBatch *b, int steps, int use_graph, double *ms);
 int artra_dev_batch_clock(ArtraBatch *b, double *clock);
 int artra_dev_batch_set_clock(ArtraBatch *b, const double *clock);
+/* tile shapes of the routed lines (plain lines have none to choose) */
 int artra_dev_batch_set_threads(ArtraBatch *b, const int *threads);
 int artra_dev_batch_tune(ArtraBatch *b, int reps, int *threads, int *grid);
 

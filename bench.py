@@ -276,8 +276,8 @@ def batched_both(with_indicator=True):
 
 def batched(seed=2026, count=64, steps=100, use_indicator=True):
     """The batched workload: `count` oblique-shock cases of uneven cubic
-    sizes (artracfd_amd.batch), tuned, then `steps` lockstep steps replayed
-    from a HIP graph; and the same cases one at a time for per-case wall
+    sizes (artracfd_amd.batch), tuned where the indicator routes their lines,
+    then `steps` lockstep steps replayed from a HIP graph; and the same cases one at a time for per-case wall
     times."""
     import tempfile
 
@@ -339,7 +339,8 @@ def batched(seed=2026, count=64, steps=100, use_indicator=True):
             "weno5_face_fraction": round(over / max(seen, 1), 4) if params is not None else None,
             "flagged_face_fraction": round(flagged / max(seen, 1), 4) if params is not None else None,
             "tuned": {"threads_per_line": {str(sd): sorted(set(t for t, d in zip(threads, drawn) if d["side"] == sd))
-                                           for sd in sides}, "grid_blocks": grid},
+                                           for sd in sides}, "grid_blocks": grid}
+            if params is not None else None,
             "setup_seconds": round(setup_s, 2), "tune_seconds": round(tune_s, 2),
             "cells": int(sum(cells))}
 

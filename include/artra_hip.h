@@ -219,10 +219,11 @@ const char *artra_hip_error(void);
  * Many independent cases advanced together.  Each time step is one device
  * CFL reduction over every case, one kernel computing every case's dt (with
  * the time loop's rectification, solve.c:65-78), then the split directional
- * operators Z Y X X Y Z, each as ONE persistent launch over the lines of
- * every case (blocks walk a tile list; a tile is 256 / T lines of one case,
- * T threads per line) followed by every case's boundary fill.  Nothing of a
- * step needs the host, so a step can be captured once in a HIP graph and
+ * operators Z Y X X Y Z, each as ONE launch over the lines of every case (a
+ * block per tile of packed lines; with the indicator persistent blocks walk
+ * a list of tiles of 256 / T lines, T threads per line); every case's
+ * boundary fill follows once, behind the marched steps.  Nothing of a step
+ * needs the host, so a step can be captured once in a HIP graph and
  * replayed.  No reference counterpart: an addition of this library.
  *
  * Cases must be three-dimensional, fluid-only, inviscid, split WENO5 with
@@ -234,12 +235,16 @@ const char *artra_hip_error(void);
 typedef struct ArtraHipBatch ArtraHipBatch;
 int artra_hip_batch_create(ArtraHipSolver *const *solvers, Time *const *times, int count, ArtraHipBatch **out);
 int artra_hip_batch_destroy(ArtraHipBatch *batch);
-/* Autotuner: per grid size the threads per line (tile shape), then the
- * persistent grid size; threads[count] and *grid receive the choice.  The
- * fields and clocks are restored afterwards. */
+/* Autotuner of a batch with the indicator: per grid size the threads per
+ * routed line (tile shape), then the persistent grid size; threads[count]
+ * and *grid receive the choice.  The fields and clocks are restored
+ * afterwards.  Plain lines take a thread per face and have no shape to tune:
+ * without the indicator nothing runs and the shapes are returned as they
+ * stand, for an indicator set later. */
 int artra_hip_batch_tune(ArtraHipBatch *batch, int reps, int *threads, int *grid);
-/* Set the tile shape instead of tuning it: threads[c] threads per line of
- * case c (64, 128 or 256, at least its longest interior line). */
+/* Set the tile shape of the routed lines instead of tuning it: threads[c]
+ * threads per line of case c (64, 128 or 256, at least its longest interior
+ * line).  Without the indicator it has no effect until one is set. */
 int artra_hip_batch_set_threads(ArtraHipBatch *batch, const int *threads);
 /* Learned indicator for every case (NULL: plain WENO5). */
 int artra_hip_batch_set_indicator(ArtraHipBatch *batch, const float *params, float logit_threshold);

@@ -80,6 +80,38 @@ def test_batch_tuner_keeps_the_field_and_the_result(tmp_path):
         c.close()
 
 
+def test_batch_tuner_with_the_indicator(tmp_path):
+    """The tuner's trial steps of routed lines leave fields, clocks and results
+    alone; a plain batch takes its shapes as they stand."""
+    print("batch tuner, routed", flush=True)
+    import mlp_oracle as M
+
+    from artracfd_amd import Case, Solver
+    from artracfd_amd.batch import Batch
+    params = M.init_params(11)
+    dirs = _cases(tmp_path, SPEC)
+    ref = _single(dirs, 3, params, 0.5)
+    cases = [Case(d) for d in dirs]
+    solvers = [Solver(c) for c in cases]
+    before = [c.interior(s.field()) for c, s in zip(cases, solvers)]
+    b = Batch(solvers)
+    plain = b.tune(reps=1)
+    b.set_threads([256] * len(dirs))
+    assert b.tune(reps=1) == ([256] * len(dirs), plain[1])
+    b.set_indicator(params, 0.5)
+    threads, grid = b.tune(reps=1)
+    assert all(t in (64, 128, 256) for t in threads) and grid > 0
+    for q, (c, s) in enumerate(zip(cases, solvers)):
+        assert np.array_equal(c.interior(s.field()), before[q])
+    b.march(3)
+    for q, (c, s) in enumerate(zip(cases, solvers)):
+        assert np.array_equal(c.interior(s.field()), ref[q][0]), q
+    b.close()
+    for s, c in zip(solvers, cases):
+        s.close()
+        c.close()
+
+
 def test_batch_with_indicator_matches_single_case_runs(tmp_path):
     print("batch hybrid vs single hybrid", flush=True)
     import mlp_oracle as M
