@@ -121,8 +121,8 @@ int artra_compute_geometric_field(Space *space, const Model *model, ArtraGhostTa
  * A scope tracks, per body, the node box of its nodes (extent) and the box of
  * the last reconstructed nodes; artra_scope_region gives, after the bodies
  * moved, the box that the passes must cover (region argument above), and
- * artra_scope_update refreshes the scope from the new classification (the
- * moving bodies' nodes all lie inside that region).
+ * artra_scope_extents refreshes the scope from the boxes that the new
+ * classification found (the moving bodies' nodes all lie inside that region).
  */
 /* The host's copy of a classification made on the device over a region of
  * `count` nodes, from its changes: change[] = place in the region in k-j-i
@@ -140,10 +140,8 @@ typedef struct {
 int artra_scope_init(const Space *space, ArtraGeometryScope *scope);
 void artra_scope_free(ArtraGeometryScope *scope);
 void artra_scope_region(const Space *space, const ArtraGeometryScope *scope, int region[DIMS][LIMIT]);
-void artra_scope_update(const Space *space, ArtraGeometryScope *scope, const ArtraGhostTable *joins,
-                        const int region[DIMS][LIMIT]);
-/* the same from the boxes that a classification found: extent[body] = lowest
- * and highest i, j, k (NULL: no moving body has nodes) */
+/* extent[body] = lowest and highest i, j, k of its nodes, lowest > highest
+ * without any (NULL: no moving body has nodes) */
 void artra_scope_extents(const Space *space, ArtraGeometryScope *scope, const ArtraGhostTable *joins,
                          const int (*extent)[2][DIMS]);
 void artra_identify_geometry_state(Geometry *geo);

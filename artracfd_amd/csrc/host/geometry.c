@@ -682,28 +682,6 @@ static void ScopeJoins(const Partition *part, ArtraGeometryScope *sc, const Artr
     }
 }
 
-void artra_scope_update(const Space *space, ArtraGeometryScope *sc, const ArtraGhostTable *joins,
-                        const int region[DIMS][LIMIT])
-{
-    const Partition *part = &space->part;
-    const Geometry *geo = &space->geo;
-    int lo[DIMS], hi[DIMS];
-    for (int s = 0; s < DIMS; ++s) {
-        lo[s] = (region[s][MIN] > part->ns[PIN][s][MIN]) ? region[s][MIN] : part->ns[PIN][s][MIN];
-        hi[s] = (region[s][MAX] < part->ns[PIN][s][MAX]) ? region[s][MAX] : part->ns[PIN][s][MAX];
-    }
-    for (int n = 0; n < geo->totN; ++n) {
-        if (1 != geo->poly[n].state) EmptyBox(sc->extent[n]);
-    }
-    for (int k = lo[Z]; k < hi[Z]; ++k)
-        for (int j = lo[Y]; j < hi[Y]; ++j)
-            for (int i = lo[X]; i < hi[X]; ++i) {
-                const int did = space->node[artra_index(k, j, i, part->n[Y], part->n[X])].did;
-                if (0 < did && did <= geo->totN && 1 != geo->poly[did - 1].state) AddNode(sc->extent[did - 1], k, j, i);
-            }
-    ScopeJoins(part, sc, joins);
-}
-
 void artra_scope_extents(const Space *space, ArtraGeometryScope *sc, const ArtraGhostTable *joins,
                          const int (*extent)[LIMIT][DIMS])
 {

@@ -7,6 +7,8 @@
  * each move copy A is classified over the whole interior (region NULL) and
  * copy B only over the scope's region; the node flags of every node and the
  * reconstruction lists (nodes, stencil nodes, weights) must be identical.
+ * The scope is refreshed from the moving bodies' node boxes within the
+ * region, as the device's classification reports them.
  * Also checks the bounded closest-facet search against the full scan on
  * every interior node and on points placed exactly on vertices, edges and
  * facets, and that the ghost table built on every thread equals the one
@@ -15,6 +17,7 @@
  *
  *   scope_check <case dir> <moves> <dx> <dy> <dz> <az>
  */
+#include <limits.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -39,6 +42,29 @@ static void Move(Space *space, const Real off[DIMS], const Real ang[DIMS])
             artra_transform_polyhedron(poly->O, unit, ang, off, poly);
         }
     }
+}
+
+/* Per body the lowest and highest i, j, k of its nodes in the region. */
+static void Boxes(const Space *space, const int region[DIMS][LIMIT], int (*extent)[LIMIT][DIMS])
+{
+    const Partition *part = &space->part;
+    for (int n = 0; n < space->geo.totN; ++n)
+        for (int s = 0; s < DIMS; ++s) {
+            extent[n][MIN][s] = INT_MAX;
+            extent[n][MAX][s] = INT_MIN;
+        }
+    for (int k = part->ns[PIN][Z][MIN]; k < part->ns[PIN][Z][MAX]; ++k)
+        for (int j = part->ns[PIN][Y][MIN]; j < part->ns[PIN][Y][MAX]; ++j)
+            for (int i = part->ns[PIN][X][MIN]; i < part->ns[PIN][X][MAX]; ++i) {
+                const int at[DIMS] = {i, j, k};
+                const int n = space->node[artra_index(k, j, i, part->n[Y], part->n[X])].did - 1;
+                int in = (0 <= n && n < space->geo.totN && 1 != space->geo.poly[n].state);
+                for (int s = 0; s < DIMS; ++s) in = in && region[s][MIN] <= at[s] && at[s] < region[s][MAX];
+                for (int s = 0; s < DIMS && in; ++s) {
+                    if (at[s] < extent[n][MIN][s]) extent[n][MIN][s] = at[s];
+                    if (at[s] > extent[n][MAX][s]) extent[n][MAX][s] = at[s];
+                }
+            }
 }
 
 static int SameJoins(const ArtraGhostTable *a, const ArtraGhostTable *b)
@@ -143,6 +169,8 @@ int main(int argc, char **argv)
     if (FacetSearch(&sa)) return 1;
     ArtraGeometryScope scope;
     if (artra_scope_init(&sb, &scope)) return 2;
+    int (*extent)[LIMIT][DIMS] = malloc((size_t)(sb.geo.totN + 1) * sizeof *extent);
+    if (NULL == extent) return 2;
     const long N = (long)sa.part.n[X] * sa.part.n[Y] * sa.part.n[Z];
     long joined = 0;
     for (int m = 0; m < moves; ++m) {
@@ -158,7 +186,8 @@ int main(int argc, char **argv)
             fprintf(stderr, "%s\n", artra_error_text());
             return 2;
         }
-        artra_scope_update(&sb, &scope, &jb, (const int (*)[LIMIT])region);
+        Boxes(&sb, (const int (*)[LIMIT])region, extent);
+        artra_scope_extents(&sb, &scope, &jb, (const int (*)[LIMIT][DIMS])extent);
         for (long q = 0; q < N; ++q) {
             const Node *a = sa.node + q, *b = sb.node + q;
             if (a->did != b->did || a->fid != b->fid || a->lid != b->lid || a->gst != b->gst) {
@@ -180,6 +209,7 @@ int main(int argc, char **argv)
         artra_free_ghost_table(&jb);
     }
     artra_scope_free(&scope);
+    free(extent);
     printf("ok %ld\n", joined);
     return 0;
 }

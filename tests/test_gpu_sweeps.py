@@ -319,3 +319,32 @@ def test_flags_of_a_moving_body_reach_the_host(tmp_path, m, r, steps):
         assert (flags != before).any(axis=0).sum() > 1024
     solver.close()
     case.close()
+
+
+def test_boxes_of_moving_bodies_are_those_of_their_nodes(tmp_path):
+    """The boxes that bound the next classification, from the device, after
+    every step: a body that crosses the grid, one that leaves it, one at rest
+    (tests/scope_device.c)."""
+    import subprocess
+
+    from artracfd_amd import library
+    d = tmp_path / "case"
+    d.mkdir()
+    m = 32
+    (d / "artracfd.case").write_text(mc.case_text(((-0.5, -0.5, -0.5), (0.5, 0.5, 0.5), (m, m, m)),
+                                                  (0, 1e9, 0.6, 0, 1, 0), (1, 1, 0, 0, 0, 1, 1), mc.INVISCID, mc.REF1,
+                                                  ("1", "0", "0", "0", "1"), [mc.OUTFLOW] * 6))
+    (d / "artracfd.geo").write_text(mc.moving_geo_text(spheres=[
+        dict(O=(-0.3, -0.2, 0.0), r=0.11, V=(2.0, 1.0, 0.5), rho=50.0, mid=2),
+        dict(O=(0.38, 0.3, 0.3), r=0.1, V=(4.0, 1.0, 1.0), rho=50.0, mid=2),
+        dict(O=(-0.3, 0.3, -0.3), r=0.12, rho="1e37", mid=2)]))
+    lib = library()._name
+    exe = str(tmp_path / "scope_device")
+    subprocess.run(["gcc", "-O1", "-std=c11", "-I" + os.path.join(ROOT, "include"),
+                    "-I" + os.path.join(ROOT, "artracfd_amd", "csrc", "host"),
+                    os.path.join(ROOT, "tests", "scope_device.c"), "-o", exe, lib, "-Wl,-rpath," + os.path.dirname(lib),
+                    "-lm"], check=True)
+    print("scope_device", flush=True)
+    out = subprocess.run([exe, str(d), "24"], capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert out.stdout.split() == ["ok", "24", "1"], out.stdout
