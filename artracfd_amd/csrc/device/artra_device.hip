@@ -14,8 +14,11 @@
 //                  (immersed_boundary.c:270-487).
 //   cfl_max        per-axis maximum characteristic speed (solve.c:108-153).
 //
-// All FP64 arithmetic follows the reference's operation order; the file is
-// compiled with -ffp-contract=off so results match the CPU bit for bit.
+// All arithmetic is FP64.  In exact arithmetic (and outside the fluxes and
+// node updates always) it follows the reference's operation order; the file
+// is compiled with -ffp-contract=off so those results match the CPU bit for
+// bit.  The default, fast arithmetic evaluates the same fluxes in fewer
+// operations (flux.hpp), equal to rounding level.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1206,10 +1209,10 @@ __device__ __forceinline__ void RoutedLine(const LineArgs &la, const FluxModel &
 
 // Plain lines, as many per block as its threads hold: `perLine` threads a
 // line, one per face up to 256 faces (K = 1), two faces each beyond (K = 2).
-// Bound by FP64 vector issue (535 of 600-626 vector instructions a stage and
-// node; 78-85 % of the issue cycles are taken at three wavefronts per SIMD).
-// At 256^3 an operator takes 1.17 ms along y, 1.14 along z, the two along x
-// in one launch 2.12 (one line to a block of whole wavefronts, component by
+// Bound by FP64 vector issue (535 of 593-616 vector instructions a stage and
+// node; 76-83 % of the issue cycles are taken at three wavefronts per SIMD).
+// At 256^3 an operator takes 1.16 ms along y, 1.13 along z, the two along x
+// in one launch 2.11 (one line to a block of whole wavefronts, component by
 // component loads, a launch per operator: 1.28, 1.25, 1.23 each with the same
 // flux arithmetic); on the 5-node lines of a 256 x 4 x 4 tube 10 us against 20.
 template <int S, int NS, bool FAST, int K>
@@ -1777,8 +1780,8 @@ __global__ __launch_bounds__(256) void geo_interface(Grid g, GeoSetup gs, GeoBox
 }
 
 // The ghost table on the device (immersed_boundary.c:270-487 via
-// artra_build_ghost_table): a wavefront per 64 nodes of a body's box; a
-// ghost of layer r takes the next entry of the table and kGhostSlot stencil
+// artra_build_ghost_table): a wavefront per kGhostNodes nodes of a body's
+// box; a ghost of layer r takes the next entry of the table and kGhostSlot stencil
 // entries, found by the same search (radius 2 around the image point's node
 // over fluid nodes for an image-point ghost, radius 1 around itself over
 // the previous layer's ghosts of the body otherwise, growing to 3).
@@ -2648,7 +2651,7 @@ struct ArtraDevice {
     int *geoChangesHost = nullptr;  // the host's copy (pinned)
     long geoRegionCap = 0;          // region nodes these hold
     int *geoMoving = nullptr;       // [bodies]: 1 for a body that moves
-    int *geoCounters = nullptr;     // ghost-table build: entries taken, overflow, each layer's end
+    int *geoCounters = nullptr;     // ghost-table build: overflow, then each layer's entries
     int *geoCountsHost = nullptr;   // their pinned host copy
     GeoSetup geo{};
     std::vector<GeoBodyDev> geoBodies;
@@ -3487,7 +3490,8 @@ int EnqueueStep(ArtraDevice *dev, const MarchScratch &ms, const double floor[3],
 }
 
 // The step as a captured graph, replayed once per step: one launch instead
-// of the step's 20 to 150 kernel launches.  Rebuilt when anything the
+// of the step's 3 (fused, one axis) to over 100 (immersed bodies) kernel
+// launches.  Rebuilt when anything the
 // step's launches depend on changed (configGen) or the body-speed floors or
 // the CFL number differ; not used with kernel timing (its events) or the
 // learned indicator (its lean-pass policy changes the launches between

@@ -42,9 +42,8 @@ FP64_PEAK_TFLOPS = 78.6
 # instruction counters).
 TRAFFIC_B_PER_CELL_STAGE = 22.4
 FP64_FLOP_PER_CELL_STAGE = 812.0
-# the stage-by-stage sweeps (profiles/sweep_shockvortex256.md: counted on the kernels before sweep_tile, whose
-# viscous and immersed cases move 120 and 126 B)
-UNFUSED_TRAFFIC_B_PER_CELL_STAGE = 112.3
+# the stage-by-stage sweeps (profiles/sweep_shockvortex256.md)
+UNFUSED_TRAFFIC_B_PER_CELL_STAGE = 113.4
 METRIC = "Mcell-stage updates/s (256³ WENO5-RK3) + learned-hybrid vs plain at ≤1e-3 L1"
 
 

@@ -1,4 +1,4 @@
-"""Batched cases: one persistent launch per directional operator over the
+"""Batched cases: one launch per directional operator over the
 lines of many independent cases must give, case by case, exactly what the
 single-case fused path gives (same dt sequence, same fields)."""
 import numpy as np
